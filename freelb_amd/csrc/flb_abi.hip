@@ -611,7 +611,7 @@ int flb_block_destroy(flb_block b) {
   else (void)hipDeviceSynchronize();
   detach_couplings(b);
   void* ptrs[] = {b->d_pops,  b->d_flags,   b->d_rho,   b->d_u,       b->d_partials, b->d_red,
-                  b->d_stage, b->d_links, b->d_rho_old, b->d_u_old, b->d_res};
+                  b->d_stage, b->d_alt, b->d_links, b->d_rho_old, b->d_u_old, b->d_res};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete b;
@@ -666,6 +666,7 @@ int flb_set_tasks(flb_block b, const flb_task* tasks, int n) {
   std::memcpy(saved, b->tasks, sizeof saved);
   for (int t = 0; t < n; ++t) b->tasks[t] = tasks[t];
   b->ntasks = n;
+  b->march = -1;
   int rc = check_layout(b);
   if (rc != FLB_OK) {
     std::memcpy(b->tasks, saved, sizeof saved);
@@ -703,6 +704,7 @@ int flb_set_halfway_bc(flb_block b, const flb_hwbc* bcs, int n) {
   for (int k = 0; k < n; ++k) b->bcs[k] = bcs[k];
   b->nbc = n;
   b->links_dirty = true;
+  b->march = -1;
   for (int k = 0; k < n; ++k)
     if (bcs[k].kind == FLB_HWBC_ANTI) return ensure_fields(b);  // the wall value is the RHO field
   return FLB_OK;
@@ -770,6 +772,7 @@ int flb_set_ghost_overlap(flb_block b, int enable) {
   CHECK_BLOCK(b);
   b->version++;
   const bool saved = b->ghost_overlap;
+  b->march = -1;
   b->ghost_overlap = enable != 0;
   const int rc = check_layout(b);
   if (rc != FLB_OK) b->ghost_overlap = saved;
@@ -801,6 +804,7 @@ int flb_upload_flags(flb_block b, const uint8_t* flags) {
   std::vector<uint8_t> saved;
   saved.swap(b->h_flags);
   b->h_flags.assign(flags, flags + b->N);
+  b->march = -1;
   const bool was_set = b->flags_set;
   b->flags_set = true;
   const int rc = check_layout(b);
@@ -1052,17 +1056,41 @@ static int watchdog_check(flb_block b) {
   return FLB_OK;
 }
 
+// n steps: passes of two steps where the block allows them (from parity 1, in
+// multiples of four steps, so that the state ends in the array it began in),
+// one launch per step otherwise.
+static int run_steps(flb_block b, int n) {
+  const bool march = n >= 5 - b->parity && march_ready(b);
+  int rc = FLB_OK;
+  while (n > 0) {
+    int k = 1;
+    if (march && b->parity == 1 && n >= 4) {
+      k = n / 4 * 4;
+      rc = march_run(b, k);
+    } else {
+      rc = launch_one(b);
+    }
+    if (rc) return rc;
+    b->parity ^= k & 1;
+    b->step += k;
+    n -= k;
+  }
+  return FLB_OK;
+}
+
 int flb_step(flb_block b, int n) {
   CHECK_BLOCK(b);
   if (n < 0) return fail(FLB_ERR_ARG, "negative step count");
   if (b->pending) return fail(FLB_ERR_STATE, "step while a Stream is pending");
   DeviceGuard g(b->device);
   Range range("flb_step");
-  for (int s = 0; s < n; ++s) {
-    int rc = launch_one(b);
+  for (int left = n; left > 0;) {
+    // up to the next watchdog check
+    int k = left;
+    if (b->watchdog > 0) k = int(std::min<int64_t>(k, b->watchdog - b->step % b->watchdog));
+    int rc = run_steps(b, k);
     if (rc) return rc;
-    b->parity ^= 1;
-    b->step += 1;
+    left -= k;
     if (b->watchdog > 0 && b->step % b->watchdog == 0 && (rc = watchdog_check(b))) return rc;
   }
   return FLB_OK;

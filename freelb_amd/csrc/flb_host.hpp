@@ -52,6 +52,8 @@ struct flb_block_s {
   int vec = 0;  // step kernel form: 0 automatic cell form, -1 row segments, -3 linear runs,
                 // 1/2/4 row form with that many cells per thread
   int wpb = 4;   // wavefronts per workgroup
+  void* d_alt = nullptr;   // second population array of the two-step march (flb_march.hip), scratch between calls
+  int march = -1;          // 1: the march may step the block, 0: not, -1: to be checked (flags, tasks or walls changed)
   uint64_t version = 0;  // bumped by every change a batch table must see
   uint64_t* d_links = nullptr;  // precomputed halfway wall links (slot layout)
   bool links_dirty = true;      // flags or halfway managers changed since d_links was built
@@ -135,6 +137,12 @@ inline bool level_due(int64_t count, int level, int max_level) {
 // Builds the block's wall-link words when flags or halfway managers changed
 // (enqueued on the block's stream); a no-op without halfway managers.
 int ensure_links(flb_block_s* b);
+
+// Two steps per pass (flb_march.hip): march_ready tells whether a run of
+// steps of the block may take it now, march_run advances a block at parity 1
+// by n steps (a multiple of 4).
+bool march_ready(flb_block_s* b);
+int march_run(flb_block_s* b, int n);
 
 // Block halo (flb_halo.hip): enqueue the exchange that follows a step leaving
 // the blocks at `parity`; refresh the device copy of the blocks' arguments;

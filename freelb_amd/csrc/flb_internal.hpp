@@ -89,6 +89,22 @@ struct KArgs {
   double cpl_rho0[kMaxCouplings];
 };
 
+// The two-step march (flb_march.hpp): target populations (slot 0 of direction
+// 0), tile extents and counts, planes per workgroup.
+struct MarchArgs {
+  void* dst;
+  int w, h;
+  int ntx, nty;
+  int zchunk, nz;  // planes per workgroup, workgroups along z
+  unsigned mask;   // flags of the updated cells, all of one dynamics
+  int dyn;
+  float cs;
+};
+constexpr int kMarchMaxRow = 130;  // widest ring row, w + 2
+// Threads of a march workgroup, one per cell of the tile and its ring: as many
+// as the LDS of a CU serves (32 values each, 132 KB).
+constexpr int march_threads(size_t elem) { return elem == 8 ? 512 : 1024; }
+
 // Launchers, one set per storage kind (defined in flb_inst_*.hip).
 #define FLB_DECLARE_LAUNCHERS(SUFFIX)                                                         \
   hipError_t launch_step_##SUFFIX(int q, int parity, int family, const KArgs& a,             \
@@ -104,6 +120,16 @@ struct KArgs {
   hipError_t launch_batch_##SUFFIX(int q, int parity, int family, bool per, const KArgs* tab, \
                                    const int64_t* wave0, const int* wblk, int nb,             \
                                    int64_t groups, int wpb, int grid, hipStream_t s);
+
+#define FLB_DECLARE_MARCH(SUFFIX) \
+  hipError_t launch_march_##SUFFIX(const KArgs& a, const MarchArgs& m, hipStream_t s);
+
+FLB_DECLARE_MARCH(f32)
+FLB_DECLARE_MARCH(f64)
+
+// Sets *open to 1 if a link of an updated cell leads to a cell that is not
+// updated and is no halfway wall link (D3Q19; left as it is otherwise).
+hipError_t launch_open_links(const KArgs& a, unsigned mask, uint32_t* open, hipStream_t s);
 
 FLB_DECLARE_LAUNCHERS(f32)
 FLB_DECLARE_LAUNCHERS(f16s)
