@@ -600,6 +600,8 @@ int flb_block_create(const flb_block_desc* desc, flb_block* out) {
     return fail(FLB_ERR_HIP, "initial clear failed");
   }
   default_rates(b);
+  readout_retain();
+  b->retained = true;
   *out = b;
   return FLB_OK;
 }
@@ -614,6 +616,7 @@ int flb_block_destroy(flb_block b) {
                   b->d_stage, b->d_alt, b->d_links, b->d_rho_old, b->d_u_old, b->d_res};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  if (b->retained) readout_release();
   delete b;
   return FLB_OK;
 }
@@ -944,11 +947,10 @@ static int download_pops(flb_block b, void* host, size_t host_real) {
   const size_t bytes = size_t(b->N) * size_t(b->desc.q) * b->real;
   int rc = ensure_stage(b, bytes);
   if (rc) return rc;
-  HIP_TRY(hipMemsetAsync(b->d_stage, 0, bytes, b->stream));
+  // the kernel writes every host cell, those outside the interior as 0
   KArgs a = make_args(b);
   HIP_TRY(launch_gather(b, a, b->d_stage));
-  HIP_TRY(hipMemcpyAsync(host, b->d_stage, bytes, hipMemcpyDeviceToHost, b->stream));
-  HIP_TRY(hipStreamSynchronize(b->stream));
+  HIP_TRY(readout(host, b->d_stage, bytes, false, b->stream));
   return FLB_OK;
 }
 
@@ -1102,13 +1104,21 @@ int flb_moments(flb_block b, uint8_t mask, void* rhou) {
   if (b->pending) return fail(FLB_ERR_STATE, "moments between ApplyCellDynamics and Stream");
   DeviceGuard g(b->device);
   const size_t bytes = size_t(b->N) * size_t(b->d + 1) * b->real;
+  // the kernel writes every host cell, the others' moments as 0
+  const KArgs a = make_args(b);
+  {
+    const DirectOut out(bytes);
+    if (out.ptr) {
+      HIP_TRY(launch_moments(b, a, mask, out.ptr));
+      HIP_TRY(hipStreamSynchronize(b->stream));
+      std::memcpy(rhou, out.ptr, bytes);
+      return FLB_OK;
+    }
+  }
   int rc = ensure_stage(b, bytes);
   if (rc) return rc;
-  HIP_TRY(hipMemsetAsync(b->d_stage, 0, bytes, b->stream));
-  KArgs a = make_args(b);
   HIP_TRY(launch_moments(b, a, mask, b->d_stage));
-  HIP_TRY(hipMemcpyAsync(rhou, b->d_stage, bytes, hipMemcpyDeviceToHost, b->stream));
-  HIP_TRY(hipStreamSynchronize(b->stream));
+  HIP_TRY(readout(rhou, b->d_stage, bytes, false, b->stream));
   return FLB_OK;
 }
 

@@ -785,6 +785,7 @@ struct flb_adjoint_s {
   double J = 0.0;
   float fwd_ms = 0.0f, bwd_ms = 0.0f;
   hipEvent_t e0 = nullptr, e1 = nullptr;
+  bool retained = false;  // holds the read-out buffers (readout_retain)
 };
 
 namespace {
@@ -1045,11 +1046,8 @@ int backward_impl(flb_adjoint_s* h, double* grad) {
     }
   }
   HIP_TRY(hipEventRecord(h->e1, h->stream));
-  std::vector<R> g(size_t(h->N));
-  HIP_TRY(hipMemcpyAsync(g.data(), h->d_grad, size_t(h->N) * sizeof(R), hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
+  HIP_TRY(readout(grad, h->d_grad, size_t(h->N) * sizeof(R), sizeof(R) == 4, h->stream));
   HIP_TRY(hipEventElapsedTime(&h->bwd_ms, h->e0, h->e1));
-  for (int64_t i = 0; i < h->N; ++i) grad[i] = double(g[size_t(i)]);
   return FLB_OK;
 }
 
@@ -1286,16 +1284,13 @@ int batch_backward_impl(flb_adjoint_batch_s* b, double* grad) {
     }
   }
   HIP_TRY(hipEventRecord(b->e1, b->stream));
-  std::vector<R> g(size_t(b->cells));
-  size_t off = 0;
+  double* out = grad;
   for (flb_adjoint_s* h : b->members) {
-    HIP_TRY(hipMemcpyAsync(g.data() + off, h->d_grad, size_t(h->N) * sizeof(R), hipMemcpyDeviceToHost, b->stream));
-    off += size_t(h->N);
+    HIP_TRY(readout(out, h->d_grad, size_t(h->N) * sizeof(R), sizeof(R) == 4, b->stream));
+    out += h->N;
   }
-  HIP_TRY(hipStreamSynchronize(b->stream));
   HIP_TRY(hipEventElapsedTime(&b->bwd_ms, b->e0, b->e1));
   for (flb_adjoint_s* h : b->members) h->bwd_ms = b->bwd_ms;
-  for (size_t i = 0; i < g.size(); ++i) grad[i] = double(g[i]);
   return FLB_OK;
 }
 
@@ -1342,6 +1337,8 @@ int flb_adjoint_create(const flb_adjoint_desc* desc, flb_adjoint* out) {
     flb_adjoint_destroy(h);
     return rc;
   }
+  readout_retain();
+  h->retained = true;
   *out = h;
   return FLB_OK;
 }
@@ -1358,6 +1355,7 @@ int flb_adjoint_destroy(flb_adjoint h) {
     if (p) (void)hipFree(p);
   if (h->e0) (void)hipEventDestroy(h->e0);
   if (h->e1) (void)hipEventDestroy(h->e1);
+  if (h->retained) readout_release();
   delete h;
   return FLB_OK;
 }
@@ -1469,15 +1467,7 @@ int flb_adjoint_state(flb_adjoint h, double* pops) {
   if (!h->last) return fail(FLB_ERR_STATE, "no forward run yet");
   DeviceGuard g(h->device);
   const size_t n = size_t(A::Q) * size_t(h->N);
-  if (h->real == 8) {
-    HIP_TRY(hipMemcpyAsync(pops, h->last, n * 8, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-  } else {
-    std::vector<float> t(n);
-    HIP_TRY(hipMemcpyAsync(t.data(), h->last, n * 4, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    for (size_t i = 0; i < n; ++i) pops[i] = double(t[i]);
-  }
+  HIP_TRY(readout(pops, h->last, n * h->real, h->real == 4, h->stream));
   // stored g = f - w; solid cells hold no populations
   for (int i = 0; i < A::Q; ++i) {
     const double w = flb::Lat<A::Q>::template w<double>(i);

@@ -54,6 +54,7 @@ struct flb_block_s {
   int wpb = 4;   // wavefronts per workgroup
   void* d_alt = nullptr;   // second population array of the two-step march (flb_march.hip), scratch between calls
   int march = -1;          // 1: the march may step the block, 0: not, -1: to be checked (flags, tasks or walls changed)
+  bool retained = false;   // holds the read-out buffers (readout_retain)
   uint64_t version = 0;  // bumped by every change a batch table must see
   uint64_t* d_links = nullptr;  // precomputed halfway wall links (slot layout)
   bool links_dirty = true;      // flags or halfway managers changed since d_links was built
@@ -143,6 +144,22 @@ int ensure_links(flb_block_s* b);
 // by n steps (a multiple of 4).
 bool march_ready(flb_block_s* b);
 int march_run(flb_block_s* b, int n);
+
+// Read-out to host memory (flb_readout.hip). readout: bytes of device memory
+// to the caller's array once the work enqueued on s is done; widen: FP32 on
+// the device, FP64 at the caller. Each block and adjoint box retains the
+// pinned buffers while it lives.
+void readout_retain();
+void readout_release();
+hipError_t readout(void* host, const void* dev, size_t bytes, bool widen, hipStream_t s);
+constexpr size_t kDirect = size_t(256) << 10;
+struct DirectOut {
+  void* ptr = nullptr;
+  explicit DirectOut(size_t bytes);
+  ~DirectOut();
+  DirectOut(const DirectOut&) = delete;
+  DirectOut& operator=(const DirectOut&) = delete;
+};
 
 // Block halo (flb_halo.hip): enqueue the exchange that follows a step leaving
 // the blocks at `parity`; refresh the device copy of the blocks' arguments;
