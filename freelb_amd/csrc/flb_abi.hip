@@ -669,7 +669,7 @@ int flb_set_tasks(flb_block b, const flb_task* tasks, int n) {
   std::memcpy(saved, b->tasks, sizeof saved);
   for (int t = 0; t < n; ++t) b->tasks[t] = tasks[t];
   b->ntasks = n;
-  b->march = -1;
+  b->march = b->closed = -1;
   int rc = check_layout(b);
   if (rc != FLB_OK) {
     std::memcpy(b->tasks, saved, sizeof saved);
@@ -707,7 +707,7 @@ int flb_set_halfway_bc(flb_block b, const flb_hwbc* bcs, int n) {
   for (int k = 0; k < n; ++k) b->bcs[k] = bcs[k];
   b->nbc = n;
   b->links_dirty = true;
-  b->march = -1;
+  b->march = b->closed = -1;
   for (int k = 0; k < n; ++k)
     if (bcs[k].kind == FLB_HWBC_ANTI) return ensure_fields(b);  // the wall value is the RHO field
   return FLB_OK;
@@ -775,7 +775,7 @@ int flb_set_ghost_overlap(flb_block b, int enable) {
   CHECK_BLOCK(b);
   b->version++;
   const bool saved = b->ghost_overlap;
-  b->march = -1;
+  b->march = b->closed = -1;
   b->ghost_overlap = enable != 0;
   const int rc = check_layout(b);
   if (rc != FLB_OK) b->ghost_overlap = saved;
@@ -807,7 +807,7 @@ int flb_upload_flags(flb_block b, const uint8_t* flags) {
   std::vector<uint8_t> saved;
   saved.swap(b->h_flags);
   b->h_flags.assign(flags, flags + b->N);
-  b->march = -1;
+  b->march = b->closed = -1;
   const bool was_set = b->flags_set;
   b->flags_set = true;
   const int rc = check_layout(b);

@@ -100,6 +100,10 @@ struct MarchArgs {
   int dyn;
   float cs;
 };
+// Workgroup of a batch's march: workgroup wg of block `block`.
+struct MarchWg {
+  int block, wg;
+};
 constexpr int kMarchMaxRow = 130;  // widest ring row, w + 2
 // Threads of a march workgroup, one per cell of the tile and its ring: as many
 // as the LDS of a CU serves (32 values each, 132 KB).
@@ -121,8 +125,10 @@ constexpr int march_threads(size_t elem) { return elem == 8 ? 512 : 1024; }
                                    const int64_t* wave0, const int* wblk, int nb,             \
                                    int64_t groups, int wpb, int grid, hipStream_t s);
 
-#define FLB_DECLARE_MARCH(SUFFIX) \
-  hipError_t launch_march_##SUFFIX(const KArgs& a, const MarchArgs& m, hipStream_t s);
+#define FLB_DECLARE_MARCH(SUFFIX)                                                                  \
+  hipError_t launch_march_##SUFFIX(const KArgs& a, const MarchArgs& m, hipStream_t s);             \
+  hipError_t launch_march_batch_##SUFFIX(int dyn, bool per, const KArgs* tab, const MarchArgs* mt, \
+                                         const MarchWg* wgs, unsigned n, int back, hipStream_t s);
 
 FLB_DECLARE_MARCH(f32)
 FLB_DECLARE_MARCH(f64)

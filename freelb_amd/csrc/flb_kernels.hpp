@@ -830,6 +830,25 @@ __global__ __launch_bounds__(kMaxThreads) void k_step_cell(KArgs a) {
   cell_update<Q, S, PAR, FAM, PER, BUF>(a, gw, lane);
 }
 
+// Pointers read from a table in memory are generic to the compiler, which
+// then forms flat loads: they hold up the LDS counter and take a wider address
+// path. Those of a block are all device memory.
+template <class T>
+__device__ __forceinline__ T* in_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<uintptr_t>(p);
+}
+__device__ __forceinline__ KArgs in_global(const KArgs& t) {
+  KArgs a = t;
+  a.pops = in_global(t.pops);
+  a.flags = in_global(t.flags);
+  a.rho_f = in_global(t.rho_f);
+  a.u_f = in_global(t.u_f);
+  a.links = in_global(t.links);
+  a.u_ext = in_global(t.u_ext);
+  for (int k = 0; k < kMaxCouplings; ++k) a.cpl_rho[k] = in_global(t.cpl_rho[k]);
+  return a;
+}
+
 // ---------------------------------------------------------------------------
 // The batched step: many blocks of one lattice and storage kind in one launch.
 // tab[e] holds block e's kernel arguments and wave0[e] the number of

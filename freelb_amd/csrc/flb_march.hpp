@@ -72,20 +72,23 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t march_rsrc(const KArgs& a, siz
   return pop_rsrc(a, elem, u);
 }
 
+// One ring row and cell of slack at both ends for the shifted reads of ring lanes.
+constexpr int kMarchSlack = kMarchMaxRow + 1;
+template <class S>
+constexpr int kMarchLds = 2 * kMarchPlanes * march_threads(sizeof(typename S::E)) + 2 * kMarchSlack;
+
+// Workgroup wg of a block's march.
 template <class S, int DYN, bool PER>
-__global__ __launch_bounds__(march_threads(sizeof(typename S::E))) void k_step_march(KArgs a, MarchArgs m) {
+__device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, unsigned wg, typename S::E* lds) {
   constexpr int Q = 19;
   constexpr int NT = march_threads(sizeof(typename S::E));
   constexpr int FAM = DYN == DYN_BGK ? FAM_BGK : FAM_FULL;
   using R = typename S::R;
   using E = typename S::E;
   constexpr uint32_t el = sizeof(E);
-  // one ring row and cell of slack at both ends for the shifted reads of ring lanes
-  constexpr int kSlack = kMarchMaxRow + 1;
-  __shared__ E lds[2 * kMarchPlanes * NT + 2 * kSlack];
+  constexpr int kSlack = kMarchSlack;
 
   const int tid = int(threadIdx.x);
-  const unsigned wg = xcd_block(blockIdx.x, gridDim.x);
   const int pw = m.w + 2;
   const int tx = int(wg % unsigned(m.ntx)), wy = int(wg / unsigned(m.ntx));
   const int ty = wy % m.nty, zc = wy / m.nty;
@@ -304,6 +307,34 @@ __global__ __launch_bounds__(march_threads(sizeof(typename S::E))) void k_step_m
   }
 }
 
+template <class S, int DYN, bool PER>
+__global__ __launch_bounds__(march_threads(sizeof(typename S::E))) void k_step_march(KArgs a, MarchArgs m) {
+  __shared__ typename S::E lds[kMarchLds<S>];
+  march_tile<S, DYN, PER>(a, m, xcd_block(blockIdx.x, gridDim.x), lds);
+}
+
+// The march of many blocks in one launch, a block and its workgroup for every
+// workgroup. back: from the second arrays to the blocks' own. The table's
+// order is that of dispatch, longest workgroup first: as contiguous runs per
+// XCD, in the blocks' order, 256 cavities of 43.2 M cells take 1.195 ms per
+// step against 1.093, 40 of 6.3 M 176 us against 170.
+template <class S, int DYN, bool PER>
+__global__ __launch_bounds__(march_threads(sizeof(typename S::E))) void k_march_batch(
+    const KArgs* __restrict__ tab, const MarchArgs* __restrict__ mt, const MarchWg* __restrict__ wgs, int back) {
+  __shared__ typename S::E lds[kMarchLds<S>];
+  const int e = __builtin_amdgcn_readfirstlane(wgs[blockIdx.x].block);
+  const unsigned wg = unsigned(__builtin_amdgcn_readfirstlane(wgs[blockIdx.x].wg));
+  KArgs a = in_global(tab[e]);
+  MarchArgs m = mt[e];
+  m.dst = in_global(m.dst);
+  if (back) {
+    void* const p = a.pops;
+    a.pops = m.dst;
+    m.dst = p;
+  }
+  march_tile<S, DYN, PER>(a, m, wg, lds);
+}
+
 // Counts the links of updated cells that lead to a cell that is not updated
 // (no task, or beyond a non-periodic face) and are no halfway wall links.
 template <int Q, bool PER>
@@ -352,13 +383,37 @@ hipError_t launch_march(const KArgs& a, const MarchArgs& m, hipStream_t s) {
   }
 }
 
+template <class S, int DYN>
+hipError_t march_batch_dyn(bool per, const KArgs* tab, const MarchArgs* mt, const MarchWg* wgs, unsigned n, int back,
+                           hipStream_t s) {
+  const dim3 grid(n), block(march_threads(sizeof(typename S::E)));
+  if (per) hipLaunchKernelGGL((k_march_batch<S, DYN, true>), grid, block, 0, s, tab, mt, wgs, back);
+  else hipLaunchKernelGGL((k_march_batch<S, DYN, false>), grid, block, 0, s, tab, mt, wgs, back);
+  return hipGetLastError();
+}
+
+template <class S>
+hipError_t launch_march_batch(int dyn, bool per, const KArgs* tab, const MarchArgs* mt, const MarchWg* wgs, unsigned n,
+                              int back, hipStream_t s) {
+  switch (dyn) {
+    case DYN_BGK: return march_batch_dyn<S, DYN_BGK>(per, tab, mt, wgs, n, back, s);
+    case DYN_BGK_FORCE: return march_batch_dyn<S, DYN_BGK_FORCE>(per, tab, mt, wgs, n, back, s);
+    case DYN_SMAG_MRT: return march_batch_dyn<S, DYN_SMAG_MRT>(per, tab, mt, wgs, n, back, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 }  // namespace kern
 }  // namespace flb
 
-// Defines the march launcher of flb_internal.hpp for one storage kind.
+// Defines the march launchers of flb_internal.hpp for one storage kind.
 #define FLB_DEFINE_MARCH(SUFFIX, STORE)                                                            \
   namespace flb {                                                                                  \
   hipError_t launch_march_##SUFFIX(const KArgs& a, const MarchArgs& m, hipStream_t s) {            \
     return kern::launch_march<STORE>(a, m, s);                                                     \
+  }                                                                                                \
+  hipError_t launch_march_batch_##SUFFIX(int dyn, bool per, const KArgs* tab, const MarchArgs* mt, \
+                                         const MarchWg* wgs, unsigned n, int back, hipStream_t s) { \
+    return kern::launch_march_batch<STORE>(dyn, per, tab, mt, wgs, n, back, s);                 \
   }                                                                                                \
   }

@@ -8,7 +8,7 @@ cavity here is compared with it directly."""
 import numpy as np
 import pytest
 
-from freelb_amd import BlockLattice, HalfwayBB, Key_TypePair, abi
+from freelb_amd import BlockLattice, BlockLatticeManager, HalfwayBB, Key_TypePair, abi
 from freelb_amd.cases import FLUID, VOID, cavity_block, cavity_flags
 from oracle import oracle as O
 from tests.gpu_case import gpu_lattice
@@ -110,3 +110,64 @@ def test_watchdog_inside_a_run():
         lat.set_watchdog(7)
         return lat
     _agree(make, (20, 3))
+
+
+# large enough together that the batch takes passes of two steps
+BATCH_DIMS = [(16, 16, 16), (96, 93, 97), (63, 90, 77), (64, 62, 64), (131, 60, 83), (5, 6, 7), (40, 81, 4),
+              (60, 75, 90), (96, 91, 94)]
+
+
+def _batch_agrees(make, runs, between=lambda k, blocks: None):
+    """BlockLatticeManager runs against the blocks stepped one at a time; runs of "replay" replay
+    a recorded graph of 10 steps."""
+    a, b = make(), make()
+    try:
+        with BlockLatticeManager(a) as m:
+            m.capture(10)
+            for k, n in enumerate(runs):
+                between(k, a)
+                between(k, b)
+                if n == "replay":
+                    m.replay()
+                else:
+                    m.step(n)
+                m.synchronize()
+                for lat in b:
+                    for _ in range(10 if n == "replay" else n):
+                        lat.step(1)
+                for x, y in zip(a, b):
+                    assert np.array_equal(x.pops(), y.pops()), (k, n, x.dims)
+    finally:
+        for lat in a + b:
+            lat.close()
+
+
+@pytest.mark.parametrize("storage,collision", [("f32", "bgk"), ("f64", "bgk"), ("f32", "mrt_les")])
+def test_batch_runs_equal_single_steps(storage, collision):
+    def make():
+        return [cavity_block(d, storage=storage, collision=collision, tau=0.6 + 0.01 * k, u_lid=0.03, u0_amp=0.02,
+                             seed=k) for k, d in enumerate(BATCH_DIMS)]
+    _batch_agrees(make, ("replay", 5, 1, "replay", 12))
+
+
+def test_batch_of_mixed_periodic_boxes():
+    per = [(False, False, False), (True, False, False), (False, True, True), (True, True, True)]
+
+    def make():
+        return [_box(d, per[k % 4], "f32", abi.DYN_BGK_FORCE, k % 2 == 0) for k, d in enumerate(BATCH_DIMS)]
+    _batch_agrees(make, ("replay", 7, 1, "replay"))
+
+
+def test_batch_replay_after_changed_walls():
+    """A recorded graph replayed after a change that its passes of two steps no longer serve, and
+    after the change is taken back."""
+    def make():
+        return [cavity_block(d, tau=0.7, u_lid=0.03, u0_amp=0.02, seed=k) for k, d in enumerate(BATCH_DIMS)]
+
+    def between(k, blocks):
+        if k == 1:
+            blocks[3].set_halfway_bc([HalfwayBB(4, VOID)])
+        elif k == 2:
+            blocks[3].set_halfway_bc([HalfwayBB(4, VOID), HalfwayBB(8, VOID, True)])
+            blocks[1].set_omega(1.2)
+    _batch_agrees(make, ("replay", "replay", "replay", 6), between)
