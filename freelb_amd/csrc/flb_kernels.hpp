@@ -461,13 +461,16 @@ __device__ __forceinline__ void st_pop(E* p, E v) {
 // from e0 to the end of the allocation, capped at 4 GiB - 1 bytes; the
 // offsets the kernels form stay below 2 GiB (KArgs::buf, checked on the host
 // for the block's strides), so allocations of any size take this form.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pop_rsrc(const KArgs& a, size_t elem, int64_t e0) {
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pop_rsrc(void* pops, uint64_t total, size_t elem, int64_t e0) {
   const uint64_t off = uint64_t(e0) * elem;
-  const uint64_t rest = a.pop_total - off;
+  const uint64_t rest = total - off;
   const uint32_t nrec = rest < 0xFFFFFFFFull ? uint32_t(rest) : 0xFFFFFFFFu;
   // word 3 of a raw (unformatted) buffer descriptor on the gfx9 family
-  return __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(a.pops) - kFrontPad * elem + off, 0, int(nrec),
+  return __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(pops) - kFrontPad * elem + off, 0, int(nrec),
                                            0x00020000);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pop_rsrc(const KArgs& a, size_t elem, int64_t e0) {
+  return pop_rsrc(a.pops, a.pop_total, elem, e0);
 }
 
 template <int Q, class S, int PAR, int FAM, bool PER, bool BUF = false>
@@ -828,25 +831,6 @@ __global__ __launch_bounds__(kMaxThreads) void k_step_cell(KArgs a) {
   const int wib = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int gw = int(xcd_block(blockIdx.x, unsigned(a.nblocks))) * a.wpb + wib;
   cell_update<Q, S, PAR, FAM, PER, BUF>(a, gw, lane);
-}
-
-// Pointers read from a table in memory are generic to the compiler, which
-// then forms flat loads: they hold up the LDS counter and take a wider address
-// path. Those of a block are all device memory.
-template <class T>
-__device__ __forceinline__ T* in_global(T* p) {
-  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<uintptr_t>(p);
-}
-__device__ __forceinline__ KArgs in_global(const KArgs& t) {
-  KArgs a = t;
-  a.pops = in_global(t.pops);
-  a.flags = in_global(t.flags);
-  a.rho_f = in_global(t.rho_f);
-  a.u_f = in_global(t.u_f);
-  a.links = in_global(t.links);
-  a.u_ext = in_global(t.u_ext);
-  for (int k = 0; k < kMaxCouplings; ++k) a.cpl_rho[k] = in_global(t.cpl_rho[k]);
-  return a;
 }
 
 // ---------------------------------------------------------------------------

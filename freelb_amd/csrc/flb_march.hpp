@@ -66,10 +66,22 @@ struct MarchCell {
 
 // pop_rsrc with its words held to scalar registers (the walk's plane index is
 // uniform, which the compiler does not always see).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t march_rsrc(const KArgs& a, size_t elem, int64_t e0) {
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t march_rsrc(void* pops, uint64_t total, size_t elem, int64_t e0) {
   const int64_t u = (int64_t(__builtin_amdgcn_readfirstlane(int(e0 >> 32))) << 32) |
                     uint32_t(__builtin_amdgcn_readfirstlane(int(e0)));
-  return pop_rsrc(a, elem, u);
+  return pop_rsrc(pops, total, elem, u);
+}
+
+// Tables in memory that no kernel writes (batches): uniform reads are scalar
+// loads also after a store, and what they point to is device memory (else the
+// compiler forms flat accesses, which wait on the LDS counter too).
+template <class T>
+__device__ __forceinline__ const T* in_const(const T* p) {
+  return (const T*)(const __attribute__((address_space(4))) T*)reinterpret_cast<uintptr_t>(p);
+}
+template <class T>
+__device__ __forceinline__ T* in_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<uintptr_t>(p);
 }
 
 // One ring row and cell of slack at both ends for the shifted reads of ring lanes.
@@ -77,9 +89,10 @@ constexpr int kMarchSlack = kMarchMaxRow + 1;
 template <class S>
 constexpr int kMarchLds = 2 * kMarchPlanes * march_threads(sizeof(typename S::E)) + 2 * kMarchSlack;
 
-// Workgroup wg of a block's march.
+// Workgroup wg of a block's march from the populations src to dst.
 template <class S, int DYN, bool PER>
-__device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, unsigned wg, typename S::E* lds) {
+__device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, void* src, void* dst, unsigned wg,
+                                           typename S::E* lds) {
   constexpr int Q = 19;
   constexpr int NT = march_threads(sizeof(typename S::E));
   constexpr int FAM = DYN == DYN_BGK ? FAM_BGK : FAM_FULL;
@@ -158,7 +171,7 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
   };
   auto cell_flag = [&](int z) -> unsigned {
     unsigned fl = 0;
-    if (z <= zb && live(z) && upd) fl = a.flags[sxy + int(a.plane) * wrap(z)];
+    if (z <= zb && live(z) && upd) fl = in_global(a.flags)[sxy + int(a.plane) * wrap(z)];
     return fl;
   };
   auto cell_info = [&](int z, unsigned fl) {
@@ -166,7 +179,7 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
     if (z > zb || !live(z) || !(fl & m.mask)) return c;
     c.lk = 1u;
     if (fl & a.bcany) {
-      const uint64_t l = a.links[sxy + int(a.plane) * wrap(z)];
+      const uint64_t l = in_global(a.links)[sxy + int(a.plane) * wrap(z)];
       c.lm = uint32_t(l >> 32);
       c.lk = 1u | uint32_t(l) | c.lm;
     }
@@ -180,7 +193,7 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
     const unsigned lk = c.lk;
     if (!lk) return;
     if constexpr (PER) {
-      const auto rs = march_rsrc(a, el, int64_t(kFrontPad) - 1);
+      const auto rs = march_rsrc(src, a.pop_total, el, int64_t(kFrontPad) - 1);
       const uint32_t zo[3] = {uint32_t(wrap(z - 1) * zp) * el, uint32_t(wrap(z) * zp) * el,
                               uint32_t(wrap(z + 1) * zp) * el};
 #pragma unroll
@@ -193,7 +206,7 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
           if ((lk >> opp(i)) & 1u) f[i] = bld_pop_s<1, E>(rs, X[1] + Y[1], uint32_t(i * dp) * el + zo[1]);
       }
     } else {
-      const auto rs = march_rsrc(a, el, int64_t(kFrontPad) + a.zpop * z + int64_t(a.ypop) * yt - B);
+      const auto rs = march_rsrc(src, a.pop_total, el, int64_t(kFrontPad) + a.zpop * z + int64_t(a.ypop) * yt - B);
       if (__ballot(lk > 1u) == 0) {
 #pragma unroll
         for (int i = 0; i < Q; ++i)
@@ -212,8 +225,6 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
   };
 
   const R om = R(a.omega), _om = R(1) - om;
-  KArgs t = a;
-  t.pops = m.dst;
 
   MarchCell cur = cell_info(za - 1, cell_flag(za - 1));
   MarchCell next = cell_info(za, cell_flag(za));
@@ -280,7 +291,7 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
 #pragma unroll
       for (int i = 0; i < Q; ++i) f[i] = pop_dec<Q, S>(P[i], i);
       collide<Q, R, FAM, kDev<Q, S>>(a, sxy + int(a.plane) * (z - 1), DYN, m.cs, f, om, _om);
-      const auto rd = march_rsrc(t, el, int64_t(kFrontPad) + a.zpop * (z - 1) + int64_t(a.ypop) * yt);
+      const auto rd = march_rsrc(dst, a.pop_total, el, int64_t(kFrontPad) + a.zpop * (z - 1) + int64_t(a.ypop) * yt);
 #pragma unroll
       for (int i = 0; i < Q; ++i) bst_pop_s<2, E>(rd, own, uint32_t(opp(i) * dp) * el, pop_enc<Q, S>(f[i], i));
     }
@@ -310,7 +321,7 @@ __device__ __forceinline__ void march_tile(const KArgs& a, const MarchArgs& m, u
 template <class S, int DYN, bool PER>
 __global__ __launch_bounds__(march_threads(sizeof(typename S::E))) void k_step_march(KArgs a, MarchArgs m) {
   __shared__ typename S::E lds[kMarchLds<S>];
-  march_tile<S, DYN, PER>(a, m, xcd_block(blockIdx.x, gridDim.x), lds);
+  march_tile<S, DYN, PER>(a, m, a.pops, m.dst, xcd_block(blockIdx.x, gridDim.x), lds);
 }
 
 // The march of many blocks in one launch, a block and its workgroup for every
@@ -322,17 +333,12 @@ template <class S, int DYN, bool PER>
 __global__ __launch_bounds__(march_threads(sizeof(typename S::E))) void k_march_batch(
     const KArgs* __restrict__ tab, const MarchArgs* __restrict__ mt, const MarchWg* __restrict__ wgs, int back) {
   __shared__ typename S::E lds[kMarchLds<S>];
+  wgs = in_const(wgs);
   const int e = __builtin_amdgcn_readfirstlane(wgs[blockIdx.x].block);
   const unsigned wg = unsigned(__builtin_amdgcn_readfirstlane(wgs[blockIdx.x].wg));
-  KArgs a = in_global(tab[e]);
-  MarchArgs m = mt[e];
-  m.dst = in_global(m.dst);
-  if (back) {
-    void* const p = a.pops;
-    a.pops = m.dst;
-    m.dst = p;
-  }
-  march_tile<S, DYN, PER>(a, m, wg, lds);
+  const KArgs& a = in_const(tab)[e];
+  const MarchArgs& m = in_const(mt)[e];
+  march_tile<S, DYN, PER>(a, m, back ? m.dst : a.pops, back ? a.pops : m.dst, wg, lds);
 }
 
 // Counts the links of updated cells that lead to a cell that is not updated
