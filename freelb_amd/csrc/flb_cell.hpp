@@ -23,6 +23,18 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) {
   return xcd * per + (xcd < rem ? xcd : rem) + slot;
 }
 
+// Tables in memory that no kernel writes (batches, exchanges): uniform reads are
+// scalar loads also after a store, and what they point to is device memory (else the
+// compiler forms flat accesses, which wait on the LDS counter too).
+template <class T>
+__device__ __forceinline__ const T* in_const(const T* p) {
+  return (const T*)(const __attribute__((address_space(4))) T*)reinterpret_cast<uintptr_t>(p);
+}
+template <class T>
+__device__ __forceinline__ T* in_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<uintptr_t>(p);
+}
+
 // ---------------------------------------------------------------------------
 // Velocity sets in FreeLB's order (lbm/lattice_set.h:168-194 D2Q9,
 // 259-296 D3Q19). Opposite pairs are (2k-1, 2k).

@@ -86,10 +86,11 @@ struct flb_halo_s {
   size_t elem = 4;
   std::vector<flb::KArgs> h_tab;
   std::vector<flb::HaloItem> h_items;
-  std::vector<int64_t> h_cell0;
+  int64_t cells = 0;  // of all items
+  unsigned wgs = 0;
   flb::KArgs* d_tab = nullptr;
   flb::HaloItem* d_items = nullptr;
-  int64_t* d_cell0 = nullptr;
+  flb::HaloWg* d_wg = nullptr;
 };
 
 namespace flbh {

@@ -151,6 +151,10 @@ struct HaloItem {
   int nx, ny, nz;
   int sx, sy, sz;
 };
+// A wavefront of the exchange: 64 cells of an item from `cell` on, x fastest.
+struct HaloWg {
+  int item, cell;
+};
 
 // Halfway wall links of every updated cell into links (slot layout), see k_links.
 hipError_t launch_links(int q, const KArgs& a, uint64_t* links, hipStream_t s);

@@ -72,18 +72,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t march_rsrc(void* pops, uint64_
   return pop_rsrc(pops, total, elem, u);
 }
 
-// Tables in memory that no kernel writes (batches): uniform reads are scalar
-// loads also after a store, and what they point to is device memory (else the
-// compiler forms flat accesses, which wait on the LDS counter too).
-template <class T>
-__device__ __forceinline__ const T* in_const(const T* p) {
-  return (const T*)(const __attribute__((address_space(4))) T*)reinterpret_cast<uintptr_t>(p);
-}
-template <class T>
-__device__ __forceinline__ T* in_global(T* p) {
-  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<uintptr_t>(p);
-}
-
 // One ring row and cell of slack at both ends for the shifted reads of ring lanes.
 constexpr int kMarchSlack = kMarchMaxRow + 1;
 template <class S>

@@ -63,6 +63,29 @@ def _compare(ref, blocks, boxes, dims, sel):
         assert np.array_equal(mine[:, m], want[:, m]), f"block at {box}"
 
 
+@pytest.mark.parametrize("ny,nz", [(9, 7), (8, 8), (13, 5), (16, 8), (43, 3)])
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+def test_exchanged_faces_around_whole_wavefronts(ny, nz, storage):
+    """Faces of 63, 64, 65, 128 and 129 cells between blocks split along x (64 cells per wavefront)."""
+    case, p = O.cavity_case("hw", 10, ny, nz)
+    dims = (case.nx, case.ny, case.nz)
+    glob = gpu_lattice(case, storage, p)
+    blocks, origins, boxes = _split_cavity(case, p, ([5, 6], [], []), storage)
+    halo = BlockHalo(blocks, origins)
+    try:
+        for n in (1, 2, 4):
+            glob.step(n)
+            for _ in range(n):
+                for b in blocks:
+                    b.step(1)
+                halo.exchange()
+            _compare(glob.pops(), blocks, boxes, dims, case.flags != O.VOID)
+    finally:
+        halo.close()
+        for b in blocks + [glob]:
+            b.close()
+
+
 @pytest.mark.parametrize("mode", ["hw", "fw", "smag"])
 @pytest.mark.parametrize("storage", ["f32", "f16s"])
 def test_split_cavity_matches_single_block(mode, storage):
