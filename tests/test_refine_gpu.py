@@ -55,6 +55,22 @@ def test_refined_cavity_matches_oracle(lattice, n, cell, p0, p1, storage):
         fine.close()
 
 
+@pytest.mark.parametrize("lattice,m", [("d2q9", 1), ("d2q9", 2), ("d2q9", 5), ("d3q19", 1), ("d3q19", 2), ("d3q19", 3)])
+def test_smallest_patches_match_oracle(lattice, m):
+    """Exchanges of fewer than 16 items, of 16, and with remainders (16 items per workgroup)."""
+    rc = O.RefinedCavity(lattice, 13, 13, 13, 1, 5, 5 + m)
+    coarse, fine, ref = gpu_refined(rc)
+    try:
+        for k in (1, 2, 3):
+            rc.run(k)
+            ref.run(k)
+            _check(rc, coarse, fine)
+    finally:
+        ref.close()
+        coarse.close()
+        fine.close()
+
+
 # Hierarchies of several patches and levels: (lattice, n, patches), patches as
 # (parent block, origin in the parent's cells, extent in parent cells)
 HIERARCHIES = [
