@@ -14,7 +14,8 @@
 //   solid or outside a non-periodic axis (halfway bounce-back,
 //   boundary/bounce_back_boundary.h:169-181).
 // Objective: J = (1/T) sum_{t=1..T} sum_{x on plane x = outlet} sum_i c_ix f_i(x, t),
-// summed in FP64 inside the forward step that writes state t (obj_fold).
+// in FP64: the plane's cells by the forward step that reads state t (the last
+// state's by k_obj_state), their sums by k_obj_sum.
 //
 // Adjoint. With lambda^t the adjoint of f^t and mu^t = P^T lambda^{t+1} the
 // adjoint of the post-collision populations (mu_i(x) = lambda_i(x + c_i), or
@@ -26,6 +27,9 @@
 //   B     = 3 V - 3 M u + 9 T u          (= sum mu_i dF_i/dF = sum mu_i dfeq_i/du / rho)
 //   A_rho = omega [M (1 - 1.5 u.u) + 3 V.u + 4.5 u.T.u] - (1 - omega/2) alpha s (B . u)
 //   A_u   = omega rho B + (1 - omega/2) [-3 M F + 9 T F - alpha s rho B].
+// Kept between the steps is mu (each step reads its own cells' and stores
+// lambda where it is the neighbours' mu), so both directions of time have the
+// same form, read - collide - push, and share the passes of two steps.
 // No reference implementation exists (FreeLB has no adjoint); the derivation
 // is pinned by FP64 finite differences and by autodiff of an FP64 CPU model.
 //
@@ -49,6 +53,7 @@
 #include "../../include/flb_abi.h"
 #include "flb_cell.hpp"
 #include "flb_host.hpp"
+#include "flb_internal.hpp"
 
 namespace flb {
 namespace adj {
@@ -365,19 +370,39 @@ __device__ __forceinline__ void pin(const R (&v)[M]) {
 }
 
 // ---- forward step: state src -> dst (push, halfway bounce-back) -------------
-// OBJ: also the cell's share of the objective of state dst, the FP64 sum, in
-// direction order, of c_jx times every value it pushes into population j of a
-// cell on the outlet plane (its own, across a wall link, or the neighbour's);
-// every population of the plane's cells is pushed by exactly one cell.
-// Wavefronts without a wall link store without testing links, and those with
-// no cell on or beside the outlet plane skip the objective.
+// The value that lands in dst when direction i of a cell moves with velocity
+// c_g (g = i forward, opp(i) backward): its own opposite across a wall link,
+// the neighbour's slot otherwise.
+template <class R, bool WALLS>
+__device__ __forceinline__ void push(const AdjArgs<R>& a, const Hops& h, uint32_t lk, R* __restrict__ dst, int i,
+                                     int g, R v) {
+  if (WALLS && i != 0 && ((lk >> g) & 1u))
+    st_pop(dst, a.N, opp(i), h.o, v);
+  else
+    st_pop(dst, a.N, i, hop(h, a, g), v);
+}
+
+// A cell's share of the objective: sum of c_ix f_i in direction order.
+template <class R>
+__device__ __forceinline__ double obj_cell(const R (&g)[Q]) {
+  double c = 0.0;
+#pragma unroll
+  for (int i = 1; i < Q; ++i) {
+    if (Lat<Q>::cx(i) > 0) c += double(g[i]);
+    else if (Lat<Q>::cx(i) < 0) c -= double(g[i]);
+  }
+  return c;
+}
+
+// obj: the shares of the outlet plane's cells of the source state, [ny * nz]
+// (null: not wanted). Every one is written (0 by a solid cell).
+// Wavefronts without a wall link store without testing links.
 // MOM: also the moment record of the source state, [4][N]: rho - 1 and u
 // (all the adjoint step needs of it).
-template <class R, bool OBJ, bool MOM>
-__device__ __forceinline__ double fwd_cell(const AdjArgs<R>& a, const R* __restrict__ src,
-                                           R* __restrict__ dst, R* __restrict__ mom, int64_t id) {
-  double c = 0.0;
-  if (id >= a.N) return c;
+template <class R, bool MOM>
+__device__ __forceinline__ void fwd_cell(const AdjArgs<R>& a, const R* __restrict__ src, R* __restrict__ dst,
+                                         R* __restrict__ mom, double* __restrict__ obj, int64_t id) {
+  if (id >= a.N) return;
   // the populations are read together with the link word (every offset is in
   // bounds, a solid cell's too), not after it
   const Hops h = hops(a, uint32_t(id));
@@ -390,10 +415,11 @@ __device__ __forceinline__ double fwd_cell(const AdjArgs<R>& a, const R* __restr
     lk = ((gptr<const uint32_t>)a.link)[id];
     pin(g);
     asm volatile("" : "+v"(lk));  // tests of lk come after every load above
-    if (lk & 1u) return c;
   } else {
     lk = face_links(a, h);
   }
+  if (obj && h.x == uint32_t(a.outlet)) obj[h.y + uint32_t(a.ny) * h.z] = (lk & 1u) ? 0.0 : obj_cell(g);
+  if (lk & 1u) return;
   R drho, rho, u[3], F[3], irD;
   force_state(g, s, a, drho, rho, u, F, irD);
   if constexpr (MOM) {
@@ -402,34 +428,10 @@ __device__ __forceinline__ double fwd_cell(const AdjArgs<R>& a, const R* __restr
     for (int d = 0; d < 3; ++d) st_pop(mom, a.N, d + 1, h.o, u[d]);
   }
   R v[Q];
-  if (__ballot(lk != 0u) == 0) {
-    post_collision(g, drho, rho, u, F, a, v, [&](int i, R x) { st_pop(dst, a.N, i, hop(h, a, i), x); });
-  } else {
-    post_collision(g, drho, rho, u, F, a, v, [&](int i, R x) {
-      if (i != 0 && ((lk >> i) & 1u))
-        st_pop(dst, a.N, opp(i), h.o, x);
-      else
-        st_pop(dst, a.N, i, hop(h, a, i), x);
-    });
-  }
-  if constexpr (OBJ) {
-    const uint32_t x = h.x, last = uint32_t(a.nx - 1), out = uint32_t(a.outlet);
-    const bool on0 = x == out, onp = (x == last ? 0u : x + 1u) == out, onm = (x == 0u ? last : x - 1u) == out;
-    if (__ballot(on0 || onp || onm) != 0) {
-#pragma unroll
-      for (int i = 1; i < Q; ++i) {
-        const int cx = Lat<Q>::cx(i);
-        if (cx == 0) continue;
-        const bool wall = (lk >> i) & 1u;
-        // across a wall the value lands in opp(i) of this cell (c_x = -cx)
-        const bool hit = wall ? on0 : (cx > 0 ? onp : onm);
-        const bool up = wall ? cx < 0 : cx > 0;
-        const double dv = double(v[i]);
-        if (hit) c += up ? dv : -dv;
-      }
-    }
-  }
-  return c;
+  if (__ballot(lk != 0u) == 0)
+    post_collision(g, drho, rho, u, F, a, v, [&](int i, R x) { push<R, false>(a, h, lk, dst, i, i, x); });
+  else
+    post_collision(g, drho, rho, u, F, a, v, [&](int i, R x) { push<R, true>(a, h, lk, dst, i, i, x); });
 }
 
 // Fixed-order sum of v over the workgroup (every thread calls it; thread 0
@@ -448,41 +450,43 @@ __device__ __forceinline__ double wg_sum(double v) {
   return s;
 }
 
-// Every thread of the workgroup holding chunk `chunk` (256 cells of the box)
-// calls this with its cell's share; the chunk's fixed-order sum goes to
-// partial[chunk]. Nothing is shared between workgroups (no atomics): k_obj_sum
-// adds the chunks of every step after the run, in chunk order, so the sums do
-// not depend on the order in which workgroups run, and a box stepped in a
-// batch (chunks aligned to 256 cells there too) gives the same bits as
-// stepped alone.
-__device__ __forceinline__ void obj_fold(double c, double* __restrict__ partial, unsigned chunk) {
-  const double s = wg_sum(c);
-  if (threadIdx.x == 0) partial[chunk] = s;
-}
-
-// Workgroup t (t = 1 .. T): jt[t] = sum of the nchunks partial sums of step t
-// (partial + t * nchunks), each thread over a fixed stride, then wg_sum.
-__device__ __forceinline__ void obj_sum(const double* __restrict__ partial, unsigned nchunks, int t,
-                                        double* __restrict__ jt) {
-  const double* p = partial + int64_t(t) * nchunks;
+// jt = sum of the n shares of one state's outlet plane, each thread over a
+// fixed stride, then wg_sum: the same bits however the steps that wrote the
+// shares were launched.
+__device__ __forceinline__ void obj_sum(const double* __restrict__ p, unsigned n, double* __restrict__ jt) {
   double v = 0.0;
-  for (unsigned k = threadIdx.x; k < nchunks; k += kThreads) v += p[k];
+  for (unsigned k = threadIdx.x; k < n; k += kThreads) v += p[k];
   const double s = wg_sum(v);
-  if (threadIdx.x == 0) jt[t] = s;
+  if (threadIdx.x == 0) *jt = s;
 }
 
-__global__ __launch_bounds__(kThreads) void k_obj_sum(const double* __restrict__ partial, unsigned nchunks,
+// Workgroup b: state t + b.
+__global__ __launch_bounds__(kThreads) void k_obj_sum(const double* __restrict__ shares, unsigned plane, int t,
                                                       double* __restrict__ jt) {
-  obj_sum(partial, nchunks, int(blockIdx.x) + 1, jt);
+  obj_sum(shares + int64_t(blockIdx.x) * plane, plane, jt + t + blockIdx.x);
 }
 
-// partial: the step's chunk sums (OBJ)
-template <class R, bool OBJ, bool MOM>
+// The shares of a state that no further step reads.
+template <class R>
+__device__ __forceinline__ void obj_state(const AdjArgs<R>& a, const R* __restrict__ f, double* __restrict__ obj,
+                                          unsigned k) {
+  if (k >= unsigned(a.ny) * unsigned(a.nz)) return;
+  const int64_t id = a.outlet + int64_t(a.nx) * k;
+  R g[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i) g[i] = f[int64_t(i) * a.N + id];
+  obj[k] = a.solid[id] ? 0.0 : obj_cell(g);
+}
+template <class R>
+__global__ __launch_bounds__(kThreads) void k_obj_state(AdjArgs<R> a, const R* __restrict__ f,
+                                                        double* __restrict__ obj) {
+  obj_state(a, f, obj, blockIdx.x * kThreads + threadIdx.x);
+}
+
+template <class R, bool MOM>
 __global__ __launch_bounds__(kThreads) void k_fwd(AdjArgs<R> a, const R* __restrict__ src, R* __restrict__ dst,
-                                                  R* __restrict__ mom, double* __restrict__ partial) {
-  const unsigned wg = xcd_block(blockIdx.x, gridDim.x);
-  const double c = fwd_cell<R, OBJ, MOM>(a, src, dst, mom, int64_t(wg) * kThreads + threadIdx.x);
-  if constexpr (OBJ) obj_fold(c, partial, wg);
+                                                  R* __restrict__ mom, double* __restrict__ obj) {
+  fwd_cell<R, MOM>(a, src, dst, mom, obj, int64_t(xcd_block(blockIdx.x, gridDim.x)) * kThreads + threadIdx.x);
 }
 
 // ---- the moment record alone (the last state of a recomputed segment) ------------
@@ -521,62 +525,40 @@ __global__ __launch_bounds__(kThreads) void k_init(AdjArgs<R> a, const R* __rest
   for (int i = 0; i < Q; ++i) f[int64_t(i) * a.N + id] = sol ? R(0) : geq(i, rho - R(1), rho, u, usq);
 }
 
-// ---- adjoint seed: lambda^T = dJ/df^T -----------------------------------------
+// ---- adjoint seed: mu^{T-1} = P^T lambda^T, lambda^T = dJ/df^T ------------------
 template <class R>
-__device__ __forceinline__ void seed_cell(const AdjArgs<R>& a, R* __restrict__ lam, int64_t id) {
+__device__ __forceinline__ void seed_cell(const AdjArgs<R>& a, R* __restrict__ mu, int64_t id) {
   if (id >= a.N) return;
-  const bool on = !a.solid[id] && int(id % a.nx) == a.outlet;
+  const uint32_t lk = a.link[id];
+  const int x = int(id % a.nx);
 #pragma unroll
-  for (int i = 0; i < Q; ++i) lam[int64_t(i) * a.N + id] = on ? R(Lat<Q>::cx(i)) * a.invT : R(0);
+  for (int i = 0; i < Q; ++i) {
+    const bool wall = i != 0 && ((lk >> i) & 1u);
+    int xn = wall ? x : x + Lat<Q>::cx(i);
+    xn = xn < 0 ? xn + a.nx : (xn >= a.nx ? xn - a.nx : xn);
+    const R c = R(Lat<Q>::cx(i));
+    mu[int64_t(i) * a.N + id] = !(lk & 1u) && xn == a.outlet ? (wall ? -c : c) * a.invT : R(0);
+  }
 }
 
 template <class R>
-__global__ __launch_bounds__(kThreads) void k_seed(AdjArgs<R> a, R* __restrict__ lam) {
-  seed_cell(a, lam, int64_t(blockIdx.x) * kThreads + threadIdx.x);
+__global__ __launch_bounds__(kThreads) void k_seed(AdjArgs<R> a, R* __restrict__ mu) {
+  seed_cell(a, mu, int64_t(blockIdx.x) * kThreads + threadIdx.x);
 }
 
-// ---- one backward step: lambda^{t+1}, f^t -> lambda^t, grad += ds ----------------
+// ---- one backward step: mu^t, f^t -> mu^{t-1}, grad += ds -------------------------
 // The weighted moments of mu are summed per weight class over opposite pairs
 // (M from the pair sums, V from the differences, T from the sums), and
-// lambda^t is written pairwise: beside their own (1 - omega) mu terms,
+// lambda^t is formed pairwise: beside their own (1 - omega) mu terms,
 // lambda_i and lambda_opp(i) share A_rho - A_u.u / rho and differ in the sign
 // of c_i.A_u / (rho D).
-// f^t enters only through rho and u, read from its moment record mom ([4][N]:
-// rho - 1, u), 16 bytes per cell in FP32 instead of the 76 of the populations.
-template <class R>
-__device__ __forceinline__ void bwd_cell(const AdjArgs<R>& a, const R* __restrict__ mom,
-                                         const R* __restrict__ lam1, R* __restrict__ lam0,
-                                         R* __restrict__ grad, int with_obj, int64_t id) {
-  if (id >= a.N) return;
-  // mu = P^T lambda^{t+1}: every lane first reads lambda_i(x + c_i), issued
-  // together with the moments and the link word (every offset is in bounds); a
-  // wall link then takes lambda_opp(i)(x) instead
-  const Hops h = hops(a, uint32_t(id));
-  R m[4], mu[Q];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) m[k] = ld_pop(mom, a.N, k, h.o);
-  const R s = ld_cell(a.s, h.o);
-  uint32_t lk;
-  if (a.solids) {
-#pragma unroll
-    for (int i = 0; i < Q; ++i) mu[i] = ld_pop(lam1, a.N, i, hop(h, a, i));
-    lk = ((gptr<const uint32_t>)a.link)[id];
-    pin(m);
-    pin(mu);
-    asm volatile("" : "+v"(lk));  // tests of lk come after every load above
-    if (lk & 1u) return;
-  } else {
-    // wall links known from the place, not from memory: the bounce-back
-    // loads below go out in the same round as these
-    lk = face_links(a, h);
-#pragma unroll
-    for (int i = 0; i < Q; ++i) mu[i] = ld_pop(lam1, a.N, i, hop(h, a, i));
-  }
-  if (__ballot(lk != 0u) != 0) {
-#pragma unroll
-    for (int i = 1; i < Q; ++i)
-      if ((lk >> i) & 1u) mu[i] = ld_pop(lam1, a.N, opp(i), h.o);
-  }
+// f^t enters only through rho and u, its moment record m (rho - 1, u), 16
+// bytes per cell in FP32 instead of the 76 of the populations.
+// obj: lambda^t has the objective's own terms (a cell of the outlet plane,
+// t >= 1). Returns the cell's part of the gradient; sink(i, lambda_i).
+template <class R, class Sink>
+__device__ __forceinline__ R adjoint_collide(const R (&mu)[Q], const R (&m)[4], R s, const AdjArgs<R>& a, bool obj,
+                                             Sink&& sink) {
   const R rho = R(1) + m[0];
   const R u[3] = {m[1], m[2], m[3]};
   const R irD = inv_rho_d(rho, s, a);
@@ -633,33 +615,406 @@ __device__ __forceinline__ void bwd_cell(const AdjArgs<R>& a, const R* __restric
   const R Auu = Au[0] * u[0] + Au[1] * u[1] + Au[2] * u[2];
   // 1 / D = rho / (rho D) and 1 / rho = D / (rho D)
   const R D = R(1) + as * R(0.5);
-  const gptr<R> gr = cell_ref(grad, h.o);
-  *gr += -(R(0.5) * a.alpha * rho * irD) * Auu - fom * a.alpha * rho * Bu;
+  const R ds = -(R(0.5) * a.alpha * rho * irD) * Auu - fom * a.alpha * rho * Bu;
   const R base = Arho - Auu * (D * irD);
   // c_j.A_u / (rho D), with the objective's c_jx / T folded into the x part
   R Ar[3] = {Au[0] * irD, Au[1] * irD, Au[2] * irD};
-  if (with_obj && h.x == uint32_t(a.outlet)) Ar[0] += a.invT;
+  if (obj) Ar[0] += a.invT;
   const R om1 = a.om1;
-  // the cell's offset as a value of this block, so that the stores take it as
-  // their 32-bit lane offset (a value carried in from an earlier block reaches
-  // them widened to 64 bits, and each store then forms a 64-bit address)
-  uint32_t o = h.o;
-  asm volatile("" : "+v"(o));
-  st_pop(lam0, a.N, 0, o, om1 * mu[0] + base);
+  sink(0, om1 * mu[0] + base);
 #pragma unroll
   for (int p = 0; p < Q / 2; ++p) {
     const int i = 2 * p + 1;
     const R ca = cdot_folded<Q>(i, Ar);
-    st_pop(lam0, a.N, i, o, om1 * mu[i] + (base + ca));
-    st_pop(lam0, a.N, i + 1, o, om1 * mu[i + 1] + (base - ca));
+    sink(i, om1 * mu[i] + (base + ca));
+    sink(i + 1, om1 * mu[i + 1] + (base - ca));
   }
+  return ds;
+}
+
+template <class R>
+__device__ __forceinline__ void bwd_cell(const AdjArgs<R>& a, const R* __restrict__ mom,
+                                         const R* __restrict__ mu1, R* __restrict__ mu0,
+                                         R* __restrict__ grad, int with_obj, int64_t id) {
+  if (id >= a.N) return;
+  const Hops h = hops(a, uint32_t(id));
+  R m[4], mu[Q];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) m[k] = ld_pop(mom, a.N, k, h.o);
+#pragma unroll
+  for (int i = 0; i < Q; ++i) mu[i] = ld_pop(mu1, a.N, i, h.o);
+  const R s = ld_cell(a.s, h.o);
+  const gptr<R> gr = cell_ref(grad, h.o);
+  const R g0 = *gr;
+  uint32_t lk;
+  if (a.solids) {
+    lk = ((gptr<const uint32_t>)a.link)[id];
+    pin(m);
+    pin(mu);
+    asm volatile("" : "+v"(lk));  // tests of lk come after every load above
+    if (lk & 1u) return;
+  } else {
+    lk = face_links(a, h);
+  }
+  const bool obj = with_obj && h.x == uint32_t(a.outlet);
+  R ds;
+  if (__ballot(lk != 0u) == 0)
+    ds = adjoint_collide(mu, m, s, a, obj, [&](int i, R v) { push<R, false>(a, h, lk, mu0, i, opp(i), v); });
+  else
+    ds = adjoint_collide(mu, m, s, a, obj, [&](int i, R v) { push<R, true>(a, h, lk, mu0, i, opp(i), v); });
+  *gr = g0 + ds;
 }
 
 template <class R>
 __global__ __launch_bounds__(kThreads) void k_bwd(AdjArgs<R> a, const R* __restrict__ mom,
-                                                  const R* __restrict__ lam1, R* __restrict__ lam0,
+                                                  const R* __restrict__ mu1, R* __restrict__ mu0,
                                                   R* __restrict__ grad, int with_obj) {
-  bwd_cell(a, mom, lam1, lam0, grad, with_obj, int64_t(xcd_block(blockIdx.x, gridDim.x)) * kThreads + threadIdx.x);
+  bwd_cell(a, mom, mu1, mu0, grad, with_obj, int64_t(xcd_block(blockIdx.x, gridDim.x)) * kThreads + threadIdx.x);
+}
+
+// ---- two steps per pass over memory ------------------------------------------------
+// Forward: state t -> t + 2; backward: mu^t -> mu^{t-2}. As the lattice's
+// own two-step march: a workgroup owns an x-y tile and walks it along z. Every
+// thread of the tile and of a one-cell ring around it reads and collides its
+// cell of the next plane; the values that move in x or y go through a plane of
+// LDS; the tile's cells of the plane below, complete then, collide and push
+// their values to dst. The state between the two steps lives in LDS and
+// registers only. Same cells, links and arithmetic as the single steps, so the
+// same bits.
+//
+// What it saves is bytes: FP32 populations 152 -> 76 per cell and step, the
+// Brinkman field and the gradient once per pass. Per step, FP32 192x96x96:
+// forward 52.2 -> 36.0 us, with every state's record 57.2 -> 43.4, backward
+// 55.8 -> 49.5; 256x128x128: 123.5 -> 92.1, 135.1 -> 107.7, 142.9 -> 112.1;
+// 100^3: 25.6 -> 20.2, 28.0 -> 22.2, 32.4 -> 27.8; FP64 96^3 forward 52.2 ->
+// 35.1. What bounds it now is the walk of one workgroup per CU, as in the
+// lattices' march. Own cells are read and values pushed, so that a wavefront
+// inside the box forms no address per lane; where a row or wall needs them,
+// they are formed at the store (kept through the walk, they spill 40 registers).
+template <class R>
+struct MarchIo {
+  const R* src;
+  R* dst;
+  R *mom0, *mom1;        // records of the first and second step's state
+  R* grad;               // backward
+  double *obj0, *obj1;   // forward: shares of the first and second step's state, or null
+  int with0, with1;      // backward: objective terms of the first and second step
+};
+
+constexpr int kMarchPlanes = 16;  // directions that move in x or y
+__host__ __device__ constexpr int march_plane(int i) { return i >= 7 ? i - 3 : ((i >= 1 && i <= 4) ? i - 1 : -1); }
+
+template <class R>
+constexpr int kMarchSlack = kMarchMaxRow + 1;
+// Threads of a workgroup. The backward walk in FP32 holds more than the 128
+// registers that 1024 threads leave each: with 768 nothing spills (192x96x96:
+// 49.8 us per step against 54.8 with 1024, 58.8 with 896, 50.3 with 640). FP64
+// goes back in single steps: it spills at 512 threads too (96^3: 61 us per
+// step against 55, 192x80x60: 60 against 65).
+template <class R, bool BWD>
+constexpr int kMarchNt = BWD && sizeof(R) == 4 ? 768 : march_threads(sizeof(R));
+template <class R, bool BWD>
+constexpr int kMarchLds = 2 * kMarchPlanes * kMarchNt<R, BWD> + 2 * kMarchSlack<R>;
+
+// Descriptor of an array of `bytes` bytes, its words in scalar registers.
+template <class T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t array_rsrc(T* p, uint32_t bytes) {
+  const uint64_t u = reinterpret_cast<uint64_t>(p);
+  const uint64_t v = (uint64_t(__builtin_amdgcn_readfirstlane(uint32_t(u >> 32))) << 32) |
+                     uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(u)));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(v), 0, int(bytes), 0x00020000);
+}
+template <class R>
+__device__ __forceinline__ R bload(__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so) {
+  if constexpr (sizeof(R) == 8) {
+    const auto w = __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 0);
+    return __longlong_as_double(int64_t((uint64_t(w[1]) << 32) | uint64_t(w[0])));
+  } else {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, vo, so, 0));
+  }
+}
+// Moment records are stored past the caches: their next reader is a whole run
+// or segment away, and what they would push out is the state (192x96x96, every
+// state's record kept: 49.6 -> 43.4 us per step).
+constexpr int kNt = 2;
+template <class R, int AUX = 0>
+__device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so, R v) {
+  if constexpr (sizeof(R) == 8) {
+    typedef unsigned int u32x2 __attribute__((__vector_size__(8)));
+    const uint64_t b = uint64_t(__double_as_longlong(v));
+    const u32x2 w = {uint32_t(b), uint32_t(b >> 32)};
+    __builtin_amdgcn_raw_buffer_store_b64(w, r, vo, so, AUX);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, vo, so, AUX);
+  }
+}
+
+// BWD: backward; MOM (forward): the records of both states are written;
+// STORE (forward): the state is written (else only its records).
+// Offsets: a state holds less than 2 GiB (checked on the host).
+template <class R, bool BWD, bool MOM, bool STORE>
+__device__ __forceinline__ void march2(const AdjArgs<R>& a, const MarchArgs& m, const MarchIo<R>& io, unsigned wg,
+                                       R* lds) {
+  constexpr int NT = kMarchNt<R, BWD>;
+  constexpr uint32_t el = sizeof(R);
+  // direction that the value in slot i moves along; slots that move straight up, straight down
+  constexpr auto geo = [](int i) { return BWD ? opp(i) : i; };
+  constexpr int kUp = BWD ? 6 : 5, kDn = BWD ? 5 : 6;
+  const int tid = int(threadIdx.x);
+  const int pw = m.w + 2;
+  const int tx = int(wg % unsigned(m.ntx)), wy = int(wg / unsigned(m.ntx));
+  const int ty = wy % m.nty, zc = wy / m.nty;
+  // the tile's columns of every row first, then the ring's two columns
+  int lx, ly;
+  if (tid < m.w * (m.h + 2)) {
+    const int r = tid / m.w;
+    lx = tid - r * m.w;
+    ly = r - 1;
+  } else {
+    const int j = tid - m.w * (m.h + 2);
+    lx = (j & 1) ? m.w : -1;
+    ly = (j >> 1) - 1;
+  }
+  const int pos = min((ly + 1) * pw + lx + 1, NT - 1);
+  int x = tx * m.w + lx, y = ty * m.h + ly;
+  const bool core = lx >= 0 && lx < m.w && ly >= 0 && ly < m.h && x < a.nx && y < a.ny;
+  bool upd = ly <= m.h;
+  if (a.px) {
+    upd = upd && x <= a.nx;
+    x = x < 0 ? x + a.nx : (x >= a.nx ? x - a.nx : x);
+  }
+  if (a.py) {
+    upd = upd && y <= a.ny;
+    y = y < 0 ? y + a.ny : (y >= a.ny ? y - a.ny : y);
+  }
+  upd = upd && x >= 0 && x < a.nx && y >= 0 && y < a.ny;
+  const uint32_t vo = (uint32_t(x) + uint32_t(a.nx) * uint32_t(y)) * el;
+  // neighbours across a face of the box wrap (a wall link's is never used)
+  const bool edge = x == 0 || x == a.nx - 1 || y == 0 || y == a.ny - 1;
+  // wall links of a box without solid cells: those of the cell's place in x and y
+  uint32_t lkxy = 0;
+  if (!a.px) lkxy |= (x == a.nx - 1 ? face_mask(0, 1) : 0u) | (x == 0 ? face_mask(0, -1) : 0u);
+  if (!a.py) lkxy |= (y == a.ny - 1 ? face_mask(1, 1) : 0u) | (y == 0 ? face_mask(1, -1) : 0u);
+  const bool out = x == a.outlet;
+  const uint32_t oo = uint32_t(y) * 8u;  // shares: [nz][ny]
+
+  const int za = __builtin_amdgcn_readfirstlane(zc * m.zchunk);
+  const int zb = min(za + m.zchunk, a.nz);
+  auto wrap = [&](int z) { return z < 0 ? z + a.nz : (z >= a.nz ? z - a.nz : z); };
+  auto live = [&](int z) { return a.pz || (z >= 0 && z < a.nz); };
+
+  const uint32_t nb = a.sn;
+  const auto rsrc = array_rsrc(io.src, uint32_t(Q) * nb);
+  const auto rdst = array_rsrc(io.dst, uint32_t(Q) * nb);
+  const auto rs = array_rsrc(a.s, nb);
+  const auto rlk = array_rsrc(a.link, nb / el * 4u);
+  const auto rm0 = array_rsrc(io.mom0, 4u * nb);
+  const auto rm1 = array_rsrc(io.mom1, 4u * nb);
+  const auto rgr = array_rsrc(io.grad, nb);
+  const uint32_t op = uint32_t(a.ny) * uint32_t(a.nz) * 8u;
+  const auto ro0 = array_rsrc(io.obj0, io.obj0 ? op : 0u);
+  const auto ro1 = array_rsrc(io.obj1, io.obj1 ? op : 0u);
+
+  // what the collision of one cell takes
+  struct In {
+    R s;
+    R m[BWD ? 4 : 1];  // record of the first step's state
+    uint32_t lk;  // bit 0: the cell is updated, bit i: its link i is a wall
+  };
+  auto fetch = [&](int z, R (&g)[Q], In& in) {
+    in.lk = 0u;
+    if (!(live(z) && upd)) return;
+    const uint32_t zo = uint32_t(wrap(z)) * a.sz;
+    in.lk = 1u | lkxy;
+    if (a.solids) {
+      in.lk = __builtin_amdgcn_raw_buffer_load_b32(rlk, vo / el * 4u, zo / el * 4u, 0) ^ 1u;
+    } else if (!a.pz) {
+      in.lk |= (z == a.nz - 1 ? face_mask(2, 1) : 0u) | (z == 0 ? face_mask(2, -1) : 0u);
+    }
+#pragma unroll
+    for (int i = 0; i < Q; ++i) g[i] = bload<R>(rsrc, vo, uint32_t(i) * nb + zo);
+    in.s = bload<R>(rs, vo, zo);
+    if constexpr (BWD) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) in.m[k] = bload<R>(rm0, vo, uint32_t(k) * nb + zo);
+    }
+  };
+  // share of a forward state's cell on the outlet plane
+  auto share = [&](__amdgpu_buffer_rsrc_t r, int z, double c) {
+    typedef unsigned int u32x2 __attribute__((__vector_size__(8)));
+    const uint64_t b = uint64_t(__double_as_longlong(c));
+    const u32x2 w = {uint32_t(b), uint32_t(b >> 32)};
+    __builtin_amdgcn_raw_buffer_store_b64(w, r, oo, uint32_t(a.ny) * uint32_t(z) * 8u, 0);
+  };
+  // one collision; sink(i, v) takes the values
+  auto collide = [&](const R (&g)[Q], R s, const R (&mm)[BWD ? 4 : 1], bool obj, R* rec, auto&& sink) -> R {
+    if constexpr (BWD) {
+      return adjoint_collide(g, mm, s, a, obj && out, sink);
+    } else {
+      R drho, rho, u[3], F[3], irD, v[Q];
+      force_state(g, s, a, drho, rho, u, F, irD);
+      rec[0] = drho;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) rec[d + 1] = u[d];
+      post_collision(g, drho, rho, u, F, a, v, sink);
+      return R(0);
+    }
+  };
+
+  R g[Q];
+  In cur;
+  fetch(za - 1, g, cur);
+  uint32_t blk = 0u;  // links of the cell below, its other data, and its streamed-in values
+  R sB = R(0), mB[BWD ? 4 : 1], gB = R(0), dB = R(0);
+  R P[Q];             // of the upward and in-plane directions
+  R N[5];             // those moving up into the plane above: straight, then the four diagonals
+#pragma unroll
+  for (int i = 0; i < Q; ++i) P[i] = R(0);
+#pragma unroll
+  for (int k = 0; k < 5; ++k) N[k] = R(0);
+#pragma unroll
+  for (int k = 0; k < (BWD ? 4 : 1); ++k) mB[k] = R(0);
+  for (int z = za - 1; z <= zb; ++z) {
+    const int k = z - (za - 1);
+    R* const L = lds + kMarchSlack<R> + (k & 1) * (kMarchPlanes * NT) + pos;
+    const R* const Lb = lds + kMarchSlack<R> + ((k & 1) ^ 1) * (kMarchPlanes * NT) + pos;
+    const bool mine = core && z >= za && z < zb;
+    R h[Q];  // values after the first collision, unset in lanes that update no cell
+    const In in = cur;
+    R ds = R(0);
+    double c0 = 0.0;
+    if constexpr (!BWD) {
+      if (mine && out && io.obj0) c0 = in.lk & 1u ? obj_cell(g) : 0.0;
+    }
+    if (in.lk & 1u) {
+      R rec[4];
+      ds = collide(g, in.s, in.m, io.with0 != 0, rec, [&](int i, R v) { h[i] = v; });
+      if constexpr (!BWD && MOM) {
+        if (mine) {
+#pragma unroll
+          for (int d = 0; d < 4; ++d) bstore<R, kNt>(rm0, vo, uint32_t(d) * nb + uint32_t(z) * a.sz, rec[d]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 1; i < Q; ++i)
+      if (march_plane(i) >= 0) L[march_plane(i) * NT] = h[i];
+    const R h0 = h[0], hup = h[kUp], hdn = h[kDn];
+    {
+      R v[Q];  // unset in lanes that fetch nothing
+      In next;
+      next.lk = 0u;
+      if (z < zb) fetch(z + 1, v, next);
+#pragma unroll
+      for (int i = 0; i < Q; ++i) g[i] = v[i];
+      cur = next;
+    }
+    if constexpr (!BWD) {
+      if (mine && out && io.obj0) share(ro0, z, c0);
+    }
+    // LDS only: the loads above stay in flight across the barrier
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    auto from = [&](int i) {
+      const int e = geo(i);
+      return L[march_plane(i) * NT - Lat<Q>::cx(e) - Lat<Q>::cy(e) * pw];
+    };
+    if (z > za && core) {
+      if (blk & 1u) {
+        P[kDn] = hdn;
+#pragma unroll
+        for (int i = 1; i < Q; ++i)
+          if (march_plane(i) >= 0 && Lat<Q>::cz(geo(i)) < 0) P[i] = from(i);
+        if (blk > 1u) {
+#pragma unroll
+          for (int i = 1; i < Q; ++i) {
+            const int o = opp(i);  // the slot of the value that came back
+            if (Lat<Q>::cz(geo(i)) < 0 && ((blk >> geo(o)) & 1u)) P[i] = o == kUp ? N[0] : Lb[march_plane(o) * NT];
+          }
+        }
+      }
+      if constexpr (!BWD) {
+        if (out && io.obj1) share(ro1, z - 1, blk ? obj_cell(P) : 0.0);
+      }
+      if (blk & 1u) {
+        const uint32_t zo = uint32_t(z - 1) * a.sz;
+        const uint32_t zn[3] = {uint32_t(wrap(z - 2)) * a.sz, zo, uint32_t(wrap(z)) * a.sz};
+        R rec[4];
+        R d1;
+        if (!STORE) {
+          d1 = collide(P, sB, mB, io.with1 != 0, rec, [&](int, R) {});
+        } else if (__ballot(edge || blk > 1u) == 0) {
+          d1 = collide(P, sB, mB, io.with1 != 0, rec, [&](int i, R v) {
+            const int e = geo(i);
+            bstore<R>(rdst, vo, uint32_t(i) * nb + zn[1 + Lat<Q>::cz(e)] + uint32_t(Lat<Q>::cy(e)) * a.sy +
+                                    uint32_t(Lat<Q>::cx(e)) * el, v);
+          });
+        } else {
+          // offsets formed here, not kept through the walk
+          uint32_t o = vo, lk = blk;
+          asm volatile("" : "+v"(o), "+v"(lk));
+          const uint32_t dx[3] = {x == 0 ? a.sy - el : 0u - el, 0u, x == a.nx - 1 ? el - a.sy : el};
+          const uint32_t dy[3] = {y == 0 ? a.sz - a.sy : 0u - a.sy, 0u, y == a.ny - 1 ? a.sy - a.sz : a.sy};
+          d1 = collide(P, sB, mB, io.with1 != 0, rec, [&](int i, R v) {
+            const int e = geo(i);
+            const uint32_t to = o + dx[1 + Lat<Q>::cx(e)] + dy[1 + Lat<Q>::cy(e)] + (uint32_t(i) * nb + zn[1 + Lat<Q>::cz(e)]);
+            const uint32_t back = o + (uint32_t(opp(i)) * nb + zo);
+            bstore<R>(rdst, i != 0 && ((lk >> e) & 1u) ? back : to, 0u, v);
+          });
+        }
+        if constexpr (!BWD && MOM) {
+#pragma unroll
+          for (int d = 0; d < 4; ++d) bstore<R, kNt>(rm1, vo, uint32_t(d) * nb + zo, rec[d]);
+        }
+        if constexpr (BWD) bstore<R>(rgr, vo, zo, (gB + dB) + d1);
+      }
+    }
+    // streamed-in values of this plane, and those moving up into the next
+    blk = in.lk & 1u ? in.lk : 0u;
+    sB = in.s;
+    dB = ds;
+    P[0] = h0;
+#pragma unroll
+    for (int i = 1; i < Q; ++i)
+      if (Lat<Q>::cz(i) == 0) P[i] = from(i);
+    {
+      int n = 1;
+      P[kUp] = N[0];
+#pragma unroll
+      for (int i = 1; i < Q; ++i)
+        if (i != kUp && Lat<Q>::cz(geo(i)) > 0) P[i] = N[n++];
+    }
+    if (blk > 1u) {
+#pragma unroll
+      for (int i = 1; i < Q; ++i) {
+        const int o = opp(i);
+        if (Lat<Q>::cz(geo(i)) >= 0 && ((blk >> geo(o)) & 1u)) P[i] = o == kDn ? hdn : L[march_plane(o) * NT];
+      }
+    }
+    N[0] = hup;
+    {
+      int n = 1;
+#pragma unroll
+      for (int i = 1; i < Q; ++i)
+        if (i != kUp && Lat<Q>::cz(geo(i)) > 0) N[n++] = from(i);
+    }
+    if constexpr (BWD) {
+      // what the second step of this plane takes, with a whole plane to arrive
+      if (mine && blk) {
+        const uint32_t zo = uint32_t(z) * a.sz;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) mB[d] = bload<R>(rm1, vo, uint32_t(d) * nb + zo);
+        gB = bload<R>(rgr, vo, zo);
+      }
+    }
+  }
+}
+
+template <class R, bool BWD, bool MOM, bool STORE>
+__global__ __launch_bounds__((kMarchNt<R, BWD>)) void k_march2(AdjArgs<R> a, MarchArgs m, MarchIo<R> io) {
+  __shared__ R lds[kMarchLds<R, BWD>];
+  march2<R, BWD, MOM, STORE>(a, m, io, xcd_block(blockIdx.x, gridDim.x), lds);
 }
 
 // ---- many boxes in one launch ------------------------------------------------------
@@ -673,7 +1028,7 @@ struct Entry {
   R* const* slots;
   R* grad;
   double* jt;
-  double* partial;  // objective partial sums, [T + 1][chunks of 256 cells]
+  double* shares;   // objective shares of kObjStates states, [ny * nz] each
   int64_t cell0;    // first cell in the batch numbering (a multiple of 256)
 };
 
@@ -696,37 +1051,41 @@ __device__ __forceinline__ const Entry<R>& entry_of(const Entry<R>* tab, int n, 
 
 // One workgroup covers 256 cells of one box (boxes start on multiples of
 // 256 in the batch numbering).
-// mom: the slot of the moment record (MOM)
-template <class R, bool OBJ, bool MOM>
+// mom: the slot of the moment record (MOM); obj: which of the states kept the
+// shares go to (-1: not wanted)
+template <class R, bool MOM>
 __global__ __launch_bounds__(kThreads) void k_fwd_b(const Entry<R>* __restrict__ tab, int n, int64_t total,
-                                                    int src, int dst, int mom, int t) {
+                                                    int src, int dst, int mom, int obj) {
   const unsigned g = xcd_block(blockIdx.x, gridDim.x);
   const int64_t k0 = int64_t(g) * kThreads;
   if (k0 >= total) return;
   const Entry<R>& E = entry_of(tab, n, g);
-  const int64_t id0 = k0 - E.cell0;
-  const double c =
-      fwd_cell<R, OBJ, MOM>(E.a, slot(E, src), slot(E, dst), MOM ? slot(E, mom) : nullptr, id0 + threadIdx.x);
-  if constexpr (OBJ) {
-    const unsigned nchunks = unsigned((E.a.N + kThreads - 1) / kThreads);
-    obj_fold(c, E.partial + int64_t(t) * nchunks, unsigned(id0 / kThreads));
-  }
+  double* const o = obj < 0 ? nullptr : E.shares + int64_t(obj) * E.a.ny * E.a.nz;
+  fwd_cell<R, MOM>(E.a, slot(E, src), slot(E, dst), MOM ? slot(E, mom) : nullptr, o, k0 - E.cell0 + threadIdx.x);
 }
 
-// grid (T, boxes)
+// grid (states, boxes): states t, t + 1, ...
 template <class R>
-__global__ __launch_bounds__(kThreads) void k_obj_sum_b(const Entry<R>* __restrict__ tab) {
+__global__ __launch_bounds__(kThreads) void k_obj_sum_b(const Entry<R>* __restrict__ tab, int t) {
   const Entry<R>& E = tab[blockIdx.y];
-  obj_sum(E.partial, unsigned((E.a.N + kThreads - 1) / kThreads), int(blockIdx.x) + 1, E.jt);
+  const unsigned plane = unsigned(E.a.ny) * unsigned(E.a.nz);
+  obj_sum(E.shares + int64_t(blockIdx.x) * plane, plane, E.jt + t + blockIdx.x);
+}
+
+// grid (workgroups of the largest plane, boxes)
+template <class R>
+__global__ __launch_bounds__(kThreads) void k_obj_state_b(const Entry<R>* __restrict__ tab, int src, int obj) {
+  const Entry<R>& E = tab[blockIdx.y];
+  obj_state(E.a, E.slots[src], E.shares + int64_t(obj) * E.a.ny * E.a.nz, blockIdx.x * kThreads + threadIdx.x);
 }
 
 template <class R>
 __global__ __launch_bounds__(kThreads) void k_seed_b(const Entry<R>* __restrict__ tab, int n, int64_t total,
-                                                     int lam) {
+                                                     int mu) {
   const int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   if (k >= total) return;
   const Entry<R>& E = entry_of(tab, n, blockIdx.x);
-  seed_cell(E.a, E.slots[lam], k - E.cell0);
+  seed_cell(E.a, E.slots[mu], k - E.cell0);
 }
 
 template <class R>
@@ -748,6 +1107,35 @@ __global__ __launch_bounds__(kThreads) void k_bwd_b(const Entry<R>* __restrict__
   bwd_cell(E.a, slot(E, mom), slot(E, lam1), slot(E, lam0), E.grad, with_obj, k0 - E.cell0 + threadIdx.x);
 }
 
+// Two steps of every box: mt and wgs as for the lattices' batches (tiles of
+// every box, box and workgroup of every workgroup, longest first); the slots
+// of the states and records, the places of the shares (-1: none).
+struct Pass {
+  int src, dst, mom0, mom1, obj0, obj1, with0, with1;
+};
+template <class R, bool BWD, bool MOM, bool STORE>
+__global__ __launch_bounds__((kMarchNt<R, BWD>)) void k_march2_b(const Entry<R>* __restrict__ tab,
+                                                                 const MarchArgs* __restrict__ mt,
+                                                                 const MarchWg* __restrict__ wgs, Pass p) {
+  __shared__ R lds[kMarchLds<R, BWD>];
+  wgs = in_const(wgs);
+  const int e = __builtin_amdgcn_readfirstlane(wgs[blockIdx.x].block);
+  const unsigned wg = unsigned(__builtin_amdgcn_readfirstlane(wgs[blockIdx.x].wg));
+  const Entry<R>& E = in_const(tab)[e];
+  const int64_t plane = int64_t(E.a.ny) * E.a.nz;
+  MarchIo<R> io;
+  io.src = slot(E, p.src);
+  io.dst = STORE ? slot(E, p.dst) : nullptr;
+  io.mom0 = BWD || MOM ? slot(E, p.mom0) : nullptr;
+  io.mom1 = BWD || MOM ? slot(E, p.mom1) : nullptr;
+  io.grad = E.grad;
+  io.obj0 = p.obj0 < 0 ? nullptr : E.shares + p.obj0 * plane;
+  io.obj1 = p.obj1 < 0 ? nullptr : E.shares + p.obj1 * plane;
+  io.with0 = p.with0;
+  io.with1 = p.with1;
+  march2<R, BWD, MOM, STORE>(E.a, in_const(mt)[e], io, wg, lds);
+}
+
 }  // namespace adj
 }  // namespace flb
 
@@ -767,12 +1155,11 @@ struct flb_adjoint_s {
   void* d_s = nullptr;
   void* d_f0 = nullptr;
   void* d_work[2] = {nullptr, nullptr};
-  void* d_lam[2] = {nullptr, nullptr};
+  void* d_lam[2] = {nullptr, nullptr};  // mu, ping-pong
   void* d_grad = nullptr;
   double* d_jt = nullptr;
   int jt_cap = 0;
-  double* d_partial = nullptr;  // objective partial sums, [T + 1][chunks of 256 cells]
-  int partial_cap = 0;          // in steps
+  double* d_shares = nullptr;  // objective shares of kObjStates states, [ny * nz] each
   std::vector<void*> ckpt;  // ckpt[k] = state at step k*K (ckpt[0] aliases d_f0)
   // moment records (rho - 1, u; [4][N]) of the states the adjoint steps read:
   // those of one recomputed segment (K > 0), or of every state (K == 0)
@@ -791,6 +1178,9 @@ struct flb_adjoint_s {
 namespace {
 
 size_t state_bytes(const flb_adjoint_s* h) { return size_t(A::Q) * size_t(h->N) * h->real; }
+// States whose objective shares are kept before they are summed.
+constexpr int kObjStates = 32;
+
 size_t mom_bytes(const flb_adjoint_s* h) { return size_t(4) * size_t(h->N) * h->real; }
 
 // Multiplier, shift and pass mask of A::div_magic for 1 <= d < 2^31.
@@ -848,13 +1238,22 @@ hipError_t build_links(const flb_adjoint_s* h) {
   return hipGetLastError();
 }
 
-// One forward step src -> dst; OBJ: the chunk sums of its objective (step t);
-// MOM: the moment record of src into mom.
-template <class R, bool OBJ, bool MOM>
-hipError_t fwd_step(const flb_adjoint_s* h, const void* src, void* dst, void* mom, int t) {
-  hipLaunchKernelGGL((A::k_fwd<R, OBJ, MOM>), dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
-                     static_cast<const R*>(src), static_cast<R*>(dst), static_cast<R*>(mom),
-                     h->d_partial + int64_t(t) * grid_of(h));
+unsigned obj_plane(const flb_adjoint_s* h) { return unsigned(h->desc.ny) * unsigned(h->desc.nz); }
+
+// One forward step src -> dst; obj: where the objective shares of src go, or
+// null; MOM: the moment record of src into mom.
+template <class R, bool MOM>
+hipError_t fwd_step(const flb_adjoint_s* h, const void* src, void* dst, void* mom, double* obj) {
+  hipLaunchKernelGGL((A::k_fwd<R, MOM>), dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
+                     static_cast<const R*>(src), static_cast<R*>(dst), static_cast<R*>(mom), obj);
+  return hipGetLastError();
+}
+
+// Sums the shares of n states from state t on (those of t in slot 0).
+hipError_t obj_flush(const flb_adjoint_s* h, int t, int n) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(A::k_obj_sum, dim3(unsigned(n)), dim3(A::kThreads), 0, h->stream, h->d_shares, obj_plane(h), t,
+                     h->d_jt);
   return hipGetLastError();
 }
 
@@ -930,15 +1329,9 @@ int prepare_forward(flb_adjoint_s* h, int T, int K) {
       return fail(FLB_ERR_NOMEM, "objective buffer allocation failed");
     h->jt_cap = T + 1;
   }
-  if (h->partial_cap < T + 1) {
-    if (h->d_partial) (void)hipFree(h->d_partial);
-    h->d_partial = nullptr;
-    h->partial_cap = 0;
-    if (hipMalloc(reinterpret_cast<void**>(&h->d_partial), size_t(T + 1) * grid_of(h) * sizeof(double)) !=
-        hipSuccess)
-      return fail(FLB_ERR_NOMEM, "objective partial-sum buffer allocation failed");
-    h->partial_cap = T + 1;
-  }
+  if (!h->d_shares && hipMalloc(reinterpret_cast<void**>(&h->d_shares),
+                                size_t(kObjStates) * obj_plane(h) * sizeof(double)) != hipSuccess)
+    return fail(FLB_ERR_NOMEM, "objective share buffer allocation failed");
   return FLB_OK;
 }
 
@@ -952,11 +1345,53 @@ void finish_forward(flb_adjoint_s* h, const double* jt, void* last) {
   h->recorded = h->K >= 0;
 }
 
-// Buffer receiving state t+1 of a forward run whose state t sits in src.
+// Buffer receiving state t of a forward run from a state in src.
 void* forward_target(const flb_adjoint_s* h, int t, const void* src) {
   const int K = h->K, T = h->T;
-  if (K > 0 && (t + 1) % K == 0 && t + 1 < T) return h->ckpt[size_t((t + 1) / K)];
+  if (K > 0 && t % K == 0 && t < T) return h->ckpt[size_t(t / K)];
   return (src == h->d_work[0]) ? h->d_work[1] : h->d_work[0];
+}
+
+// Steps taken at once from state t: two where passes of two steps serve
+// (march) unless state t + 1 is a checkpoint or the last.
+int forward_span(int T, int K, int t, bool march) {
+  return march && t + 2 <= T && !(K > 0 && (t + 1) % K == 0) ? 2 : 1;
+}
+
+int march_nt(size_t real, bool bwd) {
+  return real == 8 ? A::kMarchNt<double, false> : (bwd ? A::kMarchNt<float, true> : A::kMarchNt<float, false>);
+}
+
+// Whether one box takes two steps per pass, and its tiles. Boxes of 32 MiB of
+// populations and more, as the lattices' march; the passes address a state
+// with 31-bit byte offsets.
+bool march_of(const flb_adjoint_s* h, bool bwd, flb::MarchArgs* m) {
+  if (state_bytes(h) < kMarchMinBytes || state_bytes(h) >= (size_t(1) << 31)) return false;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) return false;
+  *m = march_plan({h->desc.nx, h->desc.ny, h->desc.nz, h->desc.nx}, int(h->real), cus, march_nt(h->real, bwd));
+  return true;
+}
+
+template <class R, bool BWD, bool MOM, bool STORE>
+hipError_t march_step(const flb_adjoint_s* h, const flb::MarchArgs& m, const A::MarchIo<R>& io) {
+  const dim3 grid(unsigned(m.ntx) * unsigned(m.nty) * unsigned(m.nz)), block(unsigned(A::kMarchNt<R, BWD>));
+  hipLaunchKernelGGL((A::k_march2<R, BWD, MOM, STORE>), grid, block, 0, h->stream, adj_args<R>(h), m, io);
+  return hipGetLastError();
+}
+
+// States t and t + 1 from src to dst (state t + 2; null: only the records).
+template <class R, bool MOM, bool STORE>
+hipError_t fwd_two(const flb_adjoint_s* h, const flb::MarchArgs& m, const void* src, void* dst, void* mom0,
+                   void* mom1, double* obj0, double* obj1) {
+  A::MarchIo<R> io{};
+  io.src = static_cast<const R*>(src);
+  io.dst = static_cast<R*>(dst);
+  io.mom0 = static_cast<R*>(mom0);
+  io.mom1 = static_cast<R*>(mom1);
+  io.obj0 = obj0;
+  io.obj1 = obj1;
+  return march_step<R, false, MOM, STORE>(h, m, io);
 }
 
 template <class R>
@@ -964,19 +1399,42 @@ int forward_impl(flb_adjoint_s* h, int T, int K, double* J) {
   int rc = prepare_forward(h, T, K);
   if (rc) return rc;
   HIP_TRY(hipEventRecord(h->e0, h->stream));
+  flb::MarchArgs m{};
+  const bool march = march_of(h, false, &m);
   const void* src = h->d_f0;
-  for (int t = 0; t < T; ++t) {
-    void* dst = forward_target(h, t, src);
-    if (K == 0)
-      HIP_TRY((fwd_step<R, true, true>(h, src, dst, h->mtape[size_t(t)], t + 1)));
-    else
-      HIP_TRY((fwd_step<R, true, false>(h, src, dst, nullptr, t + 1)));
+  int base = 1;  // state of the first shares kept
+  for (int t = 0, n = 0; t < T; t += n) {
+    n = forward_span(T, K, t, march);
+    if (t + n - base > kObjStates) {
+      HIP_TRY(obj_flush(h, base, t - base));
+      base = t;
+    }
+    double* const obj1 = h->d_shares + int64_t(t + 1 - base) * obj_plane(h);  // of state t + 1
+    double* const obj0 = t > 0 ? obj1 - obj_plane(h) : nullptr;
+    void* dst = forward_target(h, t + n, src);
+    if (n == 2) {
+      if (K == 0)
+        HIP_TRY((fwd_two<R, true, true>(h, m, src, dst, h->mtape[size_t(t)], h->mtape[size_t(t + 1)], obj0, obj1)));
+      else
+        HIP_TRY((fwd_two<R, false, true>(h, m, src, dst, nullptr, nullptr, obj0, obj1)));
+    } else if (K == 0) {
+      HIP_TRY((fwd_step<R, true>(h, src, dst, h->mtape[size_t(t)], obj0)));
+    } else {
+      HIP_TRY((fwd_step<R, false>(h, src, dst, nullptr, obj0)));
+    }
     src = dst;
   }
   if (T > 0) {
-    hipLaunchKernelGGL(A::k_obj_sum, dim3(unsigned(T)), dim3(A::kThreads), 0, h->stream, h->d_partial, grid_of(h),
-                       h->d_jt);
+    if (T + 1 - base > kObjStates) {
+      HIP_TRY(obj_flush(h, base, T - base));
+      base = T;
+    }
+    const unsigned plane = obj_plane(h);
+    hipLaunchKernelGGL(A::k_obj_state<R>, dim3((plane + A::kThreads - 1) / A::kThreads), dim3(A::kThreads), 0,
+                       h->stream, adj_args<R>(h), static_cast<const R*>(src),
+                       h->d_shares + int64_t(T - base) * plane);
     HIP_TRY(hipGetLastError());
+    HIP_TRY(obj_flush(h, base, T + 1 - base));
   }
   HIP_TRY(hipEventRecord(h->e1, h->stream));
   std::vector<double> jt(size_t(T + 1), 0.0);
@@ -992,11 +1450,38 @@ int forward_impl(flb_adjoint_s* h, int T, int K, double* J) {
 
 // One adjoint step; mom: the moment record of state t.
 template <class R>
-hipError_t bwd_step(const flb_adjoint_s* h, const void* mom, const void* lam1, void* lam0, int with_obj) {
+hipError_t bwd_step(const flb_adjoint_s* h, const void* mom, const void* mu1, void* mu0, int with_obj) {
   hipLaunchKernelGGL(A::k_bwd<R>, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
-                     static_cast<const R*>(mom), static_cast<const R*>(lam1), static_cast<R*>(lam0),
+                     static_cast<const R*>(mom), static_cast<const R*>(mu1), static_cast<R*>(mu0),
                      static_cast<R*>(h->d_grad), with_obj);
   return hipGetLastError();
+}
+
+// The adjoint steps of states t1 - 1 down to t0, whose records are mom[0 ..];
+// mu in h->d_lam[cur].
+template <class R>
+hipError_t bwd_run(const flb_adjoint_s* h, const flb::MarchArgs* m, void* const* mom, int t0, int t1, int& cur) {
+  hipError_t e = hipSuccess;
+  for (int t = t1 - 1; e == hipSuccess && t >= t0; cur ^= 1) {
+    bool two = false;
+    if constexpr (sizeof(R) == 4) two = m && t - 1 >= t0;
+    if (two) {
+      A::MarchIo<R> io{};
+      io.src = static_cast<const R*>(h->d_lam[cur]);
+      io.dst = static_cast<R*>(h->d_lam[cur ^ 1]);
+      io.mom0 = static_cast<R*>(mom[t - t0]);
+      io.mom1 = static_cast<R*>(mom[t - 1 - t0]);
+      io.grad = static_cast<R*>(h->d_grad);
+      io.with0 = t >= 1;
+      io.with1 = t - 1 >= 1;
+      if constexpr (sizeof(R) == 4) e = march_step<R, true, false, true>(h, *m, io);
+      t -= 2;
+    } else {
+      e = bwd_step<R>(h, mom[t - t0], h->d_lam[cur], h->d_lam[cur ^ 1], t >= 1);
+      t -= 1;
+    }
+  }
+  return e;
 }
 
 int prepare_backward(flb_adjoint_s* h) {
@@ -1020,29 +1505,42 @@ int backward_impl(flb_adjoint_s* h, double* grad) {
   hipLaunchKernelGGL(A::k_seed<R>, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
                      static_cast<R*>(h->d_lam[0]));
   HIP_TRY(hipGetLastError());
+  flb::MarchArgs ftiles{}, btiles{};
+  const bool march = march_of(h, false, &ftiles) && march_of(h, true, &btiles);
+  const flb::MarchArgs* const fm = march ? &ftiles : nullptr;
+  const flb::MarchArgs* const m = march && sizeof(R) == 4 ? &btiles : nullptr;
   int cur = 0;
   if (K == 0) {
-    for (int t = T - 1; t >= 0; --t) {
-      HIP_TRY(bwd_step<R>(h, h->mtape[size_t(t)], h->d_lam[cur], h->d_lam[cur ^ 1], t >= 1));
-      cur ^= 1;
-    }
+    HIP_TRY(bwd_run<R>(h, m, h->mtape.data(), 0, T, cur));
   } else {
     const int nseg = (T + K - 1) / K;
     for (int k = nseg - 1; k >= 0; --k) {
       const int t0 = k * K, t1 = std::min((k + 1) * K, T);
       // moment records of states t0 .. t1-1: the recompute steps from the
-      // checkpoint write those of their sources, k_mom that of the last state
+      // checkpoint write those of their sources (and, two at a time, of the
+      // states between), the last pass or k_mom that of the last state
       const void* src = h->ckpt[size_t(k)];
-      for (int t = t0; t < t1 - 1; ++t) {
-        void* dst = h->d_rec[(t - t0) & 1];
-        HIP_TRY((fwd_step<R, false, true>(h, src, dst, h->mtape[size_t(t - t0)], 0)));
+      int t = t0, r = 0;
+      while (t < t1) {
+        void* const mom = h->mtape[size_t(t - t0)];
+        void* const dst = h->d_rec[r];
+        if (fm && t + 2 < t1) {
+          HIP_TRY((fwd_two<R, true, true>(h, *fm, src, dst, mom, h->mtape[size_t(t + 1 - t0)], nullptr, nullptr)));
+          t += 2;
+        } else if (fm && t + 2 == t1) {
+          HIP_TRY((fwd_two<R, true, false>(h, *fm, src, nullptr, mom, h->mtape[size_t(t + 1 - t0)], nullptr, nullptr)));
+          t += 2;
+        } else if (t + 1 < t1) {
+          HIP_TRY((fwd_step<R, true>(h, src, dst, mom, nullptr)));
+          t += 1;
+        } else {
+          HIP_TRY(mom_step<R>(h, src, mom));
+          t += 1;
+        }
         src = dst;
+        r ^= 1;
       }
-      HIP_TRY(mom_step<R>(h, src, h->mtape[size_t(t1 - 1 - t0)]));
-      for (int t = t1 - 1; t >= t0; --t) {
-        HIP_TRY(bwd_step<R>(h, h->mtape[size_t(t - t0)], h->d_lam[cur], h->d_lam[cur ^ 1], t >= 1));
-        cur ^= 1;
-      }
+      HIP_TRY(bwd_run<R>(h, m, h->mtape.data(), t0, t1, cur));
     }
   }
   HIP_TRY(hipEventRecord(h->e1, h->stream));
@@ -1076,6 +1574,12 @@ struct flb_adjoint_batch_s {
   void* d_slots = nullptr;
   size_t slots_cap = 0;
   int nslots = 0;
+  // two steps per pass: forward [0] and backward [1] tiles of the boxes and
+  // workgroups of the launch (march: -1 not looked at yet, 0 not taken)
+  int march = -1;
+  flb::MarchArgs* d_mt[2] = {nullptr, nullptr};
+  flb::MarchWg* d_mwg[2] = {nullptr, nullptr};
+  unsigned nmwg[2] = {0, 0};
   int T = 0, K = -1;
   bool recorded = false;
   float fwd_ms = 0.0f, bwd_ms = 0.0f;
@@ -1088,10 +1592,10 @@ enum { kSlotF0 = 0, kSlotW0 = 1, kSlotW1 = 2, kSlotL0 = 3, kSlotL1 = 4, kSlotR0 
 
 int tape_base(int T, int K) { return kSlotCk + (K > 0 ? (T + K - 1) / K : 0); }
 
-// the slot receiving state t+1 when state t sits in slot src (forward_target
-// in slot numbers)
+// the slot receiving state t from a state in slot src (forward_target in slot
+// numbers)
 int forward_slot(int T, int K, int t, int src) {
-  if (K > 0 && (t + 1) % K == 0 && t + 1 < T) return kSlotCk + (t + 1) / K;
+  if (K > 0 && t % K == 0 && t < T) return kSlotCk + t / K;
   return src == kSlotW0 ? kSlotW1 : kSlotW0;
 }
 
@@ -1145,7 +1649,7 @@ int upload_table(flb_adjoint_batch_s* b) {
     tab[m].slots = dslots + m * size_t(nslots);
     tab[m].grad = static_cast<R*>(h->d_grad);
     tab[m].jt = h->d_jt;
-    tab[m].partial = h->d_partial;
+    tab[m].shares = h->d_shares;
     tab[m].cell0 = b->cell0[m];
   }
   HIP_TRY(hipMemcpyAsync(b->d_slots, slots.data(), bytes_slots, hipMemcpyHostToDevice, b->stream));
@@ -1163,12 +1667,70 @@ int upload_table(flb_adjoint_batch_s* b) {
   return FLB_OK;
 }
 
-// One forward step of every box, slot src -> dst; OBJ: the objectives into jt[t];
-// MOM: the moment records of src into slot mom.
-template <class R, bool OBJ, bool MOM>
-hipError_t fwd_batch(const flb_adjoint_batch_s* b, int src, int dst, int mom, int t) {
-  hipLaunchKernelGGL((A::k_fwd_b<R, OBJ, MOM>), dim3(batch_grid(b)), dim3(A::kThreads), 0, b->stream,
-                     static_cast<const A::Entry<R>*>(b->d_tab), int(b->members.size()), b->total, src, dst, mom, t);
+// One forward step of every box, slot src -> dst; obj: the shares of src go to
+// (-1: not wanted); MOM: the moment records of src into slot mom.
+template <class R, bool MOM>
+hipError_t fwd_batch(const flb_adjoint_batch_s* b, int src, int dst, int mom, int obj) {
+  hipLaunchKernelGGL((A::k_fwd_b<R, MOM>), dim3(batch_grid(b)), dim3(A::kThreads), 0, b->stream,
+                     static_cast<const A::Entry<R>*>(b->d_tab), int(b->members.size()), b->total, src, dst, mom, obj);
+  return hipGetLastError();
+}
+
+template <class R>
+hipError_t obj_flush_batch(const flb_adjoint_batch_s* b, int t, int n) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(A::k_obj_sum_b<R>, dim3(unsigned(n), unsigned(b->members.size())), dim3(A::kThreads), 0,
+                     b->stream, static_cast<const A::Entry<R>*>(b->d_tab), t);
+  return hipGetLastError();
+}
+
+template <class R>
+hipError_t obj_state_batch(const flb_adjoint_batch_s* b, int src, int obj) {
+  unsigned plane = 1;
+  for (const flb_adjoint_s* h : b->members) plane = std::max(plane, obj_plane(h));
+  hipLaunchKernelGGL(A::k_obj_state_b<R>,
+                     dim3((plane + A::kThreads - 1) / A::kThreads, unsigned(b->members.size())), dim3(A::kThreads), 0,
+                     b->stream, static_cast<const A::Entry<R>*>(b->d_tab), src, obj);
+  return hipGetLastError();
+}
+
+// Whether the batch takes two steps per pass: looked at once (its boxes do not
+// change). As for the lattices' batches, 32 MiB of populations and more, where
+// a pass is estimated to be faster than two single launches.
+int prepare_march(flb_adjoint_batch_s* b) {
+  if (b->march >= 0) return FLB_OK;
+  b->march = 0;
+  size_t live = 0;
+  std::vector<MarchBox> boxes;
+  for (const flb_adjoint_s* h : b->members) {
+    if (state_bytes(h) >= (size_t(1) << 31)) return FLB_OK;
+    live += state_bytes(h);
+    boxes.push_back({h->desc.nx, h->desc.ny, h->desc.nz, h->desc.nx});
+  }
+  if (live < kMarchMinBytes) return FLB_OK;
+  int cus = 0;
+  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
+  for (int k = 0; k < 2; ++k) {
+    std::vector<flb::MarchArgs> mt;
+    std::vector<flb::MarchWg> wg;
+    const double span = march_plan_batch(boxes, int(b->real), cus, march_nt(b->real, k == 1), mt, wg);
+    if (k == 0 && span * 0.9e-6 > 4.0 * double(live) / 4.8e12) return FLB_OK;
+    if (hipMalloc(reinterpret_cast<void**>(&b->d_mt[k]), mt.size() * sizeof(mt[0])) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void**>(&b->d_mwg[k]), wg.size() * sizeof(wg[0])) != hipSuccess)
+      return fail(FLB_ERR_NOMEM, "batch tile table allocation failed");
+    HIP_TRY(hipMemcpyAsync(b->d_mt[k], mt.data(), mt.size() * sizeof(mt[0]), hipMemcpyHostToDevice, b->stream));
+    HIP_TRY(hipMemcpyAsync(b->d_mwg[k], wg.data(), wg.size() * sizeof(wg[0]), hipMemcpyHostToDevice, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    b->nmwg[k] = unsigned(wg.size());
+  }
+  b->march = 1;
+  return FLB_OK;
+}
+
+template <class R, bool BWD, bool MOM, bool STORE>
+hipError_t march_batch(const flb_adjoint_batch_s* b, const A::Pass& p) {
+  hipLaunchKernelGGL((A::k_march2_b<R, BWD, MOM, STORE>), dim3(b->nmwg[BWD]), dim3(unsigned(A::kMarchNt<R, BWD>)), 0,
+                     b->stream, static_cast<const A::Entry<R>*>(b->d_tab), b->d_mt[BWD], b->d_mwg[BWD], p);
   return hipGetLastError();
 }
 
@@ -1187,6 +1749,25 @@ hipError_t bwd_batch(const flb_adjoint_batch_s* b, int mom, int lam1, int lam0, 
   return hipGetLastError();
 }
 
+// As bwd_run: the records of states t0 .. t1 - 1 in slots mom0 ...
+template <class R>
+hipError_t bwd_run_batch(const flb_adjoint_batch_s* b, int mom0, int t0, int t1, int& cur) {
+  hipError_t e = hipSuccess;
+  for (int t = t1 - 1; e == hipSuccess && t >= t0; cur ^= 1) {
+    const int mom = mom0 + t - t0;
+    bool two = false;
+    if constexpr (sizeof(R) == 4) {
+      two = b->march == 1 && t - 1 >= t0;
+      if (two)
+        e = march_batch<R, true, false, true>(
+            b, {kSlotL0 + cur, kSlotL0 + (cur ^ 1), mom, mom - 1, -1, -1, t >= 1, t - 1 >= 1});
+    }
+    if (!two) e = bwd_batch<R>(b, mom, kSlotL0 + cur, kSlotL0 + (cur ^ 1), t >= 1);
+    t -= two ? 2 : 1;
+  }
+  return e;
+}
+
 template <class R>
 int batch_forward_impl(flb_adjoint_batch_s* b, int T, int K, double* J) {
   b->recorded = false;
@@ -1198,23 +1779,37 @@ int batch_forward_impl(flb_adjoint_batch_s* b, int T, int K, double* J) {
   }
   b->T = T;
   b->K = K;
-  if ((rc = upload_table<R>(b))) return rc;
+  if ((rc = prepare_march(b)) || (rc = upload_table<R>(b))) return rc;
   const unsigned nm = unsigned(b->members.size());
   HIP_TRY(hipEventRecord(b->e0, b->stream));
   int src = kSlotF0;
   const int tb = tape_base(T, K);
-  for (int t = 0; t < T; ++t) {
-    const int dst = forward_slot(T, K, t, src);
-    if (K == 0)
-      HIP_TRY((fwd_batch<R, true, true>(b, src, dst, tb + t, t + 1)));
+  int base = 1;  // state of the first shares kept
+  for (int t = 0, n = 0; t < T; t += n) {
+    n = forward_span(T, K, t, b->march == 1);
+    if (t + n - base > kObjStates) {
+      HIP_TRY(obj_flush_batch<R>(b, base, t - base));
+      base = t;
+    }
+    const int obj = t > 0 ? t - base : -1;
+    const int dst = forward_slot(T, K, t + n, src);
+    if (n == 2 && K == 0)
+      HIP_TRY((march_batch<R, false, true, true>(b, {src, dst, tb + t, tb + t + 1, obj, t + 1 - base, 0, 0})));
+    else if (n == 2)
+      HIP_TRY((march_batch<R, false, false, true>(b, {src, dst, 0, 0, obj, t + 1 - base, 0, 0})));
+    else if (K == 0)
+      HIP_TRY((fwd_batch<R, true>(b, src, dst, tb + t, obj)));
     else
-      HIP_TRY((fwd_batch<R, true, false>(b, src, dst, 0, t + 1)));
+      HIP_TRY((fwd_batch<R, false>(b, src, dst, 0, obj)));
     src = dst;
   }
   if (T > 0) {
-    hipLaunchKernelGGL(A::k_obj_sum_b<R>, dim3(unsigned(T), nm), dim3(A::kThreads), 0, b->stream,
-                       static_cast<const A::Entry<R>*>(b->d_tab));
-    HIP_TRY(hipGetLastError());
+    if (T + 1 - base > kObjStates) {
+      HIP_TRY(obj_flush_batch<R>(b, base, T - base));
+      base = T;
+    }
+    HIP_TRY(obj_state_batch<R>(b, src, T - base));
+    HIP_TRY(obj_flush_batch<R>(b, base, T + 1 - base));
   }
   HIP_TRY(hipEventRecord(b->e1, b->stream));
   std::vector<double> jt(size_t(nm) * size_t(T + 1), 0.0);
@@ -1261,26 +1856,32 @@ int batch_backward_impl(flb_adjoint_batch_s* b, double* grad) {
   const int tb = tape_base(T, K);
   int cur = 0;
   if (K == 0) {
-    for (int t = T - 1; t >= 0; --t) {
-      HIP_TRY(bwd_batch<R>(b, tb + t, kSlotL0 + cur, kSlotL0 + (cur ^ 1), t >= 1));
-      cur ^= 1;
-    }
+    HIP_TRY(bwd_run_batch<R>(b, tb, 0, T, cur));
   } else {
     const int nseg = (T + K - 1) / K;
     for (int k = nseg - 1; k >= 0; --k) {
       const int t0 = k * K, t1 = std::min((k + 1) * K, T);
       // as backward_impl: moment records of states t0 .. t1-1, then the adjoint steps
-      int src = kSlotCk + k;
-      for (int t = t0; t < t1 - 1; ++t) {
-        const int dst = kSlotR0 + ((t - t0) & 1);
-        HIP_TRY((fwd_batch<R, false, true>(b, src, dst, tb + (t - t0), 0)));
+      int src = kSlotCk + k, t = t0, r = 0;
+      while (t < t1) {
+        const int mom = tb + t - t0, dst = kSlotR0 + r;
+        if (b->march == 1 && t + 2 < t1) {
+          HIP_TRY((march_batch<R, false, true, true>(b, {src, dst, mom, mom + 1, -1, -1, 0, 0})));
+          t += 2;
+        } else if (b->march == 1 && t + 2 == t1) {
+          HIP_TRY((march_batch<R, false, true, false>(b, {src, 0, mom, mom + 1, -1, -1, 0, 0})));
+          t += 2;
+        } else if (t + 1 < t1) {
+          HIP_TRY((fwd_batch<R, true>(b, src, dst, mom, -1)));
+          t += 1;
+        } else {
+          HIP_TRY(mom_batch<R>(b, src, mom));
+          t += 1;
+        }
         src = dst;
+        r ^= 1;
       }
-      HIP_TRY(mom_batch<R>(b, src, tb + (t1 - 1 - t0)));
-      for (int t = t1 - 1; t >= t0; --t) {
-        HIP_TRY(bwd_batch<R>(b, tb + (t - t0), kSlotL0 + cur, kSlotL0 + (cur ^ 1), t >= 1));
-        cur ^= 1;
-      }
+      HIP_TRY(bwd_run_batch<R>(b, tb, t0, t1, cur));
     }
   }
   HIP_TRY(hipEventRecord(b->e1, b->stream));
@@ -1350,7 +1951,7 @@ int flb_adjoint_destroy(flb_adjoint h) {
   free_vec(h->ckpt, h->d_f0);
   free_vec(h->mtape, nullptr);
   void* ptrs[] = {h->d_solid, h->d_link, h->d_s, h->d_f0, h->d_work[0], h->d_work[1], h->d_lam[0], h->d_lam[1],
-                  h->d_rec[0], h->d_rec[1], h->d_grad, h->d_jt, h->d_partial};
+                  h->d_rec[0], h->d_rec[1], h->d_grad, h->d_jt, h->d_shares};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (h->e0) (void)hipEventDestroy(h->e0);
@@ -1521,6 +2122,10 @@ int flb_adjoint_batch_destroy(flb_adjoint_batch b) {
   (void)hipStreamSynchronize(b->stream);
   if (b->d_tab) (void)hipFree(b->d_tab);
   if (b->d_slots) (void)hipFree(b->d_slots);
+  for (int k = 0; k < 2; ++k) {
+    if (b->d_mt[k]) (void)hipFree(b->d_mt[k]);
+    if (b->d_mwg[k]) (void)hipFree(b->d_mwg[k]);
+  }
   if (b->e0) (void)hipEventDestroy(b->e0);
   if (b->e1) (void)hipEventDestroy(b->e1);
   delete b;

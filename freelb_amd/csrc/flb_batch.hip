@@ -11,9 +11,6 @@
 
 #include <algorithm>
 #include <cstring>
-#include <functional>
-#include <queue>
-#include <utility>
 #include <vector>
 
 #include "../../include/flb_abi.h"
@@ -66,12 +63,12 @@ struct flb_batch_s {
   March march, graph_march;  // now, and as recorded (state 1: the graph holds passes of two steps)
   std::vector<flb::MarchArgs> h_mt;
   std::vector<flb::MarchWg> h_mwg;
-  std::vector<int> h_ext;  // extents that h_mt's tiles and h_mwg were planned for
+  std::vector<flbh::MarchBox> h_ext;  // extents that h_mt's tiles and h_mwg were planned for
   flb::MarchArgs* d_mt = nullptr;
   flb::MarchWg* d_mwg = nullptr;
   size_t mwg_cap = 0;
   char* d_alt = nullptr;
-  double march_span = 0.0;  // estimated time of a pass, in march_tiles' unit
+  double march_span = 0.0;  // estimated time of a pass, in march_plan_batch's unit
 };
 
 namespace {
@@ -171,67 +168,6 @@ int refresh(flb_batch_s* t, bool force) {
   return FLB_OK;
 }
 
-// The last end of work given longest first to the device's workgroup slots
-// (one per CU); `work` holds estimated times and how many workgroups take
-// them, longest first. Long lists end evenly.
-double march_span(const std::vector<std::pair<double, int64_t>>& work, int cus) {
-  double total = 0.0;
-  int64_t wgs = 0;
-  for (const auto& w : work) {
-    total += w.first * double(w.second);
-    wgs += w.second;
-  }
-  if (wgs > int64_t(16) * cus) return total / cus + 0.5 * work.front().first;
-  std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
-  for (int k = 0; k < cus; ++k) ends.push(0.0);
-  double span = 0.0;
-  for (const auto& w : work)
-    for (int64_t k = 0; k < w.second; ++k) {
-      const double e = ends.top() + w.first;
-      ends.pop();
-      ends.push(e);
-      span = std::max(span, e);
-    }
-  return span;
-}
-
-// Tiles of every block and the order of all workgroups, for the chunk length
-// with the least estimated time. The order is longest workgroup first, so the
-// uneven end of a launch is one of the short ones.
-double plan_march(flb_batch_s* t, int cus) {
-  const size_t nb = t->blocks.size();
-  const int elem = int(t->blocks[0]->elem);
-  double best_span = 1e300;
-  int best = 8;
-  std::vector<double> one(nb);
-  std::vector<size_t> order(nb);
-  const auto tiles = [&](int len) {
-    for (size_t k = 0; k < nb; ++k) {
-      one[k] = march_tiles(t->h_tab[k], elem, len, &t->h_mt[k]);
-      order[k] = k;
-    }
-    std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return one[x] > one[y] || (one[x] == one[y] && x < y); });
-  };
-  std::vector<std::pair<double, int64_t>> work;
-  for (int len : {4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64, 96}) {
-    tiles(len);
-    work.clear();
-    for (size_t k : order) work.emplace_back(one[k], int64_t(t->h_mt[k].ntx) * t->h_mt[k].nty * t->h_mt[k].nz);
-    const double span = march_span(work, cus);
-    if (span < best_span) {
-      best_span = span;
-      best = len;
-    }
-  }
-  tiles(best);
-  t->h_mwg.clear();
-  for (size_t k : order) {
-    const int n = t->h_mt[k].ntx * t->h_mt[k].nty * t->h_mt[k].nz;
-    for (int w = 0; w < n; ++w) t->h_mwg.push_back({int(k), w});
-  }
-  return best_span;
-}
-
 // Whether runs of steps may take two steps per pass: checked, and the tables
 // built, once after a change (with a wait for the device, so not in a
 // capture). They do where every block is of the march's form, all of one
@@ -251,7 +187,7 @@ int prepare_march(flb_batch_s* t) {
   if (t->halo) return FLB_OK;
   const size_t nb = t->blocks.size();
   std::vector<flb::MarchArgs> form(nb);
-  std::vector<int> ext;
+  std::vector<MarchBox> ext;
   mc.per = false;
   for (size_t k = 0; k < nb; ++k) {
     flb_block_s* b = t->blocks[k];
@@ -263,7 +199,7 @@ int prepare_march(flb_batch_s* t) {
     mc.per = mc.per || a.px || a.py || a.pz;
     live += size_t(19) * size_t(a.ex) * size_t(a.ey) * size_t(a.ez) * b->elem;
     alt += (size_t(b->pop_elems) * b->elem + 255) / 256 * 256;
-    ext.insert(ext.end(), {a.ex, a.ey, a.ez});
+    ext.push_back({a.ex, a.ey, a.ez, a.pitch});
   }
   // the periodic form of the kernel addresses every block from its start
   for (size_t k = 0; mc.per && k < nb; ++k)
@@ -273,8 +209,8 @@ int prepare_march(flb_batch_s* t) {
   if (ext != t->h_ext) {
     int cus = 0;
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, t->device));
-    t->h_mt.assign(nb, flb::MarchArgs{});
-    t->march_span = plan_march(t, cus);
+    t->march_span = march_plan_batch(ext, int(t->blocks[0]->elem), cus, flb::march_threads(t->blocks[0]->elem), t->h_mt,
+                                      t->h_mwg);
     t->h_ext = ext;
   }
   // a unit of the estimate is 0.75 to 0.94 us, single steps move 4.2 to 5.5 TB/s

@@ -152,13 +152,21 @@ int march_run(flb_block_s* b, int n);
 // step against 9.8 us here, 80^3: 15.9 against 13.8; FP64 32^3: 5.7 against
 // 7.7, 64^3: 15.3 against 14.4). Batches count the populations of all blocks.
 constexpr size_t kMarchMinBytes = size_t(32) << 20;
-// For batches: march_form sets *ok where a block of any size is of the form
-// the march takes, with its flags and dynamics in m (not its tiles);
-// march_tiles gives it tiles of at most zchunk planes and returns the
-// estimated time of one of its workgroups; march_fits: whether a second array
-// of `bytes` leaves the device enough memory.
+// march_form sets *ok where a block of any size is of the form the march
+// takes, with its flags and dynamics in m (not its tiles). march_plan: tiles
+// of one box of cells (rows of `pitch` slots) for
+// workgroups of `threads`; march_plan_batch: those of
+// several in one launch and the order of its workgroups, returns the estimated
+// time of a pass in units of 0.75 to 0.94 us. march_fits: whether second
+// arrays of `bytes` leave the device enough memory.
+struct MarchBox {
+  int ex, ey, ez, pitch;
+  bool operator==(const MarchBox& o) const { return ex == o.ex && ey == o.ey && ez == o.ez && pitch == o.pitch; }
+};
 int march_form(flb_block_s* b, flb::MarchArgs* m, bool* ok);
-double march_tiles(const flb::KArgs& a, int elem, int zchunk, flb::MarchArgs* m);
+flb::MarchArgs march_plan(const MarchBox& box, int elem, int cus, int threads);
+double march_plan_batch(const std::vector<MarchBox>& boxes, int elem, int cus, int threads,
+                        std::vector<flb::MarchArgs>& mt, std::vector<flb::MarchWg>& wgs);
 bool march_fits(size_t bytes);
 bool capturing(hipStream_t s);
 

@@ -4,6 +4,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <functional>
+#include <queue>
+#include <utility>
+#include <vector>
 
 #include "flb_host.hpp"
 #include "flb_internal.hpp"
@@ -21,8 +25,8 @@ double plane_time(int w, int h, int ntx, int elem) {
 
 // Calls f(w, h, ntx, nty) for the tile extents worth considering.
 template <class F>
-void each_tile(const KArgs& a, int elem, F&& f) {
-  const int threads = flb::march_threads(size_t(elem)), line = 128 / elem;
+void each_tile(const MarchBox& a, int elem, int threads, F&& f) {
+  const int line = 128 / elem;
   for (int n = 1; n <= a.ex; ++n) {
     int w = (a.ex + n - 1) / n;
     if (a.pitch >= 256) w = (w + line - 1) / line * line;
@@ -36,6 +40,8 @@ void each_tile(const KArgs& a, int elem, F&& f) {
   }
 }
 
+}  // namespace
+
 // Tiles and z chunks of the block: the split with the least estimated time,
 // rounds of the device's workgroup slots (one per CU) times the planes each
 // workgroup collides times the time of a plane. A plane's time grows with the
@@ -45,10 +51,10 @@ void each_tile(const KArgs& a, int elem, F&& f) {
 // each, where the split chosen takes 1.02 times the best one's time in the
 // mean (1.14 at worst). Rows of 256 slots and more start on line boundaries:
 // their tiles do too.
-flb::MarchArgs plan(const KArgs& a, int elem, int cus) {
+flb::MarchArgs march_plan(const MarchBox& a, int elem, int cus, int threads) {
   flb::MarchArgs best{};
   double best_cost = 1e300;
-  each_tile(a, elem, [&](int w, int h, int ntx, int nty) {
+  each_tile(a, elem, threads, [&](int w, int h, int ntx, int nty) {
     const double plane = plane_time(w, h, ntx, elem);
     const int64_t tiles = int64_t(ntx) * nty;
     for (int rounds = 1; rounds <= 4; ++rounds) {
@@ -68,6 +74,8 @@ flb::MarchArgs plan(const KArgs& a, int elem, int cus) {
   });
   return best;
 }
+
+namespace {
 
 // The flags and the dynamics of the block's updated cells when one dynamics
 // that the march is built for serves them all.
@@ -122,9 +130,13 @@ int march_form(flb_block_s* b, flb::MarchArgs* m, bool* ok) {
   return rc;
 }
 
-double march_tiles(const KArgs& a, int elem, int zchunk, flb::MarchArgs* m) {
+namespace {
+
+// Tiles of at most zchunk planes for a box of a batch; returns the estimated
+// time of one of its workgroups.
+double march_tiles(const MarchBox& a, int elem, int threads, int zchunk, flb::MarchArgs* m) {
   double best = 1e300, plane = 0.0;
-  each_tile(a, elem, [&](int w, int h, int ntx, int nty) {
+  each_tile(a, elem, threads, [&](int w, int h, int ntx, int nty) {
     const double t = plane_time(w, h, ntx, elem), cost = t * ntx * nty;
     if (cost < best) {
       best = cost;
@@ -139,6 +151,70 @@ double march_tiles(const KArgs& a, int elem, int zchunk, flb::MarchArgs* m) {
   m->zchunk = (a.ez + m->nz - 1) / m->nz;
   m->nz = (a.ez + m->zchunk - 1) / m->zchunk;
   return plane * (m->zchunk + 2);
+}
+
+// The last end of work given longest first to the device's workgroup slots
+// (one per CU); `work` holds estimated times and how many workgroups take
+// them, longest first. Long lists end evenly.
+double march_span(const std::vector<std::pair<double, int64_t>>& work, int cus) {
+  double total = 0.0;
+  int64_t wgs = 0;
+  for (const auto& w : work) {
+    total += w.first * double(w.second);
+    wgs += w.second;
+  }
+  if (wgs > int64_t(16) * cus) return total / cus + 0.5 * work.front().first;
+  std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
+  for (int k = 0; k < cus; ++k) ends.push(0.0);
+  double span = 0.0;
+  for (const auto& w : work)
+    for (int64_t k = 0; k < w.second; ++k) {
+      const double e = ends.top() + w.first;
+      ends.pop();
+      ends.push(e);
+      span = std::max(span, e);
+    }
+  return span;
+}
+
+}  // namespace
+
+// Tiles of every box and the order of all workgroups, for the chunk length
+// with the least estimated time. The order is longest workgroup first, so the
+// uneven end of a launch is one of the short ones.
+double march_plan_batch(const std::vector<MarchBox>& boxes, int elem, int cus, int threads, std::vector<flb::MarchArgs>& mt,
+                        std::vector<flb::MarchWg>& wgs) {
+  const size_t nb = boxes.size();
+  mt.assign(nb, flb::MarchArgs{});
+  double best_span = 1e300;
+  int best = 8;
+  std::vector<double> one(nb);
+  std::vector<size_t> order(nb);
+  const auto tiles = [&](int len) {
+    for (size_t k = 0; k < nb; ++k) {
+      one[k] = march_tiles(boxes[k], elem, threads, len, &mt[k]);
+      order[k] = k;
+    }
+    std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return one[x] > one[y] || (one[x] == one[y] && x < y); });
+  };
+  std::vector<std::pair<double, int64_t>> work;
+  for (int len : {4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64, 96}) {
+    tiles(len);
+    work.clear();
+    for (size_t k : order) work.emplace_back(one[k], int64_t(mt[k].ntx) * mt[k].nty * mt[k].nz);
+    const double span = march_span(work, cus);
+    if (span < best_span) {
+      best_span = span;
+      best = len;
+    }
+  }
+  tiles(best);
+  wgs.clear();
+  for (size_t k : order) {
+    const int n = mt[k].ntx * mt[k].nty * mt[k].nz;
+    for (int w = 0; w < n; ++w) wgs.push_back({int(k), w});
+  }
+  return best_span;
 }
 
 // Second arrays take at most a sixteenth of the device's memory and leave
@@ -190,7 +266,7 @@ int march_run(flb_block_s* b, int n) {
   int cus = 0;
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
   KArgs a = make_args(b);
-  flb::MarchArgs m = plan(a, int(b->elem), cus);
+  flb::MarchArgs m = march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem));
   one_dynamics(b, &m);
   char* const pops = static_cast<char*>(b->d_pops) + flb::kFrontPad * b->elem;
   char* const alt = static_cast<char*>(b->d_alt) + flb::kFrontPad * b->elem;

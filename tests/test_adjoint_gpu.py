@@ -106,6 +106,66 @@ def test_checkpoint_modes_agree_bitwise(storage):
         assert J == J0 and np.array_equal(st, s0) and np.array_equal(g, g0)
 
 
+@pytest.mark.parametrize("storage,dims,per,solids", [
+    ("f32", (131, 60, 60), (True, False, False), True), ("f32", (75, 66, 101), (False, True, True), True),
+    ("f32", (64, 96, 80), (False, False, False), False), ("f32", (200, 130, 18), (True, True, True), False),
+    ("f64", (90, 51, 60), (True, False, True), True), ("f64", (33, 140, 55), (False, False, False), False)])
+def test_two_steps_per_pass_equal_single_steps(storage, dims, per, solids):
+    """Boxes of 32 MiB of populations and more: checkpoints at every state (K 1) leave only single
+    steps; with them further apart or none, two steps are taken per pass. Objective, final state
+    and gradient, bit for bit, from runs of odd and even length."""
+    N = int(np.prod(dims))
+    rng = np.random.default_rng(7)
+    solid = rng.random(N) < 0.03 if solids else np.zeros(N, dtype=bool)
+    with Adjoint(dims, omega=1 / TAU, force=G, brinkman_alpha=ALPHA, periodic=per, storage=storage,
+                 outlet_x=dims[0] - 2) as adj:
+        adj.set_solid(solid)
+        adj.set_fraction(rng.uniform(0, 1, N))
+        adj.init_equilibrium(1 + 0.01 * rng.standard_normal(N), 0.02 * rng.standard_normal((3, N)))
+        for T in (7, 36):
+            J1, s1, g1 = adj.forward(T, 1), adj.state(), adj.backward()
+            for K in (0, 3, 4, T) if T < 10 else (5,):
+                J, st, g = adj.forward(T, K), adj.state(), adj.backward()
+                assert J == J1, K
+                assert np.array_equal(st, s1), K
+                assert np.array_equal(g, g1), K
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+def test_batch_passes_of_two_steps_equal_single_steps(storage):
+    """Members of different sizes and walls, 32 MiB of populations and more together: each equals
+    its own run in single steps (a checkpoint at every state), bit for bit."""
+    specs = [((131, 60, 60), (True, False, False), 0.03), ((75, 66, 101), (False, True, True), 0.0),
+             ((64, 96, 80), (False, False, False), 0.05), ((200, 130, 32), (True, True, True), 0.0),
+             ((10, 6, 5), (True, False, True), 0.1), ((96, 93, 97), (False, True, False), 0.0),
+             ((90, 80, 70), (True, False, False), 0.01)]
+    members = []
+    for k, (dims, per, share) in enumerate(specs):
+        N = int(np.prod(dims))
+        rng = np.random.default_rng(60 + k)
+        a = Adjoint(dims, omega=1 / (0.6 + 0.1 * k), force=(1e-3, -2e-4 * k, 1e-4), brinkman_alpha=0.2 + 0.1 * k,
+                    outlet_x=dims[0] - 1 - k, periodic=per, storage=storage)
+        a.set_solid(rng.random(N) < share)
+        a.set_fraction(rng.uniform(0, 1, N))
+        a.init_equilibrium(1 + 0.01 * rng.standard_normal(N), 0.02 * rng.standard_normal((3, N)))
+        members.append(a)
+    try:
+        T = 9
+        solo = [(a.forward(T, 1), a.state(), a.backward()) for a in members]
+        with AdjointBatch(members) as b:
+            for K in (0, 3, 4, T):
+                J = b.forward(T, K)
+                states = [a.state() for a in members]
+                grads = b.backward()
+                for k, (J1, s1, g1) in enumerate(solo):
+                    assert J[k] == J1, (K, k)
+                    assert np.array_equal(states[k], s1), (K, k)
+                    assert np.array_equal(grads[k], g1), (K, k)
+    finally:
+        for a in members:
+            a.close()
+
+
 def test_gradient_against_fd_fp64():
     adj, model, f0, s, solid = _setup()
     with adj:
