@@ -209,6 +209,16 @@ KArgs make_args(const flb_block_s* b) {
     a.nblocks = int((waves + a.wpb - 1) / a.wpb);
   }
   a.ntasks = b->ntasks;
+  a.dyns = 0;
+  a.anymask = 0;
+  bool same = true;
+  for (int t = 0; t < b->ntasks; ++t) {
+    a.dyns |= 1 << b->tasks[t].dynamics;
+    a.anymask |= uint8_t(b->tasks[t].mask);
+    for (int k = 0; k < t; ++k)
+      same = same && (b->tasks[k].dynamics != b->tasks[t].dynamics || b->tasks[k].smagorinsky == b->tasks[t].smagorinsky);
+  }
+  if (!same) a.dyns = 0;
   for (int t = 0; t < b->ntasks; ++t) {
     a.tmask[t] = b->tasks[t].mask;
     a.tdyn[t] = b->tasks[t].dynamics;

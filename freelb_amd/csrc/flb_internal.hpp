@@ -32,6 +32,27 @@ constexpr int kFrontPad = 256;
 // it, so the common BGK / bounce-back step does not pay the registers of MRT.
 // FAM_SCALAR is the advection-diffusion family of the D2Q5 / D3Q7 lattices.
 enum Family { FAM_BGK = 0, FAM_FULL = 1, FAM_SCALAR = 2 };
+// A family of exactly the dynamics in a bit set: the step kernels of the sets
+// that blocks commonly hold (with_set) carry no other collision and, with one
+// dynamics, no choice between any: MRT with LES, bound by its vector
+// instructions (482 to 546 per cell of the general kernels), gains most. Per
+// step, FP16 shift: MRT-LES 200x129x97 45.8 -> 39.6 us, 256x128x64 44.8 ->
+// 40.5; BGK 190x161x130 50.6 -> 49.8 (FP16C 57.5 -> 55.6); FP32 heated 30^3
+// 9.4 -> 8.9, refined 60 / 40 19.2 -> 18.6; larger FP32 blocks are bound by
+// memory and the same.
+constexpr int kFamSet = 1 << 16;
+constexpr int fam_set() { return kFamSet; }
+template <class... D>
+constexpr int fam_set(int dyn, D... more) { return (1 << dyn) | fam_set(more...); }
+// The one dynamics of such a family, or 0.
+constexpr int fam_only(int fam) {
+  if (fam < kFamSet) return 0;
+  const int m = fam & (kFamSet - 1);
+  if (m & (m - 1)) return 0;
+  int d = 0;
+  while ((m >> d) > 1) ++d;
+  return d;
+}
 
 // Buoyancy couplings one flow block can carry (FreeLB's examples couple a
 // temperature and a concentration lattice).
@@ -59,6 +80,8 @@ struct KArgs {
   int wpb;               // wavefronts per workgroup
   int nblocks;           // workgroups
   int ntasks;
+  int dyns;              // bit set of the tasks' dynamics, 0 if two tasks of one dynamics differ in its constant
+  uint8_t anymask;       // OR of tmask
   int nbc;
   uint8_t tmask[kMaxTasks];
   uint8_t tdyn[kMaxTasks];

@@ -129,6 +129,39 @@ __device__ __forceinline__ int match_task(const KArgs& a, uint8_t fl, float& cs)
   return DYN_NONE;
 }
 
+// match_task for a family: its one dynamics needs no search.
+template <int FAM>
+__device__ __forceinline__ int match_family(const KArgs& a, uint8_t fl, float& cs) {
+  if constexpr (fam_only(FAM) != 0) {
+    cs = a.tcs[0];
+    return (fl & a.anymask) ? fam_only(FAM) : int(DYN_NONE);
+  } else {
+    return match_task(a, fl, cs);
+  }
+}
+
+// Whether a family's collisions include a flow dynamics.
+constexpr bool fam_has(int fam, int dyn) {
+  if (fam >= kFamSet) return (fam >> dyn) & 1;
+  return fam == FAM_FULL || dyn == DYN_BGK || dyn == DYN_BGK_FIELD || dyn == DYN_BB || dyn == DYN_BB_MW;
+}
+constexpr bool fam_beyond(int fam) {
+  return fam_has(fam, DYN_MRT) || fam_has(fam, DYN_SMAG_BGK) || fam_has(fam, DYN_SMAG_MRT) ||
+         fam_has(fam, DYN_BGK_FORCE) || fam_has(fam, DYN_BGK_WRITE) || fam_has(fam, DYN_BGK_SCALAR_FORCE);
+}
+
+// Keeps the collided values of a set family apart from their conversion to 16
+// bits: with no choice of dynamics between the two, the compiler would round
+// once where the other kernels round twice (v_fma_mixlo_f16), and a block's
+// bits would depend on the kernel.
+template <int FAM, class S, int Q, class R>
+__device__ __forceinline__ void settle(R (&f)[Q]) {
+  if constexpr (FAM >= kFamSet && sizeof(typename S::E) == 2) {
+#pragma unroll
+    for (int i = 0; i < Q; ++i) asm("" : "+v"(f[i]));
+  }
+}
+
 // Halfway wall links of a cell (bit k: neighbour x + c_k is a wall), split by
 // kind; managers apply in order so a later match overrides an earlier one
 // (BlockFixedBoundary::addtoBd, basic_boundary.h:198-212).
@@ -191,14 +224,15 @@ __device__ __forceinline__ void sub_w(R (&f)[Q]) {
 // BGK writing its moments, Smagorinsky BGK, MRT and MRT+LES). DEV (D3Q19
 // only): f holds the deviations f - w; BGK, the Smagorinsky omega and MRT
 // then run on them, the forced dynamics on f = g + w.
-template <int Q, class R, bool DEV>
+template <int Q, class R, int FAM, bool DEV>
 __device__ __forceinline__ void collide_full(const KArgs& a, int slot, int dyn, float cs, R (&f)[Q],
                                              R om, R _om) {
   static_assert(!DEV || Q == 19, "deviation form of the full family: D3Q19");
+  auto is = [&](int d) { return fam_has(FAM, d) && dyn == d; };
   R rho, u[3], rho_f, u_f[3];
-  if (dyn == DYN_BGK_FORCE || dyn == DYN_BGK_SCALAR_FORCE) {
+  if (is(DYN_BGK_FORCE) || is(DYN_BGK_SCALAR_FORCE)) {
     if constexpr (DEV) add_w<Q>(f);
-    if (dyn == DYN_BGK_FORCE) {
+    if (is(DYN_BGK_FORCE)) {
       const R F[3] = {R(a.force[0]), R(a.force[1]), R(a.force[2])};
       bgk_force<Q>(f, F, om, _om);
     } else {
@@ -220,32 +254,32 @@ __device__ __forceinline__ void collide_full(const KArgs& a, int slot, int dyn, 
   }
   if constexpr (DEV) {
     // MRT and MRT + LES from the moments of the deviations (mrt_dev)
-    if (dyn == DYN_MRT || dyn == DYN_SMAG_MRT) {
+    if (is(DYN_MRT) || is(DYN_SMAG_MRT)) {
       const R* sn;
       if constexpr (sizeof(R) == 8) sn = a.mrt_sn_d;
       else sn = a.mrt_sn_f;
       rho_f = R(1);
-      if (dyn == DYN_SMAG_MRT) load_fields<Q>(a, slot, rho_f, u_f);
-      mrt_dev(f, om, dyn == DYN_SMAG_MRT, R(cs), rho_f, sn, a.mrt_shear);
+      if (is(DYN_SMAG_MRT)) load_fields<Q>(a, slot, rho_f, u_f);
+      mrt_dev(f, om, is(DYN_SMAG_MRT), R(cs), rho_f, sn, a.mrt_shear);
       return;
     }
   }
   R d = R(0);
   if constexpr (DEV) rhou_dev<Q>(f, d, rho, u);
   else rhou(f, rho, u);
-  if (dyn == DYN_BGK_WRITE) {
+  if (is(DYN_BGK_WRITE)) {
     store_fields<Q>(a, slot, rho, u);
     if constexpr (DEV) bgk_dev<Q>(f, d, rho, u, om, _om);
     else bgk_with<Q>(f, rho, u, om, _om);
     return;
   }
   R eo = om;
-  if (dyn == DYN_SMAG_BGK || dyn == DYN_SMAG_MRT) {
+  if (is(DYN_SMAG_BGK) || is(DYN_SMAG_MRT)) {
     load_fields<Q>(a, slot, rho_f, u_f);
     if constexpr (Q == 19) eo = smag_omega<DEV>(f, rho, u, om, R(cs), rho_f, d);
     else eo = smag_omega(f, rho, u, om, R(cs), rho_f);
   }
-  if (dyn == DYN_SMAG_BGK) {
+  if (is(DYN_SMAG_BGK)) {
     if constexpr (DEV) bgk_dev<Q>(f, d, rho, u, eo, R(1) - eo);
     else bgk_with<Q>(f, rho, u, eo, R(1) - eo);
   } else {
@@ -268,7 +302,7 @@ __device__ __forceinline__ void collide_full(const KArgs& a, int slot, int dyn, 
 template <int Q, class R, int FAM, bool DEV = false>
 __device__ __forceinline__ void collide(const KArgs& a, int slot, int dyn, float cs, R (&f)[Q],
                                         R om, R _om) {
-  if constexpr (FAM == FAM_SCALAR) {
+  if constexpr (kScalarLat<Q>) {
     // Advection-diffusion (collision::BGK, collision.h:39-56): the scalar is
     // advected by the VELOCITY field (moment::useFieldU, moment.h:56-69);
     // DYN_SCALAR_BGK sums it and writes it to the field
@@ -294,7 +328,8 @@ __device__ __forceinline__ void collide(const KArgs& a, int slot, int dyn, float
   R rho, u[3], rho_f, u_f[3];
   switch (dyn) {
     case DYN_BGK:
-      if constexpr (DEV) {
+      if constexpr (!fam_has(FAM, DYN_BGK)) {
+      } else if constexpr (DEV) {
         R d;
         rhou_dev<Q>(f, d, rho, u);
         bgk_dev<Q>(f, d, rho, u, om, _om);
@@ -304,23 +339,25 @@ __device__ __forceinline__ void collide(const KArgs& a, int slot, int dyn, float
       }
       break;
     case DYN_BGK_FIELD:
+      if constexpr (!fam_has(FAM, DYN_BGK_FIELD)) break;
       load_fields<Q>(a, slot, rho_f, u_f);
       if constexpr (DEV) bgk_dev<Q>(f, rho_f - R(1), rho_f, u_f, om, _om);
       else bgk_with<Q>(f, rho_f, u_f, om, _om);
       break;
     case DYN_BB:
-      bounceback<Q>(f);
+      if constexpr (fam_has(FAM, DYN_BB)) bounceback<Q>(f);
       break;
     case DYN_BB_MW:
+      if constexpr (!fam_has(FAM, DYN_BB_MW)) break;
       load_fields<Q>(a, slot, rho_f, u_f);
       bounceback_moving<Q>(f, rho_f, u_f);
       break;
     default:
-      if constexpr (FAM == FAM_FULL) {
+      if constexpr (fam_beyond(FAM)) {
         // D2Q9's full family (FreeLB's closed-form MRT) runs on f
         constexpr bool dev19 = DEV && Q == 19;
         if constexpr (DEV && !dev19) add_w<Q>(f);
-        collide_full<Q, R, dev19>(a, slot, dyn, cs, f, om, _om);
+        collide_full<Q, R, FAM, dev19>(a, slot, dyn, cs, f, om, _om);
         if constexpr (DEV && !dev19) sub_w<Q>(f);
       }
       break;
@@ -601,6 +638,7 @@ __device__ __forceinline__ void odd_buf(const KArgs& a, __amdgpu_buffer_rsrc_t r
   wall_terms_in<Q>(a, s0, lm, f);
   const R om = R(a.omega);
   collide<Q, R, FAM, kDev<Q, S>>(a, s0, dyn, cs, f, om, R(1) - om);
+  settle<FAM, S>(f);
   wall_terms_out<Q>(a, s0, lm, f);
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
@@ -686,7 +724,7 @@ __device__ __forceinline__ void cell_update_at(const KArgs& a, int c0, int y, in
   }();
   const uint8_t fl = a.flags[s0];
   float cs = 0.0f;
-  const int dyn = match_task(a, fl, cs);
+  const int dyn = match_family<FAM>(a, fl, cs);
   if (dyn == DYN_NONE) return;
   unsigned ln = 0u, lm = 0u;
   if (!EVEN && (fl & a.bcany)) {
@@ -706,6 +744,7 @@ __device__ __forceinline__ void cell_update_at(const KArgs& a, int c0, int y, in
     for (int i = 0; i < Q; ++i) f[i] = pop_dec<Q, S>(bld_pop_s<PAR, E>(rs, vo, uint32_t(B + i * dp) * el), i);
     const R om = R(a.omega);
     collide<Q, R, FAM, kDev<Q, S>>(a, s0, dyn, cs, f, om, R(1) - om);
+    settle<FAM, S>(f);
 #pragma unroll
     for (int i = 0; i < Q; ++i)
       bst_pop_s<PAR, E>(rs, vo, uint32_t(B + opp(i) * dp) * el, pop_enc<Q, S>(f[i], i));
@@ -736,6 +775,7 @@ __device__ __forceinline__ void cell_update_at(const KArgs& a, int c0, int y, in
   if (!EVEN) wall_terms_in<Q>(a, s0, lm, f);
   const R om = R(a.omega);
   collide<Q, R, FAM, kDev<Q, S>>(a, s0, dyn, cs, f, om, R(1) - om);
+  settle<FAM, S>(f);
   if (!EVEN) wall_terms_out<Q>(a, s0, lm, f);
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
@@ -790,8 +830,8 @@ __global__ __launch_bounds__(kMaxThreads) void k_step_even_pair(KArgs a) {
   const uint32_t vo = uint32_t(c0) * 2u;
   const int32_t dp = int32_t(a.dpop);
   float cs0 = 0.0f, cs1 = 0.0f;
-  const int d0 = match_task(a, a.flags[s0], cs0);
-  const int d1 = two ? match_task(a, a.flags[s0 + 1], cs1) : int(DYN_NONE);
+  const int d0 = match_family<FAM>(a, a.flags[s0], cs0);
+  const int d1 = two ? match_family<FAM>(a, a.flags[s0 + 1], cs1) : int(DYN_NONE);
   if (d0 == DYN_NONE && d1 == DYN_NONE) return;
   R f0[Q], f1[Q];
 #pragma unroll
@@ -807,7 +847,9 @@ __global__ __launch_bounds__(kMaxThreads) void k_step_even_pair(KArgs a) {
   }
   const R om = R(a.omega);
   if (d0 != DYN_NONE) collide<Q, R, FAM, kDev<Q, S>>(a, s0, d0, cs0, f0, om, R(1) - om);
+  settle<FAM, S>(f0);
   if (d1 != DYN_NONE) collide<Q, R, FAM, kDev<Q, S>>(a, s0 + 1, d1, cs1, f1, om, R(1) - om);
+  settle<FAM, S>(f1);
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
     E* const q = (P + int64_t(opp(i)) * a.dpop) + c0;
@@ -1325,10 +1367,39 @@ __global__ __launch_bounds__(kMaxThreads) void k_links(KArgs a, uint64_t* __rest
 #ifndef FLB_BUFFER_ADDR
 #define FLB_BUFFER_ADDR 1
 #endif
+// Calls f(std::integral_constant<int, F>) with the set family of the block's
+// dynamics, where there is one.
+template <int Q, class F>
+bool with_set(const KArgs& a, F&& f) {
+  auto is = [&](auto c) {
+    if (a.dyns == 0 || a.dyns != (decltype(c)::value & (kFamSet - 1))) return false;
+    f(c);
+    return true;
+  };
+  if constexpr (kScalarLat<Q>) {
+    return is(std::integral_constant<int, fam_set(DYN_SCALAR_BGK, DYN_SCALAR_BGK_FIELD)>{});
+  } else if constexpr (Q == 19) {
+    return is(std::integral_constant<int, fam_set(DYN_BGK)>{}) ||
+           is(std::integral_constant<int, fam_set(DYN_SMAG_MRT)>{}) ||
+           is(std::integral_constant<int, fam_set(DYN_BGK_FORCE)>{}) ||
+           is(std::integral_constant<int, fam_set(DYN_BGK_SCALAR_FORCE)>{}) ||
+           is(std::integral_constant<int, fam_set(DYN_BGK_WRITE)>{}) ||
+           is(std::integral_constant<int, fam_set(DYN_BGK_WRITE, DYN_BGK_FIELD)>{});
+  } else {
+    return is(std::integral_constant<int, fam_set(DYN_BGK)>{});
+  }
+}
+
 template <int Q, class S, int PAR>
 hipError_t step_cell_q(int family, bool per, const KArgs& a, hipStream_t s) {
   const dim3 grid(a.nblocks), block(kWave * a.wpb);
-  const bool buf = FLB_BUFFER_ADDR && PAR != 0 && a.buf != 0 && !per;
+  constexpr bool kBuf = FLB_BUFFER_ADDR && PAR != 0;
+  const bool buf = kBuf && a.buf != 0 && !per;
+  if (buf == kBuf && !per && with_set<Q>(a, [&](auto f) {
+        constexpr int F = decltype(f)::value;
+        hipLaunchKernelGGL((k_step_cell<Q, S, PAR, F, false, kBuf>), grid, block, 0, s, a);
+      }))
+    return hipGetLastError();
   if (family == FAM_FULL) {
     if (per) hipLaunchKernelGGL((k_step_cell<Q, S, PAR, FAM_FULL, true>), grid, block, 0, s, a);
     else if (buf) hipLaunchKernelGGL((k_step_cell<Q, S, PAR, FAM_FULL, false, true>), grid, block, 0, s, a);
@@ -1424,7 +1495,13 @@ template <int Q, class S, int PAR>
 hipError_t step_scalar_q(const KArgs& a, hipStream_t s) {
   const dim3 grid(a.nblocks), block(kWave * a.wpb);
   const bool per = a.px || a.py || a.pz;
-  const bool buf = FLB_BUFFER_ADDR && PAR != 0 && a.buf != 0 && !per;
+  constexpr bool kBuf = FLB_BUFFER_ADDR && PAR != 0;
+  const bool buf = kBuf && a.buf != 0 && !per;
+  if (buf == kBuf && !per && with_set<Q>(a, [&](auto f) {
+        constexpr int F = decltype(f)::value;
+        hipLaunchKernelGGL((k_step_cell<Q, S, PAR, F, false, kBuf>), grid, block, 0, s, a);
+      }))
+    return hipGetLastError();
   if (per) hipLaunchKernelGGL((k_step_cell<Q, S, PAR, FAM_SCALAR, true>), grid, block, 0, s, a);
   else if (buf) hipLaunchKernelGGL((k_step_cell<Q, S, PAR, FAM_SCALAR, false, true>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((k_step_cell<Q, S, PAR, FAM_SCALAR, false>), grid, block, 0, s, a);
@@ -1439,6 +1516,12 @@ hipError_t even_pair_q(int family, bool nt, const KArgs& a0, hipStream_t s) {
   a.wpr = (a.ex + 2 * kWave - 1) / (2 * kWave);
   a.nblocks = int((int64_t(a.wpr) * a.ey * a.ez + a.wpb - 1) / a.wpb);
   const dim3 grid(a.nblocks), block(kWave * a.wpb);
+  if (with_set<Q>(a, [&](auto f) {
+        constexpr int F = decltype(f)::value;
+        if (nt) hipLaunchKernelGGL((k_step_even_pair<Q, S, 0, F>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_step_even_pair<Q, S, 2, F>), grid, block, 0, s, a);
+      }))
+    return hipGetLastError();
   if (family == FAM_FULL) {
     if (nt) hipLaunchKernelGGL((k_step_even_pair<Q, S, 0, FAM_FULL>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((k_step_even_pair<Q, S, 2, FAM_FULL>), grid, block, 0, s, a);

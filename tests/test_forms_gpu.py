@@ -5,6 +5,8 @@ pitches. Same per-cell arithmetic, so results agree bit for bit."""
 import numpy as np
 import pytest
 
+from freelb_amd import BlockLattice, BlockLatticeManager, HalfwayBB, Key_TypePair, abi
+from freelb_amd.cases import FLUID, LID, VOID, WALL, cavity_flags
 from gpu_case import gpu_lattice, interior_mask
 from oracle import oracle as O
 
@@ -54,3 +56,39 @@ def test_d2q9_linear_form(monkeypatch, mode):
         assert np.array_equal(lat.pops()[:, inner], p[:, inner])
     finally:
         lat.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64", "f16s", "f16c", "bf16s"])
+@pytest.mark.parametrize("dyn", [abi.DYN_BGK, abi.DYN_SMAG_MRT, abi.DYN_BGK_FORCE, abi.DYN_BGK_WRITE])
+@pytest.mark.parametrize("dims", [(70, 9, 7), (23, 11, 5), (262, 5, 4)])
+def test_kernels_of_one_dynamics_equal_the_general_ones(storage, dyn, dims):
+    """A block whose cells share one dynamics steps in a kernel of that dynamics alone; the batched
+    step carries every dynamics of the family. Same bits, also in the fields."""
+    shape = tuple(n + 2 for n in dims)
+    flags = cavity_flags(*dims)
+    rng = np.random.default_rng(3)
+    u0 = rng.uniform(-0.02, 0.02, size=(3, flags.size))
+
+    def make():
+        lat = BlockLattice(19, shape, omega=1 / 0.6, storage=storage)
+        lat.upload_flags(flags)
+        lat.set_tasks([Key_TypePair(FLUID | WALL | LID, dyn, 0.17 if dyn == abi.DYN_SMAG_MRT else 0.0)])
+        lat.set_halfway_bc([HalfwayBB(WALL, VOID), HalfwayBB(LID, VOID, True)])
+        lat.set_field_rho(np.ones(flags.size))
+        lat.set_field_u(np.where(flags == LID, 0.05, 0.0) * np.array([[1.0], [0.0], [0.0]]))
+        lat.set_force((1e-5, 2e-6, -3e-6))
+        lat.init_equilibrium(np.ones(flags.size), u0)
+        return lat
+    a, b = make(), make()
+    try:
+        with BlockLatticeManager([b]) as m:
+            for n in (1, 2, 4):
+                for _ in range(n):
+                    a.step(1)
+                    m.step(1)
+                m.synchronize()
+                assert np.array_equal(a.pops(), b.pops()), n
+                assert np.array_equal(a.download_fields(), b.download_fields()), n
+    finally:
+        a.close()
+        b.close()
