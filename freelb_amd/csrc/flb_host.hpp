@@ -147,11 +147,19 @@ int ensure_links(flb_block_s* b);
 // by n steps (a multiple of 4).
 bool march_ready(flb_block_s* b);
 int march_run(flb_block_s* b, int n);
-// Populations of 32 MiB and more, what the eight L2 caches hold together: the
-// one-step kernels run smaller blocks out of the caches (FP32 64^3: 8.8 us a
-// step against 9.8 us here, 80^3: 15.9 against 13.8; FP64 32^3: 5.7 against
-// 7.7, 64^3: 15.3 against 14.4). Batches count the populations of all blocks.
-constexpr size_t kMarchMinBytes = size_t(32) << 20;
+// Bytes of populations from which on a block takes it; smaller ones run out of
+// the caches. BGK over 110 blocks of 34 MB to 300 MB: 0.95 to 1.06 times the
+// single steps' time up to 43 MB, 0.78 to 0.92 beyond. MRT with LES is bound by
+// its instructions, those of the ring's cells included: FP32 takes single
+// steps (1.0 to 1.4 times their time in the march up to 256^3), FP64 marches
+// from 400 MB on (140^3 180 -> 156 us, 200x160x150 303 -> 261; below 320 MB 1.0
+// to 1.5 times). In batches, whose single steps run at 4.5 TB/s, both take it
+// from there on (40 blocks of 481 MB: 234 -> 197 us), all blocks counted.
+constexpr size_t kMarchMinBytes = size_t(42) << 20;
+inline bool march_pays(int dyn, size_t elem, size_t bytes, bool batch) {
+  if (dyn == FLB_DYN_SMAG_MRT) return bytes >= size_t(400) * 1000 * 1000 && (batch || elem == 8);
+  return bytes >= kMarchMinBytes;
+}
 // march_form sets *ok where a block of any size is of the form the march
 // takes, with its flags and dynamics in m (not its tiles). march_plan: tiles
 // of one box of cells (rows of `pitch` slots) for

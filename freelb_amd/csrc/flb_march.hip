@@ -245,7 +245,9 @@ bool march_ready(flb_block_s* b) {
     flb::MarchArgs m;
     bool ok = false;
     const int64_t cells = int64_t(axis_ext(b, 0)) * axis_ext(b, 1) * axis_ext(b, 2);
-    if (size_t(19 * cells) * b->elem >= kMarchMinBytes && march_form(b, &m, &ok) != FLB_OK) return false;
+    const size_t bytes = size_t(19 * cells) * b->elem;
+    if (bytes >= kMarchMinBytes && march_form(b, &m, &ok) != FLB_OK) return false;
+    ok = ok && march_pays(m.dyn, b->elem, bytes, false);
     b->march = ok ? 1 : 0;
     if (!ok) return false;
   }

@@ -372,7 +372,9 @@ hipError_t launch_march(const KArgs& a, const MarchArgs& m, hipStream_t s) {
   switch (m.dyn) {
     case DYN_BGK: return march_dyn<S, DYN_BGK>(a, m, s);
     case DYN_BGK_FORCE: return march_dyn<S, DYN_BGK_FORCE>(a, m, s);
-    case DYN_SMAG_MRT: return march_dyn<S, DYN_SMAG_MRT>(a, m, s);
+    case DYN_SMAG_MRT:
+      if constexpr (sizeof(typename S::E) == 8) return march_dyn<S, DYN_SMAG_MRT>(a, m, s);
+      else return hipErrorInvalidValue;  // single steps (march_pays)
     default: return hipErrorInvalidValue;
   }
 }
