@@ -29,7 +29,7 @@ HWBC_NORMAL, HWBC_MOVING, HWBC_ANTI = 0, 1, 2
 EXPORTS = (
     "flb_last_error", "flb_abi_version", "flb_block_layout", "flb_block_create", "flb_block_destroy", "flb_get_info",
     "flb_synchronize", "flb_set_tasks", "flb_set_halfway_bc", "flb_set_mrt_rates", "flb_set_omega",
-    "flb_set_force", "flb_share_velocity", "flb_add_buoyancy", "flb_clear_buoyancy",
+    "flb_set_force", "flb_share_velocity", "flb_add_buoyancy", "flb_clear_buoyancy", "flb_step_coupled",
     "flb_upload_flags", "flb_set_field_rho", "flb_set_field_u", "flb_upload_pops_f32",
     "flb_upload_pops_f64", "flb_download_pops_f32", "flb_download_pops_f64", "flb_init_equilibrium",
     "flb_apply_cell_dynamics", "flb_stream", "flb_set_level", "flb_set_watchdog", "flb_apply_halfway_bc", "flb_step", "flb_moments",
@@ -125,6 +125,7 @@ def lib() -> C.CDLL:
         "flb_share_velocity": [P, P],
         "flb_add_buoyancy": [P, P, C.c_uint8, C.c_double, C.c_double],
         "flb_clear_buoyancy": [P],
+        "flb_step_coupled": [P, P, C.c_int],
         "flb_upload_flags": [P, C.POINTER(C.c_uint8)],
         "flb_set_field_rho": [P, C.POINTER(C.c_double)],
         "flb_set_field_u": [P, C.POINTER(C.c_double)],

@@ -1008,6 +1008,45 @@ static int launch_one(flb_block b) {
   return FLB_OK;
 }
 
+// Whether the two blocks may step in one launch: one stream, the same cells
+// in the same slots, the same storage, parity and step, nothing pending.
+static bool pair_steps(const flb_block_s* f, const flb_block_s* c) {
+  const flb_block_desc &a = f->desc, &d = c->desc;
+  return f->device == c->device && f->stream == c->stream && a.nx == d.nx && a.ny == d.ny && a.nz == d.nz &&
+         a.overlap == d.overlap && f->pitch == c->pitch && f->stride == c->stride && a.storage == d.storage &&
+         (a.storage == FLB_STORE_F32 || a.storage == FLB_STORE_F64) && f->parity == c->parity && f->flags_set &&
+         c->flags_set && !f->pending && !c->pending && f->watchdog <= 0 && c->watchdog <= 0 && !a.periodic[0] &&
+         !a.periodic[1] && !a.periodic[2] && !d.periodic[0] && !d.periodic[1] && !d.periodic[2];
+}
+
+int flb_step_coupled(flb_block flow, flb_block scalar, int n) {
+  CHECK_BLOCK(flow);
+  CHECK_BLOCK(scalar);
+  if (n < 0) return fail(FLB_ERR_ARG, "negative step count");
+  int done = 0, rc = FLB_OK;
+  if (pair_steps(flow, scalar)) {
+    DeviceGuard g(flow->device);
+    Range range("flb_step_coupled");
+    if ((rc = ensure_links(flow)) || (rc = ensure_links(scalar))) return rc;
+    const KArgs f = make_args(flow), c = make_args(scalar);
+    for (; done < n; ++done) {
+      const hipError_t e =
+          flow->desc.storage == FLB_STORE_F64
+              ? flb::launch_coupled_f64(flow->desc.q, scalar->desc.q, flow->parity, f, c, flow->stream)
+              : flb::launch_coupled_f32(flow->desc.q, scalar->desc.q, flow->parity, f, c, flow->stream);
+      if (e == hipErrorNotSupported) break;
+      HIP_TRY(e);
+      for (flb_block b : {flow, scalar}) {
+        b->parity ^= 1;
+        b->step += 1;
+      }
+    }
+  }
+  for (; done < n; ++done)
+    if ((rc = flb_step(flow, 1)) || (rc = flb_step(scalar, 1))) return rc;
+  return FLB_OK;
+}
+
 int flb_set_level(flb_block b, int level, int max_level) {
   CHECK_BLOCK(b);
   if (level < 0 || max_level < level || max_level > 30)

@@ -136,6 +136,8 @@ constexpr int march_threads(size_t elem) { return elem == 8 ? 512 : 1024; }
 #define FLB_DECLARE_LAUNCHERS(SUFFIX)                                                         \
   hipError_t launch_step_##SUFFIX(int q, int parity, int family, const KArgs& a,             \
                                   hipStream_t s);                                           \
+  hipError_t launch_coupled_##SUFFIX(int qf, int qs, int parity, const KArgs& f,             \
+                                     const KArgs& c, hipStream_t s);                        \
   hipError_t launch_gather_##SUFFIX(int q, int parity, const KArgs& a, void* out,            \
                                     hipStream_t s);                                         \
   hipError_t launch_scatter_##SUFFIX(int q, const KArgs& a, const void* in, hipStream_t s);  \

@@ -304,9 +304,7 @@ class BlockLatManagerCoupling:
 
     def step(self, n: int = 1) -> None:
         """n iterations of the coupled loop: the flow step, then the scalar step."""
-        for _ in range(int(n)):
-            self.flow.step(1)
-            self.scalar.step(1)
+        abi.check(abi.lib().flb_step_coupled(self.flow.handle, self.scalar.handle, max(0, int(n))))
 
 
 class BlockHalo:

@@ -213,6 +213,10 @@ int flb_share_velocity(flb_block scalar, flb_block flow);
  * the order added. */
 int flb_add_buoyancy(flb_block flow, flb_block scalar, uint8_t mask, double gbeta, double rho_init);
 int flb_clear_buoyancy(flb_block flow);
+/* n iterations of the coupled loop: flb_step(flow, 1), flb_step(scalar, 1),
+ * with the same results; pairs over the same cells of one storage kind take
+ * one launch for both. */
+int flb_step_coupled(flb_block flow, flb_block scalar, int n);
 /* MRT relaxation rates, q values; NaN marks the shear-viscosity rates that
  * take omega. NULL restores the defaults. */
 int flb_set_mrt_rates(flb_block b, const double* rates, int q);

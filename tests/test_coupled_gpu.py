@@ -261,3 +261,36 @@ def test_coupling_rejects_blocks_on_different_streams():
             b.close()
         hip.hipStreamDestroy(s1)
         hip.hipStreamDestroy(s2)
+
+
+@pytest.mark.parametrize("n,d,storage", [(5, 3, "f32"), (23, 3, "f64"), (64, 3, "f32"), (66, 3, "f32"),
+                                         (40, 2, "f32"), (250, 2, "f64")])
+def test_one_launch_for_both_blocks_equals_two(n, d, storage):
+    """The coupled loop in one launch per step against the two blocks' own steps, bit for bit: short
+    and long rows, both parities, and from blocks at different parities (two launches)."""
+    from freelb_amd.cases import heated_cavity
+    a, b = [heated_cavity(n, d, storage, tau_flow=0.6, gbeta=1e-3) for _ in range(2)]
+    try:
+        for flow, temp, _ in (a, b):
+            u = np.random.default_rng(2).uniform(-0.02, 0.02, size=(d, flow.N))
+            flow.init_equilibrium(np.ones(flow.N), u)
+        for k in (1, 2, 5):
+            a[2].step(k)
+            for _ in range(k):
+                b[0].step(1)
+                b[1].step(1)
+            for x, y in zip(a[:2], b[:2]):
+                assert np.array_equal(x.pops(), y.pops()), k
+                assert np.array_equal(x.download_fields(), y.download_fields()), k
+        for flow, temp, _ in (a, b):
+            flow.step(1)
+        a[2].step(3)
+        for _ in range(3):
+            b[0].step(1)
+            b[1].step(1)
+        for x, y in zip(a[:2], b[:2]):
+            assert np.array_equal(x.pops(), y.pops())
+    finally:
+        for flow, temp, _ in (a, b):
+            flow.close()
+            temp.close()
