@@ -3,10 +3,11 @@
 
 Workload: the 256^3 lid-driven cavity (D3Q19, BGK, tau = 0.53, halfway
 bounce-back on five walls, moving lid u = 0.1), populations resident in HBM.
-One step = one fused collide-and-stream launch over the 256^3 fluid cells.
-`value` is MLUPS of FP32 storage; the same workload with FP16 / BF16 shifted
-storage is reported beside it, with each run's HBM roofline fraction
-(152 B per cell update in FP32, 76 B in the shifted half formats).
+One step = one fused collide-and-stream update of the 256^3 fluid cells; runs
+in FP32 take two steps per launch, every population read and written once for
+both. `value` is MLUPS of FP32 storage; the same workload with FP16 / BF16
+shifted storage is reported beside it, with each run's HBM roofline fraction
+(76 B per cell update in FP32 and in the shifted half formats).
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu]
 """
@@ -81,10 +82,11 @@ def time_storage(storage, steps, warmup, timer):
     mass = lat.mass_momentum()
     finite = bool(np.isfinite(mass).all())
     lat.close()
-    bytes_per = 152 if storage == "f32" else (76 if storage in ("f16s", "bf16s", "f16c") else 304)
+    # populations moved per cell and step: FP32 and FP64 runs take two steps per launch
+    bytes_per = 152 if storage == "f64" else 76
     ms_step = ms / steps
     mlups = n_active * steps / (ms / 1e3) / 1e6
-    achieved = n_active * bytes_per / (ms_step / 1e3) / 1e9  # GB/s, algorithmic bytes per launch
+    achieved = n_active * bytes_per / (ms_step / 1e3) / 1e9  # GB/s, algorithmic bytes per step
     return {"storage": storage, "ms_per_step": ms_step, "mlups": mlups, "wall_s": wall,
             "achieved_gbs": achieved, "frac": achieved / HBM_PEAK_GBS, "bytes_per_cell": bytes_per,
             "finite": finite}
@@ -154,7 +156,8 @@ def precision_study(n=N_EDGE, steps=2000, collisions=("bgk", "mrt_les"),
                 m = lat.moments()
             finally:
                 lat.close()
-            bpc = {"f64": 304, "f32": 152}.get(s, 76)
+            # two steps per launch in FP64 and in FP32 BGK
+            bpc = 152 if s == "f64" or (s == "f32" and coll != "bgk") else 76
             rec = {"mlups": round(n ** 3 * steps / dt / 1e6, 1),
                    "hbm_frac": round(n ** 3 * steps * bpc / dt / (HBM_PEAK_GBS * 1e9), 4),
                    "finite": bool(np.isfinite(m[:, live]).all())}
@@ -234,7 +237,7 @@ def batch_bench(timer, nblocks=512, seed=2025, graph_steps=500, storage="f32", l
     # blocks pairing tau near 0.51 with a lid near 0.1 are unstable under BGK
     # (the oracle diverges on them too); the rate counts every block's cells
     diverged = [k for k in range(nblocks) if not np.isfinite(mass[k])]
-    bytes_per = 152 if storage == "f32" else 76
+    bytes_per = 76  # FP32: two steps per launch
     how = f"{graph_steps} eager batch launches" if eager else f"hipGraph of {graph_steps} steps"
     return {"workload": f"{nblocks} cavities, edges U{{16..96}}^3 (seed {seed}), tau U[0.51,0.9], "
                         f"lid U[0.02,0.1], {how}",
@@ -248,20 +251,24 @@ def batch_bench(timer, nblocks=512, seed=2025, graph_steps=500, storage="f32", l
             "diverged_blocks": [(k, round(specs[k]["tau"], 4), round(specs[k]["u_lid"], 3)) for k in diverged]}
 
 
-# algorithmic HBM bytes per cell of the FP32 adjoint kernels, for boxes
+# algorithmic HBM bytes per cell of the FP32 adjoint passes, for boxes
 # without solid cells (their link words come from the cell's place; a box
-# with solid cells also reads a 4-byte link word per cell and kernel):
-# - forward push: reads and writes 19 populations, reads s (4 B);
-# - moment record (rho - 1, u) a recompute step, or a forward step with
-#   checkpoint_every 0, also writes: 16 B;
-# - moment record alone (the last state of each recomputed segment): reads
-#   19 populations and s, writes 16 B;
-# - adjoint step: reads the moment record and 19 adjoint values, writes 19
-#   adjoint values, reads s and updates dJ/ds (8 B).
+# with solid cells also reads a 4-byte link word per cell and pass). A pass
+# takes two steps where it can:
+# - forward: reads and writes 19 populations, reads s (4 B); each moment record
+#   (rho - 1, u) written with it is 16 B; a recomputed segment's last pass, or
+#   its last state alone, writes records only;
+# - adjoint: reads and writes 19 adjoint values, reads s and a record per step,
+#   updates dJ/ds (8 B).
 ADJ_FWD_BYTES = 19 * 4 * 2 + 4
 ADJ_MOM_BYTES = 4 * 4
-ADJ_MOMONLY_BYTES = 19 * 4 + 4 + 4 * 4
-ADJ_BWD_BYTES = 4 * 4 + 19 * 4 * 2 + 4 + 8
+ADJ_READ_BYTES = 19 * 4 + 4
+ADJ_BWD_BYTES = 19 * 4 * 2 + 4 + 8
+
+
+def _passes(steps):
+    """Passes of `steps` steps, two at a time."""
+    return (steps + 1) // 2
 
 
 def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms):
@@ -269,10 +276,13 @@ def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms):
     (T adjoint steps plus the T - ceil(T/K) recomputed forward steps and the
     ceil(T/K) moment records of segment ends) and of the whole gradient, with
     the bandwidth each pass reaches."""
-    nseg = -(-T // K) if K > 0 else 0
-    rec = T - nseg if K > 0 else 0
-    fwd_b = cells * T * (ADJ_FWD_BYTES + (ADJ_MOM_BYTES if K == 0 else 0))
-    bwd_b = cells * (T * ADJ_BWD_BYTES + rec * (ADJ_FWD_BYTES + ADJ_MOM_BYTES) + nseg * ADJ_MOMONLY_BYTES)
+    segs = [min(K, T - t) for t in range(0, T, K)] if K > 0 else [T]
+    rec = T - len(segs) if K > 0 else 0
+    fwd_b = cells * (sum(map(_passes, segs)) * ADJ_FWD_BYTES + (T * ADJ_MOM_BYTES if K == 0 else 0))
+    bwd_b = cells * (sum(map(_passes, segs)) * ADJ_BWD_BYTES + T * ADJ_MOM_BYTES)
+    if K > 0:
+        bwd_b += cells * (sum(_passes(n) - 1 for n in segs) * ADJ_FWD_BYTES + len(segs) * ADJ_READ_BYTES +
+                          T * ADJ_MOM_BYTES)
     return {"forward_mlups": round(cells * T / fwd_ms / 1e3, 1),
             "adjoint_mlups": round(cells * T / bwd_ms / 1e3, 1),
             "gradient_mlups": round(cells * T / (fwd_ms + bwd_ms) / 1e3, 1),
@@ -418,15 +428,15 @@ def coupled_bench(timer, n=256, steps=100, warmup=4):
 
 
 def profiled_traffic(storage):
-    """HBM bytes per launch of the step kernel for this workload, from the
-    committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary (counters scaled by a
-    copy kernel of known size in the same runs). None when absent."""
-    path = os.path.join(ROOT, "profiles", "k_step_cell_d3q19_cavity256.md")
+    """HBM bytes per step of this workload, from the committed rocprofv3
+    FETCH_SIZE / WRITE_SIZE summary (counters scaled by a copy kernel of known
+    size in the same runs). None when absent."""
+    path = os.path.join(ROOT, "profiles", "k_step_march_cavity256.md")
     try:
         text = open(path).read()
     except OSError:
         return None
-    m = re.search(rf"^traffic_bytes_per_launch {storage} = (\d+)", text, re.M)
+    m = re.search(rf"^traffic_bytes_per_step {storage} = (\d+)", text, re.M)
     return int(m.group(1)) if m else None
 
 

@@ -17,8 +17,8 @@
 //
 // The one-step kernels are bound by HBM (152 bytes per cell and step in FP32,
 // at 88 % of the copy rate on the 256^3 cavity), so the bytes are what can be
-// saved: two steps here read 1.41 GB there and write 1.29 GB, against
-// 2 x 2.58 GB. Measured per step, FP32 BGK cavities: 256^3 0.444 -> 0.291 ms
+// saved: two steps here read 1.45 GB there and write 1.28 GB, against
+// 2 x 2.59 GB. Measured per step, FP32 BGK cavities: 256^3 0.444 -> 0.291 ms
 // (57.6 GLUPS), 192^3 222 -> 142 us, 100^3 27.1 -> 21.5 us; FP64 256x200x160
 // 436 -> 292 us. What bounds it now is the walk of one workgroup of 16
 // wavefronts per CU (LDS holds no second one): matrix-free VALU work half the
