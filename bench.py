@@ -251,24 +251,22 @@ def batch_bench(timer, nblocks=512, seed=2025, graph_steps=500, storage="f32", l
             "diverged_blocks": [(k, round(specs[k]["tau"], 4), round(specs[k]["u_lid"], 3)) for k in diverged]}
 
 
-# algorithmic HBM bytes per cell of the FP32 adjoint passes, for boxes
-# without solid cells (their link words come from the cell's place; a box
-# with solid cells also reads a 4-byte link word per cell and pass). A pass
-# takes two steps where it can:
-# - forward: reads and writes 19 populations, reads s (4 B); each moment record
-#   (rho - 1, u) written with it is 16 B; a recomputed segment's last pass, or
-#   its last state alone, writes records only;
-# - adjoint: reads and writes 19 adjoint values, reads s and a record per step,
-#   updates dJ/ds (8 B).
+# algorithmic HBM bytes per cell of the FP32 adjoint's single steps (larger
+# boxes take two steps per launch, which move about half as much: the rates are
+# then what single steps would need), for boxes without solid cells (their link
+# words come from the cell's place; a box with solid cells also reads a 4-byte
+# link word per cell and kernel):
+# - forward push: reads and writes 19 populations, reads s (4 B);
+# - moment record (rho - 1, u) a recompute step, or a forward step with
+#   checkpoint_every 0, also writes: 16 B;
+# - moment record alone (the last state of each recomputed segment): reads
+#   19 populations and s, writes 16 B;
+# - adjoint step: reads the moment record and 19 adjoint values, writes 19
+#   adjoint values, reads s and updates dJ/ds (8 B).
 ADJ_FWD_BYTES = 19 * 4 * 2 + 4
 ADJ_MOM_BYTES = 4 * 4
-ADJ_READ_BYTES = 19 * 4 + 4
-ADJ_BWD_BYTES = 19 * 4 * 2 + 4 + 8
-
-
-def _passes(steps):
-    """Passes of `steps` steps, two at a time."""
-    return (steps + 1) // 2
+ADJ_MOMONLY_BYTES = 19 * 4 + 4 + 4 * 4
+ADJ_BWD_BYTES = 4 * 4 + 19 * 4 * 2 + 4 + 8
 
 
 def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms):
@@ -276,13 +274,10 @@ def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms):
     (T adjoint steps plus the T - ceil(T/K) recomputed forward steps and the
     ceil(T/K) moment records of segment ends) and of the whole gradient, with
     the bandwidth each pass reaches."""
-    segs = [min(K, T - t) for t in range(0, T, K)] if K > 0 else [T]
-    rec = T - len(segs) if K > 0 else 0
-    fwd_b = cells * (sum(map(_passes, segs)) * ADJ_FWD_BYTES + (T * ADJ_MOM_BYTES if K == 0 else 0))
-    bwd_b = cells * (sum(map(_passes, segs)) * ADJ_BWD_BYTES + T * ADJ_MOM_BYTES)
-    if K > 0:
-        bwd_b += cells * (sum(_passes(n) - 1 for n in segs) * ADJ_FWD_BYTES + len(segs) * ADJ_READ_BYTES +
-                          T * ADJ_MOM_BYTES)
+    nseg = -(-T // K) if K > 0 else 0
+    rec = T - nseg if K > 0 else 0
+    fwd_b = cells * T * (ADJ_FWD_BYTES + (ADJ_MOM_BYTES if K == 0 else 0))
+    bwd_b = cells * (T * ADJ_BWD_BYTES + rec * (ADJ_FWD_BYTES + ADJ_MOM_BYTES) + nseg * ADJ_MOMONLY_BYTES)
     return {"forward_mlups": round(cells * T / fwd_ms / 1e3, 1),
             "adjoint_mlups": round(cells * T / bwd_ms / 1e3, 1),
             "gradient_mlups": round(cells * T / (fwd_ms + bwd_ms) / 1e3, 1),
