@@ -108,7 +108,7 @@ class Adjoint:
 
 class AdjointBatch:
     """Several Adjoint boxes (any sizes, one storage kind) stepped together,
-    one launch per time step over all of their cells. Each member keeps its
+    one launch per one or two time steps over all of their cells. Each member keeps its
     own fields; after forward() every member also holds its own objective,
     final state and recorded run."""
 

@@ -5,7 +5,9 @@
 // blocks stay ordinary flb_block objects (their own allocations, flags,
 // tasks, fields, read-out); the batch only replaces the per-block launch loop
 // of FreeLB's BlockLatticeManager::ApplyCellDynamics / CuDevApplyCellDynamics
-// (data_struct/block_lattice.hh:744-778, 919-936) with a single launch.
+// (data_struct/block_lattice.hh:744-778, 919-936) with a single launch. Runs
+// without an exchange between the steps take two steps per launch where that
+// pays (prepare_march).
 
 #include <hip/hip_runtime.h>
 

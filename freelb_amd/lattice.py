@@ -469,8 +469,8 @@ class RefinementManager:
 
 
 class BlockLatticeManager:
-    """Many BlockLattice blocks stepped together, one launch per time step
-    (FreeLB's BlockLatticeManager::ApplyCellDynamics / Stream over its blocks,
+    """Many BlockLattice blocks stepped together, one launch per one or two
+    time steps (FreeLB's BlockLatticeManager::ApplyCellDynamics / Stream over its blocks,
     data_struct/block_lattice.hh:744-778). The blocks keep their own set-up
     and read-out and must stay open while the manager lives."""
 

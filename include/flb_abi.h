@@ -312,7 +312,7 @@ int flb_reduce_mass_momentum_noalloc(flb_block b, uint8_t mask, double* d_out);
 
 /* ---- batches ----------------------------------------------------------------
  * Many blocks of one lattice and storage kind stepped by one launch per time
- * step: a device table of the blocks' kernel arguments, walked by a grid of
+ * step (or per two steps): a device table of the blocks' kernel arguments, walked by a grid of
  * workgroups that is either one workgroup per group of wavefronts or a
  * persistent grid; steps can be recorded once as a hipGraph and replayed.
  * Replaces the per-block launch loop of
@@ -463,7 +463,7 @@ int flb_adjoint_state(flb_adjoint h, double* pops);
 int flb_adjoint_timing(flb_adjoint h, double* forward_ms, double* backward_ms);
 
 /* Many boxes of any sizes stepped together: one launch per time step (and
- * per adjoint step) covers the cells of every member. Members keep their own
+ * per adjoint step), or per two, covers the cells of every member. Members keep their own
  * fields and buffers; all must use the same storage kind and device. After a
  * batch forward run each member holds its own result exactly as after
  * flb_adjoint_forward (its objective, final state and recorded run, so
