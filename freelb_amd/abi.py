@@ -25,6 +25,10 @@ STORAGE = {"f32": STORE_F32, "f16s": STORE_F16S, "bf16s": STORE_BF16S, "f64": ST
  DYN_SCALAR_BGK_FIELD) = range(13)
 HWBC_NORMAL, HWBC_MOVING, HWBC_ANTI = 0, 1, 2
 
+# Kinds counted by flb_block_paths / flb_adjoint_paths, in the header's order.
+BLOCK_PATHS = ("two_step", "coupled")
+ADJ_PATHS = ("forward_two", "backward_two")
+
 # Every symbol include/flb_abi.h declares (checked by the CPU test suite).
 EXPORTS = (
     "flb_last_error", "flb_abi_version", "flb_block_layout", "flb_block_create", "flb_block_destroy", "flb_get_info",
@@ -44,7 +48,7 @@ EXPORTS = (
     "flb_adjoint_init_equilibrium", "flb_adjoint_forward", "flb_adjoint_backward", "flb_adjoint_state",
     "flb_adjoint_timing", "flb_adjoint_batch_create", "flb_adjoint_batch_destroy", "flb_adjoint_batch_forward",
     "flb_adjoint_batch_backward", "flb_adjoint_batch_timing", "flb_bandwidth_probe",
-    "flb_bandwidth_probe_ex", "flb_reduce_mass_momentum_noalloc",
+    "flb_bandwidth_probe_ex", "flb_reduce_mass_momentum_noalloc", "flb_block_paths", "flb_adjoint_paths",
 )
 
 
@@ -188,6 +192,8 @@ def lib() -> C.CDLL:
         "flb_adjoint_batch_forward": [P, C.c_int, C.c_int, C.POINTER(C.c_double)],
         "flb_adjoint_batch_backward": [P, C.POINTER(C.c_double)],
         "flb_adjoint_batch_timing": [P, C.POINTER(C.c_double), C.POINTER(C.c_double)],
+        "flb_block_paths": [P, C.POINTER(C.c_int64), C.c_int],
+        "flb_adjoint_paths": [P, C.POINTER(C.c_int64), C.c_int],
         "flb_bandwidth_probe": [C.c_size_t, C.c_int, C.POINTER(C.c_double)],
         "flb_reduce_mass_momentum_noalloc": [P, C.c_uint8, C.c_void_p],
         "flb_bandwidth_probe_ex": [C.c_int, C.c_int, C.c_int, C.c_int, C.c_size_t, C.c_int,
@@ -208,3 +214,10 @@ def check(rc: int) -> None:
 
 def ptr(a: np.ndarray, T):
     return a.ctypes.data_as(C.POINTER(T))
+
+
+def paths(fn, handle, names) -> dict:
+    """The counts of flb_block_paths / flb_adjoint_paths by name."""
+    n = (C.c_int64 * len(names))()
+    check(fn(handle, n, len(names)))
+    return dict(zip(names, n))

@@ -105,6 +105,10 @@ class Adjoint:
         abi.check(abi.lib().flb_adjoint_timing(self._h, C.byref(f), C.byref(b)))
         return f.value, b.value
 
+    def paths(self) -> dict:
+        """Launches since creation that took two steps, forward and backward, in batches too."""
+        return abi.paths(abi.lib().flb_adjoint_paths, self._h, abi.ADJ_PATHS)
+
 
 class AdjointBatch:
     """Several Adjoint boxes (any sizes, one storage kind) stepped together,

@@ -165,6 +165,12 @@ uint32_t buffer_form_ok(const KArgs& a, int elem, int dims) {
   return span * uint64_t(elem) < (uint64_t(1) << 31) ? 1u : 0u;
 }
 
+int copy_paths(const int64_t* from, int have, int64_t* out, int n) {
+  if (n < 0 || n > have || (n > 0 && !out)) return fail(FLB_ERR_ARG, "path counts: %d outside [0, %d] or null output", n, have);
+  std::copy(from, from + n, out);
+  return FLB_OK;
+}
+
 KArgs make_args(const flb_block_s* b) {
   KArgs a{};
   a.pops = static_cast<char*>(b->d_pops) + flb::kFrontPad * b->elem;
@@ -651,6 +657,11 @@ int flb_get_info(flb_block b, flb_block_info* info) {
   return FLB_OK;
 }
 
+int flb_block_paths(flb_block b, int64_t* counts, int n) {
+  CHECK_BLOCK(b);
+  return copy_paths(b->paths, FLB_PATHS, counts, n);
+}
+
 int flb_synchronize(flb_block b) {
   CHECK_BLOCK(b);
   DeviceGuard g(b->device);
@@ -1039,6 +1050,7 @@ int flb_step_coupled(flb_block flow, flb_block scalar, int n) {
       for (flb_block b : {flow, scalar}) {
         b->parity ^= 1;
         b->step += 1;
+        b->paths[FLB_PATH_COUPLED] += 1;
       }
     }
   }
@@ -1117,7 +1129,7 @@ static int run_steps(flb_block b, int n) {
     int k = 1;
     if (march && b->parity == 1 && n >= 4) {
       k = n / 4 * 4;
-      rc = march_run(b, k);
+      if ((rc = march_run(b, k)) == FLB_OK) b->paths[FLB_PATH_TWO_STEP] += k / 2;
     } else {
       rc = launch_one(b);
     }

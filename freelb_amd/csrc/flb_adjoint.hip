@@ -1173,6 +1173,7 @@ struct flb_adjoint_s {
   float fwd_ms = 0.0f, bwd_ms = 0.0f;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   bool retained = false;  // holds the read-out buffers (readout_retain)
+  int64_t paths[FLB_ADJ_PATHS] = {};  // flb_adjoint_paths
 };
 
 namespace {
@@ -1375,8 +1376,11 @@ bool march_of(const flb_adjoint_s* h, bool bwd, flb::MarchArgs* m) {
   return true;
 }
 
+constexpr int path_of(bool bwd) { return bwd ? FLB_ADJ_PATH_BACKWARD_TWO : FLB_ADJ_PATH_FORWARD_TWO; }
+
 template <class R, bool BWD, bool MOM, bool STORE>
-hipError_t march_step(const flb_adjoint_s* h, const flb::MarchArgs& m, const A::MarchIo<R>& io) {
+hipError_t march_step(flb_adjoint_s* h, const flb::MarchArgs& m, const A::MarchIo<R>& io) {
+  h->paths[path_of(BWD)] += 1;
   const dim3 grid(unsigned(m.ntx) * unsigned(m.nty) * unsigned(m.nz)), block(unsigned(A::kMarchNt<R, BWD>));
   hipLaunchKernelGGL((A::k_march2<R, BWD, MOM, STORE>), grid, block, 0, h->stream, adj_args<R>(h), m, io);
   return hipGetLastError();
@@ -1384,7 +1388,7 @@ hipError_t march_step(const flb_adjoint_s* h, const flb::MarchArgs& m, const A::
 
 // States t and t + 1 from src to dst (state t + 2; null: only the records).
 template <class R, bool MOM, bool STORE>
-hipError_t fwd_two(const flb_adjoint_s* h, const flb::MarchArgs& m, const void* src, void* dst, void* mom0,
+hipError_t fwd_two(flb_adjoint_s* h, const flb::MarchArgs& m, const void* src, void* dst, void* mom0,
                    void* mom1, double* obj0, double* obj1) {
   A::MarchIo<R> io{};
   io.src = static_cast<const R*>(src);
@@ -1462,7 +1466,7 @@ hipError_t bwd_step(const flb_adjoint_s* h, const void* mom, const void* mu1, vo
 // The adjoint steps of states t1 - 1 down to t0, whose records are mom[0 ..];
 // mu in h->d_lam[cur].
 template <class R>
-hipError_t bwd_run(const flb_adjoint_s* h, const flb::MarchArgs* m, void* const* mom, int t0, int t1, int& cur) {
+hipError_t bwd_run(flb_adjoint_s* h, const flb::MarchArgs* m, void* const* mom, int t0, int t1, int& cur) {
   hipError_t e = hipSuccess;
   for (int t = t1 - 1; e == hipSuccess && t >= t0; cur ^= 1) {
     bool two = false;
@@ -1731,6 +1735,7 @@ int prepare_march(flb_adjoint_batch_s* b) {
 
 template <class R, bool BWD, bool MOM, bool STORE>
 hipError_t march_batch(const flb_adjoint_batch_s* b, const A::Pass& p) {
+  for (flb_adjoint_s* h : b->members) h->paths[path_of(BWD)] += 1;
   hipLaunchKernelGGL((A::k_march2_b<R, BWD, MOM, STORE>), dim3(b->nmwg[BWD]), dim3(unsigned(A::kMarchNt<R, BWD>)), 0,
                      b->stream, static_cast<const A::Entry<R>*>(b->d_tab), b->d_mt[BWD], b->d_mwg[BWD], p);
   return hipGetLastError();
@@ -2079,6 +2084,11 @@ int flb_adjoint_state(flb_adjoint h, double* pops) {
       p[c] = (!h->h_solid.empty() && h->h_solid[size_t(c)]) ? 0.0 : p[c] + w;
   }
   return FLB_OK;
+}
+
+int flb_adjoint_paths(flb_adjoint h, int64_t* counts, int n) {
+  CHECK_ADJ(h);
+  return copy_paths(h->paths, FLB_ADJ_PATHS, counts, n);
 }
 
 int flb_adjoint_timing(flb_adjoint h, double* forward_ms, double* backward_ms) {

@@ -297,10 +297,17 @@ int join_out(flb_batch_s* t) {
   return FLB_OK;
 }
 
-void advance(flb_batch_s* t, int n) {
+// Launches of two steps among n steps from `parity` (enqueue_steps).
+int two_steps(int parity, int n, bool march) {
+  const int single = parity == 1 ? 0 : 1;
+  return march ? std::max(0, n - single) / 4 * 2 : 0;
+}
+
+void advance(flb_batch_s* t, int n, int two) {
   for (flb_block_s* b : t->blocks) {
     b->parity ^= (n & 1);
     b->step += n;
+    b->paths[FLB_PATH_TWO_STEP] += two;
   }
 }
 
@@ -418,8 +425,9 @@ int flb_batch_step(flb_batch t, int n) {
   const bool run = n >= 5 - parity;  // long enough for a pass of two steps and one back
   if (run && (rc = prepare_march(t))) return rc;
   if ((rc = join_in(t))) return rc;
-  HIP_TRY(enqueue_steps(t, parity, n, run && t->march.state == 1, t->stream));
-  advance(t, n);
+  const bool march = run && t->march.state == 1;
+  HIP_TRY(enqueue_steps(t, parity, n, march, t->stream));
+  advance(t, n, two_steps(parity, n, march));
   return join_out(t);
 }
 
@@ -500,11 +508,10 @@ int flb_batch_replay(flb_batch t) {
   const bool passes = t->graph_march.state == 1;
   if (passes && (rc = prepare_march(t))) return rc;
   if ((rc = join_in(t))) return rc;
-  if (passes && !t->march.same_launch(t->graph_march))
-    HIP_TRY(enqueue_steps(t, parity, t->graph_steps, false, t->stream));
-  else
-    HIP_TRY(hipGraphLaunch(t->exec, t->stream));
-  advance(t, t->graph_steps);
+  const bool as_recorded = !passes || t->march.same_launch(t->graph_march);
+  if (as_recorded) HIP_TRY(hipGraphLaunch(t->exec, t->stream));
+  else HIP_TRY(enqueue_steps(t, parity, t->graph_steps, false, t->stream));
+  advance(t, t->graph_steps, two_steps(parity, t->graph_steps, passes && as_recorded));
   return join_out(t);
 }
 

@@ -56,6 +56,7 @@ struct flb_block_s {
   int march = -1;          // 1: the march may step the block, 0: not, -1: to be checked (flags, tasks or walls changed)
   int closed = -1;         // 1: no link of an updated cell leads to a cell that is not updated but wall links, 0, -1 likewise
   bool retained = false;   // holds the read-out buffers (readout_retain)
+  int64_t paths[FLB_PATHS] = {};  // flb_block_paths
   uint64_t version = 0;  // bumped by every change a batch table must see
   uint64_t* d_links = nullptr;  // precomputed halfway wall links (slot layout)
   bool links_dirty = true;      // flags or halfway managers changed since d_links was built
@@ -133,6 +134,8 @@ struct DeviceGuard {
 KArgs make_args(const flb_block_s* b);
 int axis_ext(const flb_block_s* b, int ax);
 uint32_t buffer_form_ok(const KArgs& a, int elem, int dims);
+// Copies the first n of `have` counts to out; FLB_ERR_ARG for a bad n or a null out.
+int copy_paths(const int64_t* from, int have, int64_t* out, int n);
 // True when a count-gated call acts on a block of `level` in a hierarchy whose
 // finest level is max_level (BlockLatticeManager's 2^(maxlevel - level) rule).
 inline bool level_due(int64_t count, int level, int max_level) {

@@ -114,6 +114,10 @@ class BlockLattice:
         abi.check(abi.lib().flb_get_info(self._h, C.byref(inf)))
         return inf
 
+    def paths(self) -> dict:
+        """Launches since creation that took two steps, or stepped a coupled block too."""
+        return abi.paths(abi.lib().flb_block_paths, self._h, abi.BLOCK_PATHS)
+
     def synchronize(self) -> None:
         abi.check(abi.lib().flb_synchronize(self._h))
 

@@ -478,6 +478,20 @@ int flb_adjoint_batch_backward(flb_adjoint_batch b, double* grad);
 int flb_adjoint_batch_timing(flb_adjoint_batch b, double* forward_ms, double* backward_ms);
 
 /* ---- diagnostics ------------------------------------------------------------ */
+/* How a block's or box's steps ran, counted since its creation, its steps in a
+ * batch included. counts[n] takes the first n of the kinds below. */
+enum {
+  FLB_PATH_TWO_STEP = 0,  /* launches that took two steps (flb_step, flb_batch_step, a replayed batch graph) */
+  FLB_PATH_COUPLED = 1,   /* launches shared with a coupled block (flb_step_coupled) */
+  FLB_PATHS = 2
+};
+int flb_block_paths(flb_block b, int64_t* counts, int n);
+enum {
+  FLB_ADJ_PATH_FORWARD_TWO = 0,   /* forward launches of two steps, those of recomputed segments included */
+  FLB_ADJ_PATH_BACKWARD_TWO = 1,  /* backward launches of two steps */
+  FLB_ADJ_PATHS = 2
+};
+int flb_adjoint_paths(flb_adjoint h, int64_t* counts, int n);
 /* Device copy bandwidth: a float4 copy kernel over `bytes` (rounded down to a
  * multiple of 16) between two fresh buffers, `reps` timed launches; *gbs gets
  * (read + written bytes) / mean launch time. No reference counterpart: it

@@ -1,0 +1,133 @@
+"""Which kernels served a run (flb_block_paths, flb_adjoint_paths): the boxes of the bit-for-bit
+tests of two-step launches do take them, and the ones meant to step singly do not. Moving a
+threshold past one of those boxes fails here, where it would otherwise compare single steps with
+single steps."""
+import numpy as np
+import pytest
+
+from freelb_amd import Adjoint, AdjointBatch, BlockLatticeManager, HalfwayBB, abi
+from freelb_amd.cases import VOID, cavity_block, heated_cavity
+from tests import test_adjoint_gpu as adjoint_tests
+from tests import test_march_gpu as march_tests
+
+pytestmark = pytest.mark.gpu
+
+
+def _params(test, names):
+    """The values of a test's parametrize mark over `names`."""
+    return next(m.args[1] for m in test.pytestmark if m.name == "parametrize" and m.args[0] == names)
+
+
+@pytest.mark.parametrize("storage,dims", _params(march_tests.test_runs_equal_single_steps, "storage,dims"))
+@pytest.mark.parametrize("periodic,dyn,obstacles",
+                         _params(march_tests.test_runs_equal_single_steps, "periodic,dyn,obstacles"))
+def test_boxes_of_the_run_tests_take_two_steps(storage, dims, periodic, dyn, obstacles):
+    with march_tests._box(dims, periodic, storage, dyn, obstacles) as lat:
+        for n, two in ((4, 0), (5, 2), (9, 4), (1, 0)):  # parities 0, 0, 1, 0
+            before = lat.paths()["two_step"]
+            lat.step(n)
+            assert lat.paths()["two_step"] - before == two, n
+        assert lat.paths()["coupled"] == 0
+
+
+@pytest.mark.parametrize("storage,dims,collision",
+                         _params(march_tests.test_moving_lid_runs_equal_single_steps, "storage,dims,collision"))
+def test_lid_boxes_take_the_meant_path(storage, dims, collision):
+    marches = storage != "f16s" and dims != (40, 40, 40) and (collision == "bgk" or storage == "f64")
+    with cavity_block(dims, storage=storage, collision=collision, tau=0.6) as lat:
+        lat.step(9)
+        assert lat.paths()["two_step"] == (4 if marches else 0)
+
+
+def test_open_walls_and_watchdog():
+    with cavity_block((92, 83, 77), tau=0.6) as lat:
+        lat.set_watchdog(7)
+        lat.step(14)  # 7 steps to each check: 1, 4 in two launches, 2; then 4 in two launches, 3
+        assert lat.paths()["two_step"] == 4
+        lat.set_halfway_bc([HalfwayBB(4, VOID)])
+        lat.step(9)
+        assert lat.paths()["two_step"] == 4
+
+
+def test_batches_take_two_steps():
+    blocks = [cavity_block(d, tau=0.7, u_lid=0.03, seed=k) for k, d in enumerate(march_tests.BATCH_DIMS)]
+
+    def two():
+        counts = {b.paths()["two_step"] for b in blocks}
+        assert len(counts) == 1
+        return counts.pop()
+    try:
+        with BlockLatticeManager(blocks) as m:
+            m.capture(10)
+            assert two() == 0
+            m.replay()
+            assert two() == 4
+            m.step(9)
+            assert two() == 8
+            m.step(1)
+            blocks[3].set_halfway_bc([HalfwayBB(4, VOID)])
+            m.replay()
+            assert two() == 8
+    finally:
+        for b in blocks:
+            b.close()
+
+
+ADJ = "storage,dims,per,solids"
+
+
+@pytest.mark.parametrize(ADJ, _params(adjoint_tests.test_two_steps_per_pass_equal_single_steps, ADJ))
+def test_adjoint_boxes_take_two_steps(storage, dims, per, solids):
+    with Adjoint(dims, omega=1.6, periodic=per, storage=storage) as adj:
+        N = int(np.prod(dims))
+        adj.init_equilibrium(np.ones(N), np.zeros((3, N)))
+        back = 0 if storage == "f64" else 1
+        for T, K, f, b in ((7, 1, 0, 0), (7, 0, 3, 3), (7, 3, 2 + 2, 2), (8, 4, 4 + 4, 4)):
+            was = adj.paths()
+            adj.forward(T, K)
+            adj.backward()
+            now = adj.paths()
+            assert now["forward_two"] - was["forward_two"] == f, (T, K)
+            assert now["backward_two"] - was["backward_two"] == b * back, (T, K)
+
+
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+def test_adjoint_batch_takes_two_steps(storage):
+    members = []
+    try:
+        for dims in ((131, 60, 60), (75, 66, 101), (64, 96, 80), (200, 130, 32), (10, 6, 5), (96, 93, 97), (90, 80, 70)):
+            members.append(Adjoint(dims, omega=1.6, periodic=(True, False, False), storage=storage))
+            N = int(np.prod(dims))
+            members[-1].init_equilibrium(np.ones(N), np.zeros((3, N)))
+        with AdjointBatch(members) as b:
+            b.forward(9, 0)
+            b.backward()
+            assert all(a.paths() == dict(members[0].paths(), forward_two=4, backward_two=0 if storage == "f64" else 4)
+                       for a in members)
+            was = members[0].paths()
+            b.forward(9, 1)
+            b.backward()
+            assert all(a.paths()[k] == was[k] for a in members for k in ("forward_two", "backward_two"))
+    finally:
+        for a in members:
+            a.close()
+
+
+@pytest.mark.parametrize("n,d,storage", [(5, 3, "f32"), (23, 3, "f64"), (64, 3, "f32"), (40, 2, "f32"), (250, 2, "f64")])
+def test_coupled_pairs_take_one_launch(n, d, storage):
+    flow, temp, cpl = heated_cavity(n, d, storage)
+    try:
+        cpl.step(5)
+        assert flow.paths() == temp.paths() == dict(two_step=0, coupled=5)
+        flow.step(1)
+        cpl.step(3)
+        assert flow.paths()["coupled"] == 5
+    finally:
+        flow.close()
+        temp.close()
+
+
+def test_bad_count_is_refused():
+    with cavity_block((8, 8, 8)) as lat:
+        with pytest.raises(abi.FLBError):
+            abi.paths(abi.lib().flb_block_paths, lat.handle, abi.BLOCK_PATHS + ("x",))
