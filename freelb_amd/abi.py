@@ -27,7 +27,7 @@ HWBC_NORMAL, HWBC_MOVING, HWBC_ANTI = 0, 1, 2
 
 # Kinds counted by flb_block_paths / flb_adjoint_paths, in the header's order.
 BLOCK_PATHS = ("two_step", "coupled")
-ADJ_PATHS = ("forward_two", "backward_two")
+ADJ_PATHS = ("forward_two", "backward_two", "backward_pull")
 
 # Every symbol include/flb_abi.h declares (checked by the CPU test suite).
 EXPORTS = (

@@ -532,12 +532,18 @@ __global__ __launch_bounds__(kThreads) void k_init(AdjArgs<R> a, const R* __rest
   for (int i = 0; i < Q; ++i) f[int64_t(i) * a.N + id] = sol ? R(0) : geq(i, rho - R(1), rho, u, usq);
 }
 
-// ---- adjoint seed: mu^{T-1} = P^T lambda^T, lambda^T = dJ/df^T ------------------
-template <class R>
+// ---- adjoint seed: lambda^T = dJ/df^T (PULL), or mu^{T-1} = P^T lambda^T ---------
+template <class R, bool PULL>
 __device__ __forceinline__ void seed_cell(const AdjArgs<R>& a, R* __restrict__ mu, int64_t id) {
   if (id >= a.N) return;
   const uint32_t lk = a.link[id];
   const int x = int(id % a.nx);
+  if constexpr (PULL) {
+    const bool on = !(lk & 1u) && x == a.outlet;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) mu[int64_t(i) * a.N + id] = on ? R(Lat<Q>::cx(i)) * a.invT : R(0);
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < Q; ++i) {
     const bool wall = i != 0 && ((lk >> i) & 1u);
@@ -548,12 +554,19 @@ __device__ __forceinline__ void seed_cell(const AdjArgs<R>& a, R* __restrict__ m
   }
 }
 
-template <class R>
+template <class R, bool PULL>
 __global__ __launch_bounds__(kThreads) void k_seed(AdjArgs<R> a, R* __restrict__ mu) {
-  seed_cell(a, mu, int64_t(blockIdx.x) * kThreads + threadIdx.x);
+  seed_cell<R, PULL>(a, mu, int64_t(blockIdx.x) * kThreads + threadIdx.x);
 }
 
-// ---- one backward step: mu^t, f^t -> mu^{t-1}, grad += ds -------------------------
+// ---- one backward step: mu^t, f^t -> lambda^t, grad += ds -------------------------
+// Of two forms, with the same arithmetic. PULL keeps lambda between the steps:
+// mu_i = lambda_i(x + c_i) is read from the neighbours and lambda^t stored at
+// the cell. The other keeps mu: it is read at the cell, and lambda^t pushed to
+// where it is mu^{t-1}, as the two-step passes do, between whose passes it
+// takes the odd steps. Runs without passes pull, which is faster: per step,
+// FP32 64^3 8.2 us against 9.0, 128x50x60 12.2 against 13.4, 2 channels of
+// 0.38 M cells 12.9 against 14.9, 4 of 1.2 M 42.4 against 44.7.
 // The weighted moments of mu are summed per weight class over opposite pairs
 // (M from the pair sums, V from the differences, T from the sums), and
 // lambda^t is formed pairwise: beside their own (1 - omega) mu terms,
@@ -562,10 +575,11 @@ __global__ __launch_bounds__(kThreads) void k_seed(AdjArgs<R> a, R* __restrict__
 // f^t enters only through rho and u, its moment record m (rho - 1, u), 16
 // bytes per cell in FP32 instead of the 76 of the populations.
 // obj: lambda^t has the objective's own terms (a cell of the outlet plane,
-// t >= 1). Returns the cell's part of the gradient; sink(i, lambda_i).
-template <class R, class Sink>
-__device__ __forceinline__ R adjoint_collide(const R (&mu)[Q], const R (&m)[4], R s, const AdjArgs<R>& a, bool obj,
-                                             Sink&& sink) {
+// t >= 1). grad takes the cell's part of the gradient as soon as it is formed,
+// then sink(i, lambda_i).
+template <class R, class Grad, class Sink>
+__device__ __forceinline__ void adjoint_collide(const R (&mu)[Q], const R (&m)[4], R s, const AdjArgs<R>& a, bool obj,
+                                                Grad&& grad, Sink&& sink) {
   const R rho = R(1) + m[0];
   const R u[3] = {m[1], m[2], m[3]};
   const R irD = inv_rho_d(rho, s, a);
@@ -622,7 +636,7 @@ __device__ __forceinline__ R adjoint_collide(const R (&mu)[Q], const R (&m)[4], 
   const R Auu = Au[0] * u[0] + Au[1] * u[1] + Au[2] * u[2];
   // 1 / D = rho / (rho D) and 1 / rho = D / (rho D)
   const R D = R(1) + as * R(0.5);
-  const R ds = -(R(0.5) * a.alpha * rho * irD) * Auu - fom * a.alpha * rho * Bu;
+  grad(-(R(0.5) * a.alpha * rho * irD) * Auu - fom * a.alpha * rho * Bu);
   const R base = Arho - Auu * (D * irD);
   // c_j.A_u / (rho D), with the objective's c_jx / T folded into the x part
   R Ar[3] = {Au[0] * irD, Au[1] * irD, Au[2] * irD};
@@ -636,47 +650,71 @@ __device__ __forceinline__ R adjoint_collide(const R (&mu)[Q], const R (&m)[4], 
     sink(i, om1 * mu[i] + (base + ca));
     sink(i + 1, om1 * mu[i + 1] + (base - ca));
   }
-  return ds;
 }
 
-template <class R>
+template <class R, bool PULL>
 __device__ __forceinline__ void bwd_cell(const AdjArgs<R>& a, const R* __restrict__ mom,
-                                         const R* __restrict__ mu1, R* __restrict__ mu0,
+                                         const R* __restrict__ from, R* __restrict__ to,
                                          R* __restrict__ grad, int with_obj, int64_t id) {
   if (id >= a.N) return;
+  // all loads are issued together with the link word, not after it (every
+  // offset is in bounds); a wall link then takes lambda_opp(i)(x) instead
   const Hops h = hops(a, uint32_t(id));
   R m[4], mu[Q];
 #pragma unroll
   for (int k = 0; k < 4; ++k) m[k] = ld_pop(mom, a.N, k, h.o);
+  auto load = [&] {
 #pragma unroll
-  for (int i = 0; i < Q; ++i) mu[i] = ld_pop(mu1, a.N, i, h.o);
+    for (int i = 0; i < Q; ++i) mu[i] = ld_pop(from, a.N, i, PULL ? hop(h, a, i) : h.o);
+  };
   const R s = ld_cell(a.s, h.o);
   const gptr<R> gr = cell_ref(grad, h.o);
-  const R g0 = *gr;
+  R g0 = R(0);
+  if constexpr (!PULL) g0 = *gr;
   uint32_t lk;
   if (a.solids) {
+    load();
     lk = ((gptr<const uint32_t>)a.link)[id];
     pin(m);
     pin(mu);
     asm volatile("" : "+v"(lk));  // tests of lk come after every load above
     if (lk & 1u) return;
   } else {
+    // wall links known from the place, not from memory: the bounce-back
+    // loads below go out in the same round as these
     lk = face_links(a, h);
+    load();
   }
   const bool obj = with_obj && h.x == uint32_t(a.outlet);
-  R ds;
-  if (__ballot(lk != 0u) == 0)
-    ds = adjoint_collide(mu, m, s, a, obj, [&](int i, R v) { push<R, false>(a, h, lk, mu0, i, opp(i), v); });
-  else
-    ds = adjoint_collide(mu, m, s, a, obj, [&](int i, R v) { push<R, true>(a, h, lk, mu0, i, opp(i), v); });
-  *gr = g0 + ds;
+  if constexpr (PULL) {
+    if (__ballot(lk != 0u) != 0) {
+#pragma unroll
+      for (int i = 1; i < Q; ++i)
+        if ((lk >> i) & 1u) mu[i] = ld_pop(from, a.N, opp(i), h.o);
+    }
+    // the cell's offset as a value of this block, so that the stores take it as
+    // their 32-bit lane offset (a value carried in from an earlier block reaches
+    // them widened to 64 bits, and each store then forms a 64-bit address)
+    uint32_t o = h.o;
+    asm volatile("" : "+v"(o));
+    adjoint_collide(mu, m, s, a, obj, [&](R ds) { *gr += ds; }, [&](int i, R v) { st_pop(to, a.N, i, o, v); });
+  } else {
+    R ds;
+    const auto part = [&](R v) { ds = v; };
+    if (__ballot(lk != 0u) == 0)
+      adjoint_collide(mu, m, s, a, obj, part, [&](int i, R v) { push<R, false>(a, h, lk, to, i, opp(i), v); });
+    else
+      adjoint_collide(mu, m, s, a, obj, part, [&](int i, R v) { push<R, true>(a, h, lk, to, i, opp(i), v); });
+    *gr = g0 + ds;
+  }
 }
 
-template <class R>
+template <class R, bool PULL>
 __global__ __launch_bounds__(kThreads) void k_bwd(AdjArgs<R> a, const R* __restrict__ mom,
-                                                  const R* __restrict__ mu1, R* __restrict__ mu0,
+                                                  const R* __restrict__ from, R* __restrict__ to,
                                                   R* __restrict__ grad, int with_obj) {
-  bwd_cell(a, mom, mu1, mu0, grad, with_obj, int64_t(xcd_block(blockIdx.x, gridDim.x)) * kThreads + threadIdx.x);
+  bwd_cell<R, PULL>(a, mom, from, to, grad, with_obj,
+                    int64_t(xcd_block(blockIdx.x, gridDim.x)) * kThreads + threadIdx.x);
 }
 
 // ---- two steps per pass over memory ------------------------------------------------
@@ -856,7 +894,9 @@ __device__ __forceinline__ void march2(const AdjArgs<R>& a, const MarchArgs& m, 
   // one collision; sink(i, v) takes the values
   auto collide = [&](const R (&g)[Q], R s, const R (&mm)[BWD ? 4 : 1], bool obj, R* rec, auto&& sink) -> R {
     if constexpr (BWD) {
-      return adjoint_collide(g, mm, s, a, obj && out, sink);
+      R ds;
+      adjoint_collide(g, mm, s, a, obj && out, [&](R v) { ds = v; }, sink);
+      return ds;
     } else {
       R drho, rho, u[3], F[3], irD, v[Q];
       force_state(g, s, a, drho, rho, u, F, irD);
@@ -1086,13 +1126,13 @@ __global__ __launch_bounds__(kThreads) void k_obj_state_b(const Entry<R>* __rest
   obj_state(E.a, E.slots[src], E.shares + int64_t(obj) * E.a.ny * E.a.nz, blockIdx.x * kThreads + threadIdx.x);
 }
 
-template <class R>
+template <class R, bool PULL>
 __global__ __launch_bounds__(kThreads) void k_seed_b(const Entry<R>* __restrict__ tab, int n, int64_t total,
                                                      int mu) {
   const int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   if (k >= total) return;
   const Entry<R>& E = entry_of(tab, n, blockIdx.x);
-  seed_cell(E.a, E.slots[mu], k - E.cell0);
+  seed_cell<R, PULL>(E.a, E.slots[mu], k - E.cell0);
 }
 
 template <class R>
@@ -1104,14 +1144,14 @@ __global__ __launch_bounds__(kThreads) void k_mom_b(const Entry<R>* __restrict__
   mom_cell(E.a, slot(E, src), slot(E, mom), k0 - E.cell0 + threadIdx.x);
 }
 
-template <class R>
+template <class R, bool PULL>
 __global__ __launch_bounds__(kThreads) void k_bwd_b(const Entry<R>* __restrict__ tab, int n, int64_t total,
                                                     int mom, int lam1, int lam0, int with_obj) {
   const unsigned g = xcd_block(blockIdx.x, gridDim.x);
   const int64_t k0 = int64_t(g) * kThreads;
   if (k0 >= total) return;
   const Entry<R>& E = entry_of(tab, n, g);
-  bwd_cell(E.a, slot(E, mom), slot(E, lam1), slot(E, lam0), E.grad, with_obj, k0 - E.cell0 + threadIdx.x);
+  bwd_cell<R, PULL>(E.a, slot(E, mom), slot(E, lam1), slot(E, lam0), E.grad, with_obj, k0 - E.cell0 + threadIdx.x);
 }
 
 // Two steps of every box: mt and wgs as for the lattices' batches (tiles of
@@ -1162,7 +1202,7 @@ struct flb_adjoint_s {
   void* d_s = nullptr;
   void* d_f0 = nullptr;
   void* d_work[2] = {nullptr, nullptr};
-  void* d_lam[2] = {nullptr, nullptr};  // mu, ping-pong
+  void* d_lam[2] = {nullptr, nullptr};  // lambda or mu (A::bwd_cell), ping-pong
   void* d_grad = nullptr;
   double* d_jt = nullptr;
   int jt_cap = 0;
@@ -1462,17 +1502,26 @@ int forward_impl(flb_adjoint_s* h, int T, int K, double* J) {
   return FLB_OK;
 }
 
-// One adjoint step; mom: the moment record of state t.
+// Whether some adjoint steps of a run of T states, in segments of K (0: one),
+// can be taken two at a time: K and T leave more than one state to a segment.
+bool pairs(int T, int K) { return T > 1 && K != 1; }
+
+// One adjoint step (pull: the form of A::bwd_cell); mom: the moment record of state t.
 template <class R>
-hipError_t bwd_step(const flb_adjoint_s* h, const void* mom, const void* mu1, void* mu0, int with_obj) {
-  hipLaunchKernelGGL(A::k_bwd<R>, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
-                     static_cast<const R*>(mom), static_cast<const R*>(mu1), static_cast<R*>(mu0),
-                     static_cast<R*>(h->d_grad), with_obj);
-  return hipGetLastError();
+hipError_t bwd_step(flb_adjoint_s* h, bool pull, const void* mom, const void* from, void* to, int with_obj) {
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
+                       static_cast<const R*>(mom), static_cast<const R*>(from), static_cast<R*>(to),
+                       static_cast<R*>(h->d_grad), with_obj);
+    return hipGetLastError();
+  };
+  if (!pull) return go(A::k_bwd<R, false>);
+  h->paths[FLB_ADJ_PATH_BACKWARD_PULL] += 1;
+  return go(A::k_bwd<R, true>);
 }
 
 // The adjoint steps of states t1 - 1 down to t0, whose records are mom[0 ..];
-// mu in h->d_lam[cur].
+// h->d_lam[cur] holds mu where m is set, else lambda.
 template <class R>
 hipError_t bwd_run(flb_adjoint_s* h, const flb::MarchArgs* m, void* const* mom, int t0, int t1, int& cur) {
   hipError_t e = hipSuccess;
@@ -1491,7 +1540,7 @@ hipError_t bwd_run(flb_adjoint_s* h, const flb::MarchArgs* m, void* const* mom, 
       if constexpr (sizeof(R) == 4) e = march_step<R, true, false, true>(h, *m, io);
       t -= 2;
     } else {
-      e = bwd_step<R>(h, mom[t - t0], h->d_lam[cur], h->d_lam[cur ^ 1], t >= 1);
+      e = bwd_step<R>(h, m == nullptr, mom[t - t0], h->d_lam[cur], h->d_lam[cur ^ 1], t >= 1);
       t -= 1;
     }
   }
@@ -1516,13 +1565,14 @@ int backward_impl(flb_adjoint_s* h, double* grad) {
   if (rc) return rc;
   HIP_TRY(hipEventRecord(h->e0, h->stream));
   HIP_TRY(hipMemsetAsync(h->d_grad, 0, size_t(h->N) * h->real, h->stream));
-  hipLaunchKernelGGL(A::k_seed<R>, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
-                     static_cast<R*>(h->d_lam[0]));
-  HIP_TRY(hipGetLastError());
   flb::MarchArgs ftiles{}, btiles{};
   const bool march = march_of(h, false, &ftiles) && march_of(h, true, &btiles);
   const flb::MarchArgs* const fm = march ? &ftiles : nullptr;
-  const flb::MarchArgs* const m = march && sizeof(R) == 4 ? &btiles : nullptr;
+  const flb::MarchArgs* const m = march && sizeof(R) == 4 && pairs(T, K) ? &btiles : nullptr;
+  const auto seed = m ? A::k_seed<R, false> : A::k_seed<R, true>;
+  hipLaunchKernelGGL(seed, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
+                     static_cast<R*>(h->d_lam[0]));
+  HIP_TRY(hipGetLastError());
   int cur = 0;
   if (K == 0) {
     HIP_TRY(bwd_run<R>(h, m, h->mtape.data(), 0, T, cur));
@@ -1758,27 +1808,30 @@ hipError_t mom_batch(const flb_adjoint_batch_s* b, int src, int mom) {
 }
 
 template <class R>
-hipError_t bwd_batch(const flb_adjoint_batch_s* b, int mom, int lam1, int lam0, int with_obj) {
-  hipLaunchKernelGGL(A::k_bwd_b<R>, dim3(batch_grid(b)), dim3(A::kThreads), 0, b->stream,
+hipError_t bwd_batch(const flb_adjoint_batch_s* b, bool pull, int mom, int lam1, int lam0, int with_obj) {
+  const auto kernel = pull ? A::k_bwd_b<R, true> : A::k_bwd_b<R, false>;
+  hipLaunchKernelGGL(kernel, dim3(batch_grid(b)), dim3(A::kThreads), 0, b->stream,
                      static_cast<const A::Entry<R>*>(b->d_tab), int(b->members.size()), b->total, mom, lam1,
                      lam0, with_obj);
+  for (flb_adjoint_s* h : b->members) h->paths[FLB_ADJ_PATH_BACKWARD_PULL] += pull;
   return hipGetLastError();
 }
 
-// As bwd_run: the records of states t0 .. t1 - 1 in slots mom0 ...
+// As bwd_run: the records of states t0 .. t1 - 1 in slots mom0 ...; march: steps
+// are taken two at a time where a segment leaves two.
 template <class R>
-hipError_t bwd_run_batch(const flb_adjoint_batch_s* b, int mom0, int t0, int t1, int& cur) {
+hipError_t bwd_run_batch(const flb_adjoint_batch_s* b, bool march, int mom0, int t0, int t1, int& cur) {
   hipError_t e = hipSuccess;
   for (int t = t1 - 1; e == hipSuccess && t >= t0; cur ^= 1) {
     const int mom = mom0 + t - t0;
     bool two = false;
     if constexpr (sizeof(R) == 4) {
-      two = b->march == 1 && t - 1 >= t0;
+      two = march && t - 1 >= t0;
       if (two)
         e = march_batch<R, true, false, true>(
             b, {kSlotL0 + cur, kSlotL0 + (cur ^ 1), mom, mom - 1, -1, -1, t >= 1, t - 1 >= 1});
     }
-    if (!two) e = bwd_batch<R>(b, mom, kSlotL0 + cur, kSlotL0 + (cur ^ 1), t >= 1);
+    if (!two) e = bwd_batch<R>(b, !march, mom, kSlotL0 + cur, kSlotL0 + (cur ^ 1), t >= 1);
     t -= two ? 2 : 1;
   }
   return e;
@@ -1866,13 +1919,15 @@ int batch_backward_impl(flb_adjoint_batch_s* b, double* grad) {
   HIP_TRY(hipEventRecord(b->e0, b->stream));
   for (flb_adjoint_s* h : b->members)
     HIP_TRY(hipMemsetAsync(h->d_grad, 0, size_t(h->N) * h->real, b->stream));
-  hipLaunchKernelGGL(A::k_seed_b<R>, dim3(batch_grid(b)), dim3(A::kThreads), 0, b->stream, tab, int(nm), b->total,
+  const bool march = b->march == 1 && sizeof(R) == 4 && pairs(T, K);
+  const auto seed = march ? A::k_seed_b<R, false> : A::k_seed_b<R, true>;
+  hipLaunchKernelGGL(seed, dim3(batch_grid(b)), dim3(A::kThreads), 0, b->stream, tab, int(nm), b->total,
                      int(kSlotL0));
   HIP_TRY(hipGetLastError());
   const int tb = tape_base(T, K);
   int cur = 0;
   if (K == 0) {
-    HIP_TRY(bwd_run_batch<R>(b, tb, 0, T, cur));
+    HIP_TRY(bwd_run_batch<R>(b, march, tb, 0, T, cur));
   } else {
     const int nseg = (T + K - 1) / K;
     for (int k = nseg - 1; k >= 0; --k) {
@@ -1897,7 +1952,7 @@ int batch_backward_impl(flb_adjoint_batch_s* b, double* grad) {
         src = dst;
         r ^= 1;
       }
-      HIP_TRY(bwd_run_batch<R>(b, tb, t0, t1, cur));
+      HIP_TRY(bwd_run_batch<R>(b, march, tb, t0, t1, cur));
     }
   }
   HIP_TRY(hipEventRecord(b->e1, b->stream));

@@ -489,7 +489,8 @@ int flb_block_paths(flb_block b, int64_t* counts, int n);
 enum {
   FLB_ADJ_PATH_FORWARD_TWO = 0,   /* forward launches of two steps, those of recomputed segments included */
   FLB_ADJ_PATH_BACKWARD_TWO = 1,  /* backward launches of two steps */
-  FLB_ADJ_PATHS = 2
+  FLB_ADJ_PATH_BACKWARD_PULL = 2, /* single backward steps of runs without launches of two */
+  FLB_ADJ_PATHS = 3
 };
 int flb_adjoint_paths(flb_adjoint h, int64_t* counts, int n);
 /* Device copy bandwidth: a float4 copy kernel over `bytes` (rounded down to a

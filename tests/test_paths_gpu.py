@@ -113,6 +113,31 @@ def test_adjoint_batch_takes_two_steps(storage):
             a.close()
 
 
+@pytest.mark.parametrize("storage,dims,T,K,pulls", [("f32", (33, 20, 17), 9, 0, 9), ("f32", (33, 20, 17), 9, 4, 9),
+                                                    ("f64", (96, 60, 60), 7, 0, 7), ("f64", (96, 60, 60), 7, 3, 7),
+                                                    ("f32", (131, 60, 60), 7, 1, 7), ("f32", (131, 60, 60), 1, 0, 1),
+                                                    ("f32", (131, 60, 60), 7, 0, 0), ("f32", (131, 60, 60), 7, 3, 0)])
+def test_single_backward_steps_pull(storage, dims, T, K, pulls):
+    """Backward runs without launches of two steps read their neighbours (the faster form of a
+    single step); odd steps between such launches push. Alone and in a batch of one."""
+    with Adjoint(dims, omega=1.6, periodic=(True, False, False), storage=storage) as adj:
+        N = int(np.prod(dims))
+        rng = np.random.default_rng(5)
+        adj.set_fraction(rng.uniform(0, 1, N))
+        adj.init_equilibrium(np.ones(N), rng.uniform(-0.01, 0.01, (3, N)))
+        J = adj.forward(T, K)
+        g = adj.backward()
+        assert adj.paths()["backward_pull"] == pulls
+        was = adj.paths()
+        with AdjointBatch([adj]) as b:
+            assert b.forward(T, K)[0] == J
+            assert np.array_equal(b.backward()[0], g)
+        now = adj.paths()
+        # the batch decides on launches of two by its own estimate
+        two = now["backward_two"] > was["backward_two"]
+        assert now["backward_pull"] - was["backward_pull"] == (0 if two else T)
+
+
 @pytest.mark.parametrize("n,d,storage", [(5, 3, "f32"), (23, 3, "f64"), (64, 3, "f32"), (40, 2, "f32"), (250, 2, "f64")])
 def test_coupled_pairs_take_one_launch(n, d, storage):
     flow, temp, cpl = heated_cavity(n, d, storage)
