@@ -247,7 +247,14 @@ bool march_ready(flb_block_s* b) {
     const int64_t cells = int64_t(axis_ext(b, 0)) * axis_ext(b, 1) * axis_ext(b, 2);
     const size_t bytes = size_t(19 * cells) * b->elem;
     if (bytes >= kMarchMinBytes && march_form(b, &m, &ok) != FLB_OK) return false;
-    ok = ok && march_pays(m.dyn, b->elem, bytes, false);
+    if (ok) {
+      const KArgs a = make_args(b);
+      int cus = 0;
+      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess) return false;
+      const flb::MarchArgs tiles =
+          march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem));
+      ok = march_pays(m.dyn, b->elem, bytes, false, {tiles.ntx > 1, a.pitch >= 256, a.px || a.py || a.pz});
+    }
     b->march = ok ? 1 : 0;
     if (!ok) return false;
   }

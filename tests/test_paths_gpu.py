@@ -39,6 +39,23 @@ def test_lid_boxes_take_the_meant_path(storage, dims, collision):
         assert lat.paths()["two_step"] == (4 if marches else 0)
 
 
+# around the sizes where one population array fits the memory-side cache and two do not
+@pytest.mark.parametrize("storage,dyn,dims,per,marches", [
+    ("f32", abi.DYN_BGK, (134, 130, 122), 0, True), ("f32", abi.DYN_BGK, (136, 136, 134), 0, False),
+    ("f32", abi.DYN_BGK, (148, 146, 141), 0, True), ("f32", abi.DYN_BGK, (97, 160, 160), 0, True),
+    ("f32", abi.DYN_BGK, (256, 97, 100), 0, True), ("f64", abi.DYN_BGK, (104, 100, 95), 0, True),
+    ("f64", abi.DYN_BGK, (110, 110, 105), 0, False), ("f64", abi.DYN_BGK, (117, 117, 115), 0, True),
+    ("f32", abi.DYN_BGK_FORCE, (97, 150, 125), 1, True), ("f32", abi.DYN_BGK_FORCE, (97, 160, 160), 1, False),
+    ("f32", abi.DYN_BGK_FORCE, (136, 150, 152), 1, True), ("f64", abi.DYN_BGK_FORCE, (97, 100, 90), 0, True),
+    ("f64", abi.DYN_BGK_FORCE, (110, 110, 105), 1, False), ("f64", abi.DYN_BGK_FORCE, (117, 118, 120), 1, True),
+    ("f64", abi.DYN_BGK_FORCE, (256, 70, 70), 1, False), ("f64", abi.DYN_BGK_FORCE, (256, 70, 70), 0, True),
+    ("f32", abi.DYN_BGK_FORCE, (256, 97, 100), 1, True)])
+def test_band_of_the_memory_side_cache_steps_singly(storage, dyn, dims, per, marches):
+    with march_tests._box(dims, (bool(per), False, False), storage, dyn, False) as lat:
+        lat.step(5)
+        assert lat.paths()["two_step"] == (2 if marches else 0)
+
+
 def test_open_walls_and_watchdog():
     with cavity_block((92, 83, 77), tau=0.6) as lat:
         lat.set_watchdog(7)
