@@ -1525,12 +1525,17 @@ hipError_t launch_coupled(int qf, int qs, int parity, const KArgs& f, const KArg
   if constexpr (kPlainStore<S>) {
     constexpr int kScalars = (1 << DYN_SCALAR_BGK) | (1 << DYN_SCALAR_BGK_FIELD);
     const bool per = f.px || f.py || f.pz;
-    // Around the 256 MB of the memory-side cache two sweeps keep more of their
-    // arrays in it than one sweep over both: 128^3 FP32 (260 MB of populations
-    // and fields) 109.9 us in two launches against 112.5, 136^3 (312 MB) 127
-    // against 133; 126^3 (248 MB) the same in both, 150^3 (418 MB) as above.
+    // Around the 256 MB of the memory-side cache two sweeps in 3D keep more of
+    // their arrays in it than one sweep over both. Cubes, two launches against
+    // one: FP32 128^3 (260 MB of populations and fields) 110.6 us against
+    // 112.4, 136^3 (312 MB) 127.1 against 134.7, 144^3 (370 MB) 159.6 against
+    // 163.3, 146^3 (386 MB) 170.2 against 171.1; FP64 108^3 (312 MB) 114.5
+    // against 121, 114^3 (367 MB) 148.4 against 151.1. The same in both, or one
+    // ahead, up to 126^3 (248 MB) and from 147^3 (394 MB) on, FP64 from 116^3
+    // (387 MB). In 2D one launch is faster throughout (2000^2 FP32, 304 MB, 90.9
+    // us against 99.4; 1400^2 FP64, 298 MB, 87.5 against 91.9).
     const int64_t bytes = int64_t(f.ex) * f.ey * f.ez * (qf + qs + 5) * int64_t(sizeof(typename S::E));
-    const bool edge = bytes > 240000000 && bytes < 360000000;
+    const bool edge = qf == 19 && bytes > 240000000 && bytes < 388000000;
     const bool ok = !per && !edge && f.buf && c.buf && f.dyns == (1 << DYN_BGK_SCALAR_FORCE) && c.dyns != 0 &&
                     (c.dyns & ~kScalars) == 0 && (f.vec == 0 || f.vec == -3) && f.vec == c.vec && f.wpb == c.wpb &&
                     f.nblocks == c.nblocks;

@@ -169,6 +169,19 @@ def test_coupled_pairs_take_one_launch(n, d, storage):
         temp.close()
 
 
+@pytest.mark.parametrize("n,d,storage,one", [(124, 3, "f32", True), (144, 3, "f32", False), (148, 3, "f32", True),
+                                             (114, 3, "f64", False), (117, 3, "f64", True), (1900, 2, "f32", True),
+                                             (1300, 2, "f64", True)])
+def test_coupled_pairs_around_the_cache_take_the_faster_way(n, d, storage, one):
+    flow, temp, cpl = heated_cavity(n, d, storage)
+    try:
+        cpl.step(2)
+        assert flow.paths()["coupled"] == (2 if one else 0)
+    finally:
+        flow.close()
+        temp.close()
+
+
 def test_bad_count_is_refused():
     with cavity_block((8, 8, 8)) as lat:
         with pytest.raises(abi.FLBError):
