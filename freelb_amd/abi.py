@@ -26,8 +26,8 @@ STORAGE = {"f32": STORE_F32, "f16s": STORE_F16S, "bf16s": STORE_BF16S, "f64": ST
 HWBC_NORMAL, HWBC_MOVING, HWBC_ANTI = 0, 1, 2
 
 # Kinds counted by flb_block_paths / flb_adjoint_paths, in the header's order.
-BLOCK_PATHS = ("two_step", "coupled")
-ADJ_PATHS = ("forward_two", "backward_two", "backward_pull")
+BLOCK_PATHS = ("two_step", "coupled", "plans")
+ADJ_PATHS = ("forward_two", "backward_two", "backward_pull", "plans")
 
 # Every symbol include/flb_abi.h declares (checked by the CPU test suite).
 EXPORTS = (

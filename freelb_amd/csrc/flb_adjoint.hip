@@ -1221,6 +1221,7 @@ struct flb_adjoint_s {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   bool retained = false;  // holds the read-out buffers (readout_retain)
   int64_t paths[FLB_ADJ_PATHS] = {};  // flb_adjoint_paths
+  flb::MarchArgs tiles[2] = {};       // of the two-step passes, forward and backward, planned once (ntx 0: not yet)
 };
 
 namespace {
@@ -1411,17 +1412,21 @@ int march_nt(size_t real, bool bwd) {
   return real == 8 ? A::kMarchNt<double, false> : (bwd ? A::kMarchNt<float, true> : A::kMarchNt<float, false>);
 }
 
-// Whether one box takes two steps per pass, and its tiles. Boxes of 32 MiB of
+// The tiles of a box that takes two steps per pass, else null. Boxes of 32 MiB of
 // populations and more (128x64x64 FP32, 40 MB: 14.7 -> 12.8 us forward, 17.2
 // -> 15.1 backward; smaller ones run out of the caches); the passes address a
 // state with 31-bit byte offsets.
 constexpr size_t kTwoStepBytes = size_t(32) << 20;
-bool march_of(const flb_adjoint_s* h, bool bwd, flb::MarchArgs* m) {
-  if (state_bytes(h) < kTwoStepBytes || state_bytes(h) >= (size_t(1) << 31)) return false;
-  int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) return false;
-  *m = march_plan({h->desc.nx, h->desc.ny, h->desc.nz, h->desc.nx}, int(h->real), cus, march_nt(h->real, bwd));
-  return true;
+const flb::MarchArgs* march_of(flb_adjoint_s* h, bool bwd) {
+  if (state_bytes(h) < kTwoStepBytes || state_bytes(h) >= (size_t(1) << 31)) return nullptr;
+  flb::MarchArgs& m = h->tiles[bwd];
+  if (m.ntx == 0) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) return nullptr;
+    m = march_plan({h->desc.nx, h->desc.ny, h->desc.nz, h->desc.nx}, int(h->real), cus, march_nt(h->real, bwd));
+    h->paths[FLB_ADJ_PATH_PLANS] += 1;
+  }
+  return &m;
 }
 
 constexpr int path_of(bool bwd) { return bwd ? FLB_ADJ_PATH_BACKWARD_TWO : FLB_ADJ_PATH_FORWARD_TWO; }
@@ -1453,12 +1458,11 @@ int forward_impl(flb_adjoint_s* h, int T, int K, double* J) {
   int rc = prepare_forward(h, T, K);
   if (rc) return rc;
   HIP_TRY(hipEventRecord(h->e0, h->stream));
-  flb::MarchArgs m{};
-  const bool march = march_of(h, false, &m);
+  const flb::MarchArgs* const m = march_of(h, false);
   const void* src = h->d_f0;
   int base = 1;  // state of the first shares kept
   for (int t = 0, n = 0; t < T; t += n) {
-    n = forward_span(T, K, t, march);
+    n = forward_span(T, K, t, m != nullptr);
     if (t + n - base > kObjStates) {
       HIP_TRY(obj_flush(h, base, t - base));
       base = t;
@@ -1468,9 +1472,9 @@ int forward_impl(flb_adjoint_s* h, int T, int K, double* J) {
     void* dst = forward_target(h, t + n, src);
     if (n == 2) {
       if (K == 0)
-        HIP_TRY((fwd_two<R, true, true>(h, m, src, dst, h->mtape[size_t(t)], h->mtape[size_t(t + 1)], obj0, obj1)));
+        HIP_TRY((fwd_two<R, true, true>(h, *m, src, dst, h->mtape[size_t(t)], h->mtape[size_t(t + 1)], obj0, obj1)));
       else
-        HIP_TRY((fwd_two<R, false, true>(h, m, src, dst, nullptr, nullptr, obj0, obj1)));
+        HIP_TRY((fwd_two<R, false, true>(h, *m, src, dst, nullptr, nullptr, obj0, obj1)));
     } else if (K == 0) {
       HIP_TRY((fwd_step<R, true>(h, src, dst, h->mtape[size_t(t)], obj0)));
     } else {
@@ -1565,10 +1569,8 @@ int backward_impl(flb_adjoint_s* h, double* grad) {
   if (rc) return rc;
   HIP_TRY(hipEventRecord(h->e0, h->stream));
   HIP_TRY(hipMemsetAsync(h->d_grad, 0, size_t(h->N) * h->real, h->stream));
-  flb::MarchArgs ftiles{}, btiles{};
-  const bool march = march_of(h, false, &ftiles) && march_of(h, true, &btiles);
-  const flb::MarchArgs* const fm = march ? &ftiles : nullptr;
-  const flb::MarchArgs* const m = march && sizeof(R) == 4 && pairs(T, K) ? &btiles : nullptr;
+  const flb::MarchArgs* const fm = march_of(h, false);
+  const flb::MarchArgs* const m = sizeof(R) == 4 && pairs(T, K) ? march_of(h, true) : nullptr;
   const auto seed = m ? A::k_seed<R, false> : A::k_seed<R, true>;
   hipLaunchKernelGGL(seed, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),
                      static_cast<R*>(h->d_lam[0]));

@@ -54,6 +54,7 @@ struct flb_block_s {
   int wpb = 4;   // wavefronts per workgroup
   void* d_alt = nullptr;   // second population array of the two-step march (flb_march.hip), scratch between calls
   int march = -1;          // 1: the march may step the block, 0: not, -1: to be checked (flags, tasks or walls changed)
+  flb::MarchArgs tiles{};  // its tiles, planned once (ntx 0: not yet)
   int closed = -1;         // 1: no link of an updated cell leads to a cell that is not updated but wall links, 0, -1 likewise
   bool retained = false;   // holds the read-out buffers (readout_retain)
   int64_t paths[FLB_PATHS] = {};  // flb_block_paths

@@ -26,12 +26,13 @@ double plane_time(int w, int h, int ntx, int elem) {
 // Calls f(w, h, ntx, nty) for the tile extents worth considering.
 template <class F>
 void each_tile(const MarchBox& a, int elem, int threads, F&& f) {
-  const int line = 128 / elem;
-  for (int n = 1; n <= a.ex; ++n) {
+  const int line = 128 / elem, least = a.pitch >= 256 ? line : 8;
+  for (int n = 1, last = 0; n <= a.ex && last != line; ++n) {
     int w = (a.ex + n - 1) / n;
     if (a.pitch >= 256) w = (w + line - 1) / line * line;
-    if (w + 2 > flb::kMarchMaxRow) continue;
-    if (w < 8 && n > 1) break;
+    if (w + 2 > flb::kMarchMaxRow || w == last) continue;
+    if (w < least && n > 1) break;
+    if (a.pitch >= 256) last = w;
     const int hmax = std::min(a.ey, threads / (w + 2) - 2), first = (a.ey + hmax - 1) / hmax;
     for (int nty = first; nty <= first + 1 && nty <= a.ey; ++nty) {
       const int h = (a.ey + nty - 1) / nty;
@@ -50,7 +51,9 @@ void each_tile(const MarchBox& a, int elem, int threads, F&& f) {
 // fitted to 25 blocks of 40^2 x 400 to 256^3 cells with 10 to 60 splits
 // each, where the split chosen takes 1.02 times the best one's time in the
 // mean (1.14 at worst). Rows of 256 slots and more start on line boundaries:
-// their tiles do too.
+// their tiles do too. Made once per block or box, as a run may be four steps:
+// in each run, and with every aligned width tried over and over, it cost 36 us
+// at 256^3 and 140 us at 1000x60x12 (1 us in the mean now).
 flb::MarchArgs march_plan(const MarchBox& a, int elem, int cus, int threads) {
   flb::MarchArgs best{};
   double best_cost = 1e300;
@@ -249,11 +252,13 @@ bool march_ready(flb_block_s* b) {
     if (bytes >= kMarchMinBytes && march_form(b, &m, &ok) != FLB_OK) return false;
     if (ok) {
       const KArgs a = make_args(b);
-      int cus = 0;
-      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess) return false;
-      const flb::MarchArgs tiles =
-          march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem));
-      ok = march_pays(m.dyn, b->elem, bytes, false, {tiles.ntx > 1, a.pitch >= 256, a.px || a.py || a.pz});
+      if (b->tiles.ntx == 0) {
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess) return false;
+        b->tiles = march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem));
+        b->paths[FLB_PATH_PLANS] += 1;
+      }
+      ok = march_pays(m.dyn, b->elem, bytes, false, {b->tiles.ntx > 1, a.pitch >= 256, a.px || a.py || a.pz});
     }
     b->march = ok ? 1 : 0;
     if (!ok) return false;
@@ -272,10 +277,8 @@ bool march_ready(flb_block_s* b) {
 }
 
 int march_run(flb_block_s* b, int n) {
-  int cus = 0;
-  HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
   KArgs a = make_args(b);
-  flb::MarchArgs m = march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem));
+  flb::MarchArgs m = b->tiles;
   one_dynamics(b, &m);
   char* const pops = static_cast<char*>(b->d_pops) + flb::kFrontPad * b->elem;
   char* const alt = static_cast<char*>(b->d_alt) + flb::kFrontPad * b->elem;

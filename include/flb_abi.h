@@ -483,14 +483,16 @@ int flb_adjoint_batch_timing(flb_adjoint_batch b, double* forward_ms, double* ba
 enum {
   FLB_PATH_TWO_STEP = 0,  /* launches that took two steps (flb_step, flb_batch_step, a replayed batch graph) */
   FLB_PATH_COUPLED = 1,   /* launches shared with a coupled block (flb_step_coupled) */
-  FLB_PATHS = 2
+  FLB_PATH_PLANS = 2,     /* tile plans made for launches of two steps */
+  FLB_PATHS = 3
 };
 int flb_block_paths(flb_block b, int64_t* counts, int n);
 enum {
   FLB_ADJ_PATH_FORWARD_TWO = 0,   /* forward launches of two steps, those of recomputed segments included */
   FLB_ADJ_PATH_BACKWARD_TWO = 1,  /* backward launches of two steps */
   FLB_ADJ_PATH_BACKWARD_PULL = 2, /* single backward steps of runs without launches of two */
-  FLB_ADJ_PATHS = 3
+  FLB_ADJ_PATH_PLANS = 3,         /* tile plans made for launches of two steps, one per direction */
+  FLB_ADJ_PATHS = 4
 };
 int flb_adjoint_paths(flb_adjoint h, int64_t* counts, int n);
 /* Device copy bandwidth: a float4 copy kernel over `bytes` (rounded down to a

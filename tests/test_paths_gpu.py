@@ -119,8 +119,8 @@ def test_adjoint_batch_takes_two_steps(storage):
         with AdjointBatch(members) as b:
             b.forward(9, 0)
             b.backward()
-            assert all(a.paths() == dict(members[0].paths(), forward_two=4, backward_two=0 if storage == "f64" else 4)
-                       for a in members)
+            two = (4, 0 if storage == "f64" else 4)
+            assert all((a.paths()["forward_two"], a.paths()["backward_two"]) == two for a in members)
             was = members[0].paths()
             b.forward(9, 1)
             b.backward()
@@ -160,7 +160,7 @@ def test_coupled_pairs_take_one_launch(n, d, storage):
     flow, temp, cpl = heated_cavity(n, d, storage)
     try:
         cpl.step(5)
-        assert flow.paths() == temp.paths() == dict(two_step=0, coupled=5)
+        assert flow.paths() == temp.paths() == dict(two_step=0, coupled=5, plans=0)
         flow.step(1)
         cpl.step(3)
         assert flow.paths()["coupled"] == 5
@@ -180,6 +180,23 @@ def test_coupled_pairs_around_the_cache_take_the_faster_way(n, d, storage, one):
     finally:
         flow.close()
         temp.close()
+
+
+def test_tiles_are_planned_once():
+    with cavity_block((300, 60, 40), tau=0.6) as lat:
+        for _ in range(3):
+            lat.step(9)
+        lat.set_omega(1.3)
+        lat.set_halfway_bc([HalfwayBB(4, VOID), HalfwayBB(8, VOID, True)])
+        lat.step(9)
+        assert lat.paths()["two_step"] == 16 and lat.paths()["plans"] == 1
+    for storage, plans in (("f32", 2), ("f64", 1)):  # FP64 goes back in single steps
+        with Adjoint((131, 60, 60), omega=1.6, storage=storage) as adj:
+            adj.init_equilibrium(np.ones(adj.N), np.zeros((3, adj.N)))
+            for K in (0, 3, 0):
+                adj.forward(7, K)
+                adj.backward()
+            assert adj.paths()["plans"] == plans
 
 
 def test_bad_count_is_refused():
