@@ -28,6 +28,7 @@ HWBC_NORMAL, HWBC_MOVING, HWBC_ANTI = 0, 1, 2
 # Kinds counted by flb_block_paths / flb_adjoint_paths, in the header's order.
 BLOCK_PATHS = ("two_step", "coupled", "plans")
 ADJ_PATHS = ("forward_two", "backward_two", "backward_pull", "plans")
+READ_PATHS = ("direct", "ring", "plain", "pinned")
 
 # Every symbol include/flb_abi.h declares (checked by the CPU test suite).
 EXPORTS = (
@@ -48,7 +49,7 @@ EXPORTS = (
     "flb_adjoint_init_equilibrium", "flb_adjoint_forward", "flb_adjoint_backward", "flb_adjoint_state",
     "flb_adjoint_timing", "flb_adjoint_batch_create", "flb_adjoint_batch_destroy", "flb_adjoint_batch_forward",
     "flb_adjoint_batch_backward", "flb_adjoint_batch_timing", "flb_bandwidth_probe",
-    "flb_bandwidth_probe_ex", "flb_reduce_mass_momentum_noalloc", "flb_block_paths", "flb_adjoint_paths",
+    "flb_bandwidth_probe_ex", "flb_reduce_mass_momentum_noalloc", "flb_block_paths", "flb_adjoint_paths", "flb_readout_paths",
 )
 
 
@@ -194,6 +195,7 @@ def lib() -> C.CDLL:
         "flb_adjoint_batch_timing": [P, C.POINTER(C.c_double), C.POINTER(C.c_double)],
         "flb_block_paths": [P, C.POINTER(C.c_int64), C.c_int],
         "flb_adjoint_paths": [P, C.POINTER(C.c_int64), C.c_int],
+        "flb_readout_paths": [C.POINTER(C.c_int64), C.c_int],
         "flb_bandwidth_probe": [C.c_size_t, C.c_int, C.POINTER(C.c_double)],
         "flb_reduce_mass_momentum_noalloc": [P, C.c_uint8, C.c_void_p],
         "flb_bandwidth_probe_ex": [C.c_int, C.c_int, C.c_int, C.c_int, C.c_size_t, C.c_int,
@@ -221,3 +223,10 @@ def paths(fn, handle, names) -> dict:
     n = (C.c_int64 * len(names))()
     check(fn(handle, n, len(names)))
     return dict(zip(names, n))
+
+
+def readout_paths() -> dict:
+    """The process's read-outs by the way they took, and the pinned bytes they hold (flb_readout_paths)."""
+    n = (C.c_int64 * len(READ_PATHS))()
+    check(lib().flb_readout_paths(n, len(READ_PATHS)))
+    return dict(zip(READ_PATHS, n))

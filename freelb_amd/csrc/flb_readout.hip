@@ -31,6 +31,8 @@ constexpr int kWorkers = 8;
 
 // The ring serves one read-out at a time (busy); it is made at the first large
 // read-out and given back when the last block or box of the process goes.
+// Small moments have a buffer of their own (DirectOut): in the ring, the first
+// of them pinned 32 MiB, and a large read-out beside it found the ring taken.
 // Never destroyed itself: blocks may outlive static objects.
 struct Ring {
   std::mutex busy;
@@ -39,10 +41,30 @@ struct Ring {
   char* buf = nullptr;
   hipEvent_t ev[kRing] = {};
   int device = -1;  // of the events
+  std::mutex direct_busy;
+  char* direct = nullptr;
+  bool second = false;  // small moments were read since the buffer was given back
+  std::atomic<int64_t> paths[FLB_READ_PATHS] = {};  // flb_readout_paths
 };
 Ring& ring() {
   static Ring* r = new Ring();
   return *r;
+}
+
+bool pin(Ring& r, char** p, size_t bytes) {
+  if (hipHostMalloc(reinterpret_cast<void**>(p), bytes, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+  }
+  r.paths[FLB_READ_PINNED] += int64_t(bytes);
+  return true;
+}
+void unpin(Ring& r, char** p, size_t bytes) {
+  if (!*p) return;
+  (void)hipHostFree(*p);
+  *p = nullptr;
+  r.paths[FLB_READ_PINNED] -= int64_t(bytes);
 }
 
 void drop(Ring& r) {
@@ -50,8 +72,7 @@ void drop(Ring& r) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
   }
-  if (r.buf) (void)hipHostFree(r.buf);
-  r.buf = nullptr;
+  unpin(r, &r.buf, kChunk * kRing);
   r.device = -1;
 }
 
@@ -61,11 +82,7 @@ bool ready(Ring& r) {
   if (hipGetDevice(&dev) != hipSuccess) return false;
   if (r.buf && r.device == dev) return true;
   drop(r);
-  if (hipHostMalloc(reinterpret_cast<void**>(&r.buf), kChunk * kRing, hipHostMallocPortable) != hipSuccess) {
-    (void)hipGetLastError();
-    r.buf = nullptr;
-    return false;
-  }
+  if (!pin(r, &r.buf, kChunk * kRing)) return false;
   for (hipEvent_t& e : r.ev)
     if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
       (void)hipGetLastError();
@@ -179,20 +196,30 @@ void readout_release() {
   if (--r.users > 0) return;
   std::lock_guard<std::mutex> b(r.busy);
   drop(r);
+  std::lock_guard<std::mutex> d(r.direct_busy);
+  unpin(r, &r.direct, kDirect);
+  r.second = false;
 }
 
 // A kernel's output of at most kDirect bytes may go straight into pinned
 // memory instead of a device buffer that is copied afterwards: one operation
-// less on the stream. Holds the ring while it lives; ptr is null where the
-// ring is taken.
+// less on the stream (a step of 16^3 cells and its moments 39 -> 28 us). Holds the
+// buffer while it lives; ptr is null where another thread holds it, and for
+// the first such read-out, as pinning costs 40 us: a program that makes, reads
+// once and closes a 16^3 block at a time takes 175 us with the copy, 222 without.
 DirectOut::DirectOut(size_t bytes) {
   Ring& r = ring();
-  if (bytes > kDirect || !r.busy.try_lock()) return;
-  if (ready(r)) ptr = r.buf;
-  else r.busy.unlock();
+  if (bytes > kDirect || !r.direct_busy.try_lock()) return;
+  if (r.direct || (r.second && pin(r, &r.direct, kDirect))) {
+    ptr = r.direct;
+    r.paths[FLB_READ_DIRECT] += 1;
+    return;
+  }
+  r.second = true;
+  r.direct_busy.unlock();
 }
 DirectOut::~DirectOut() {
-  if (ptr) ring().busy.unlock();
+  if (ptr) ring().direct_busy.unlock();
 }
 
 // Workers pay from two chunks on; a second read-out at the same time takes the
@@ -200,10 +227,13 @@ DirectOut::~DirectOut() {
 hipError_t readout(void* host, const void* dev, size_t bytes, bool widen, hipStream_t s) {
   char* const h = static_cast<char*>(host);
   const char* const d = static_cast<const char*>(dev);
-  if (bytes < 2 * kChunk) return plain(h, d, bytes, widen, s);
   Ring& r = ring();
-  std::unique_lock<std::mutex> busy(r.busy, std::try_to_lock);
-  if (!busy.owns_lock() || !ready(r)) return plain(h, d, bytes, widen, s);
+  std::unique_lock<std::mutex> busy(r.busy, std::defer_lock);
+  if (bytes < 2 * kChunk || !busy.try_lock() || !ready(r)) {
+    r.paths[FLB_READ_PLAIN] += 1;
+    return plain(h, d, bytes, widen, s);
+  }
+  r.paths[FLB_READ_RING] += 1;
   Job job{r, h, d, bytes, widen, s, r.device, {}, {}, 0, {}, hipSuccess};
   job.emptied.assign(job.chunks(), 0);
   const size_t n = std::min<size_t>(kWorkers, job.chunks());
@@ -223,3 +253,9 @@ hipError_t readout(void* host, const void* dev, size_t bytes, bool widen, hipStr
 }
 
 }  // namespace flbh
+
+int flb_readout_paths(int64_t* counts, int n) {
+  int64_t now[FLB_READ_PATHS];
+  for (int k = 0; k < FLB_READ_PATHS; ++k) now[k] = flbh::ring().paths[k];
+  return flbh::copy_paths(now, FLB_READ_PATHS, counts, n);
+}

@@ -495,6 +495,17 @@ enum {
   FLB_ADJ_PATHS = 4
 };
 int flb_adjoint_paths(flb_adjoint h, int64_t* counts, int n);
+/* How the process's read-outs of moments, populations and gradients ran, and
+ * the bytes of pinned host memory that they hold now (none once the last block
+ * and box is destroyed). */
+enum {
+  FLB_READ_DIRECT = 0,  /* small moments, written by their kernel into pinned memory */
+  FLB_READ_RING = 1,    /* through the ring of pinned buffers */
+  FLB_READ_PLAIN = 2,   /* one copy */
+  FLB_READ_PINNED = 3,  /* bytes */
+  FLB_READ_PATHS = 4
+};
+int flb_readout_paths(int64_t* counts, int n);
 /* Device copy bandwidth: a float4 copy kernel over `bytes` (rounded down to a
  * multiple of 16) between two fresh buffers, `reps` timed launches; *gbs gets
  * (read + written bytes) / mean launch time. No reference counterpart: it
