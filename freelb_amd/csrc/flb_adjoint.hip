@@ -1958,11 +1958,13 @@ int batch_backward_impl(flb_adjoint_batch_s* b, double* grad) {
     }
   }
   HIP_TRY(hipEventRecord(b->e1, b->stream));
+  std::vector<ReadPart> parts;
   double* out = grad;
   for (flb_adjoint_s* h : b->members) {
-    HIP_TRY(readout(out, h->d_grad, size_t(h->N) * sizeof(R), sizeof(R) == 4, b->stream));
+    parts.push_back({out, h->d_grad, size_t(h->N) * sizeof(R)});
     out += h->N;
   }
+  HIP_TRY(readout(parts.data(), parts.size(), sizeof(R) == 4, b->stream));
   HIP_TRY(hipEventElapsedTime(&b->bwd_ms, b->e0, b->e1));
   for (flb_adjoint_s* h : b->members) h->bwd_ms = b->bwd_ms;
   return FLB_OK;

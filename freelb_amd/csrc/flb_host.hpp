@@ -215,12 +215,18 @@ bool march_fits(size_t bytes);
 bool capturing(hipStream_t s);
 
 // Read-out to host memory (flb_readout.hip). readout: bytes of device memory
-// to the caller's array once the work enqueued on s is done; widen: FP32 on
-// the device, FP64 at the caller. Each block and adjoint box retains the
-// pinned buffers while it lives.
+// to the caller's array once the work enqueued on s is done, or several arrays
+// at once; widen: FP32 on the device, FP64 at the caller. Each block and
+// adjoint box retains the pinned buffers while it lives.
+struct ReadPart {
+  void* host;
+  const void* dev;
+  size_t bytes;  // on the device
+};
 void readout_retain();
 void readout_release();
 hipError_t readout(void* host, const void* dev, size_t bytes, bool widen, hipStream_t s);
+hipError_t readout(const ReadPart* parts, size_t n, bool widen, hipStream_t s);
 constexpr size_t kDirect = size_t(256) << 10;
 struct DirectOut {
   void* ptr = nullptr;

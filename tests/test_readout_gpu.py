@@ -8,7 +8,7 @@ import threading
 import numpy as np
 import pytest
 
-from freelb_amd import BlockLattice, Key_TypePair, abi
+from freelb_amd import Adjoint, AdjointBatch, BlockLattice, Key_TypePair, abi
 from freelb_amd.cases import FLUID, VOID
 from freelb_amd.lattice import weights
 
@@ -120,3 +120,32 @@ def test_threads_read_at_once():
     finally:
         for lat in (a, b, c):
             lat.close()
+
+
+@pytest.mark.parametrize("storage,dims,way", [("f32", [(64, 60, 50), (63, 61, 49), (7, 5, 3)] * 3, 1),
+                                              ("f64", [(64, 60, 50), (130, 61, 49), (7, 5, 3)], 1),
+                                              ("f32", [(20, 11, 9), (7, 5, 3)], 2)])
+def test_gradients_of_a_batch_are_one_read_out(storage, dims, way):
+    """Equal to the members' own, with parts of more than a chunk, of less, and of a few bytes."""
+    rng = np.random.default_rng(3)
+    boxes = []
+    try:
+        for d in dims:
+            boxes.append(Adjoint(d, omega=1.5, periodic=(True, False, False), storage=storage))
+            N = boxes[-1].N
+            boxes[-1].set_fraction(rng.uniform(0, 1, N))
+            boxes[-1].init_equilibrium(np.ones(N), rng.uniform(-0.01, 0.01, (3, N)))
+        alone = []
+        for a in boxes:
+            a.forward(3, 0)
+            alone.append(a.backward())
+        with AdjointBatch(boxes) as b:
+            b.forward(3, 0)
+            was = abi.readout_paths()
+            got = b.backward()
+            assert _took(was) == (0, way == 1, way == 2)
+        for g, w in zip(got, alone):
+            assert np.array_equal(g, w)
+    finally:
+        for a in boxes:
+            a.close()
