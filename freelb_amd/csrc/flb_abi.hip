@@ -428,7 +428,7 @@ int ensure_links(flb_block_s* b) {
   if (b->nbc == 0 || !b->flags_set) return FLB_OK;
   if (!b->links_dirty && b->d_links) return FLB_OK;
   if (!b->d_links) {
-    if (hipMalloc(reinterpret_cast<void**>(&b->d_links), size_t(b->stride) * sizeof(uint64_t)) != hipSuccess)
+    if (dev_alloc(&b->d_links, size_t(b->stride) * sizeof(uint64_t)) != hipSuccess)
       return fail(FLB_ERR_NOMEM, "wall-link allocation failed");
   }
   KArgs a = make_args(b);
@@ -442,7 +442,7 @@ int ensure_stage(flb_block b, size_t bytes) {
   if (b->d_stage) HIP_TRY(hipFree(b->d_stage));
   b->d_stage = nullptr;
   b->stage_bytes = 0;
-  if (hipMalloc(&b->d_stage, bytes) != hipSuccess)
+  if (dev_alloc(&b->d_stage, bytes) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "staging allocation of %zu bytes failed", bytes);
   b->stage_bytes = bytes;
   return FLB_OK;
@@ -453,7 +453,7 @@ int ensure_stage(flb_block b, size_t bytes) {
 int upload_field(flb_block b, const double* host, int ncomp, void** dst) {
   const size_t bytes = size_t(b->stride) * ncomp * b->real;
   if (!*dst) {
-    if (hipMalloc(dst, bytes) != hipSuccess)
+    if (dev_alloc(dst, bytes) != hipSuccess)
       return fail(FLB_ERR_NOMEM, "field allocation of %zu bytes failed", bytes);
   }
   if (b->real == 8) {
@@ -600,12 +600,12 @@ int flb_block_create(const flb_block_desc* desc, flb_block* out) {
     }
   }
   const size_t pop_bytes = size_t(b->pop_elems) * b->elem;
-  if (hipMalloc(&b->d_pops, pop_bytes) != hipSuccess) {
+  if (dev_alloc(&b->d_pops, pop_bytes) != hipSuccess) {
     delete b;
     return fail(FLB_ERR_NOMEM, "population allocation of %zu bytes failed", pop_bytes);
   }
-  if (hipMalloc(reinterpret_cast<void**>(&b->d_flags), size_t(b->stride)) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&b->d_red), 4 * sizeof(double)) != hipSuccess) {
+  if (dev_alloc(&b->d_flags, size_t(b->stride)) != hipSuccess ||
+      dev_alloc(&b->d_red, 4 * sizeof(double)) != hipSuccess) {
     flb_block_destroy(b);
     return fail(FLB_ERR_NOMEM, "flag allocation failed");
   }
@@ -629,9 +629,10 @@ int flb_block_destroy(flb_block b) {
   else (void)hipDeviceSynchronize();
   detach_couplings(b);
   void* ptrs[] = {b->d_pops,  b->d_flags,   b->d_rho,   b->d_u,       b->d_partials, b->d_red,
-                  b->d_stage, b->d_alt, b->d_links, b->d_rho_old, b->d_u_old, b->d_res};
+                  b->d_stage, b->d_links, b->d_rho_old, b->d_u_old, b->d_res};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  twin_drop(b->twin);
   if (b->retained) readout_release();
   delete b;
   return FLB_OK;
@@ -867,11 +868,11 @@ int flb_enable_tolerance(flb_block b) {
     return fail(FLB_ERR_STATE, "the block has no RHO / VELOCITY fields (FLB_DYN_BGK_WRITE tasks create them)");
   DeviceGuard g(b->device);
   const size_t one = size_t(b->stride) * b->real;
-  if (!b->d_rho_old && hipMalloc(&b->d_rho_old, one) != hipSuccess)
+  if (!b->d_rho_old && dev_alloc(&b->d_rho_old, one) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "residual field allocation failed");
-  if (!b->d_u_old && hipMalloc(&b->d_u_old, one * size_t(b->d)) != hipSuccess)
+  if (!b->d_u_old && dev_alloc(&b->d_u_old, one * size_t(b->d)) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "residual field allocation failed");
-  if (!b->d_res && hipMalloc(reinterpret_cast<void**>(&b->d_res), sizeof(unsigned long long)) != hipSuccess)
+  if (!b->d_res && dev_alloc(&b->d_res, sizeof(unsigned long long)) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "residual allocation failed");
   HIP_TRY(hipMemcpyAsync(b->d_rho_old, b->d_rho, one, hipMemcpyDeviceToDevice, b->stream));
   HIP_TRY(hipMemcpyAsync(b->d_u_old, b->d_u, one * size_t(b->d), hipMemcpyDeviceToDevice, b->stream));
@@ -1123,6 +1124,7 @@ static int watchdog_check(flb_block b) {
 // multiples of four steps, so that the state ends in the array it began in),
 // one launch per step otherwise.
 static int run_steps(flb_block b, int n) {
+  const TwinUse use(b->twin);
   const bool march = n >= 5 - b->parity && march_ready(b);
   int rc = FLB_OK;
   while (n > 0) {
@@ -1192,7 +1194,7 @@ int flb_reduce_mass_momentum(flb_block b, uint8_t mask, double out[4]) {
   if (!b->d_partials) {
     // one double4 per workgroup of the per-cell kernels
     const size_t nb = flb::cell_blocks(b->N);
-    if (hipMalloc(reinterpret_cast<void**>(&b->d_partials), nb * 4 * sizeof(double)) != hipSuccess)
+    if (dev_alloc(&b->d_partials, nb * 4 * sizeof(double)) != hipSuccess)
       return fail(FLB_ERR_NOMEM, "reduction scratch allocation failed");
   }
   HIP_TRY(launch_reduce(b, a, mask, b->d_partials, b->d_red));
@@ -1275,8 +1277,8 @@ int run_probe(int mode, int unroll, bool nt, int wg_per_cu, bool legacy, size_t 
   const size_t grid = wg_per_cu > 0 ? std::min(ntile, size_t(wg_per_cu) * size_t(cus)) : ntile;
   if (grid > size_t(0x7fffffff)) return fail(FLB_ERR_ARG, "probe grid too large");
   void *src = nullptr, *dst = nullptr;
-  if (hipMalloc(&src, n4 * 16) != hipSuccess) return fail(FLB_ERR_NOMEM, "probe allocation failed");
-  if (hipMalloc(&dst, n4 * 16) != hipSuccess) {
+  if (dev_alloc(&src, n4 * 16) != hipSuccess) return fail(FLB_ERR_NOMEM, "probe allocation failed");
+  if (dev_alloc(&dst, n4 * 16) != hipSuccess) {
     (void)hipFree(src);
     return fail(FLB_ERR_NOMEM, "probe allocation failed");
   }

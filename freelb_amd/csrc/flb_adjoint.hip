@@ -1316,7 +1316,7 @@ hipError_t mom_step(const flb_adjoint_s* h, const void* src, void* mom) {
 
 int alloc_state(flb_adjoint_s* h, void** p) {
   if (*p) return FLB_OK;
-  if (hipMalloc(p, state_bytes(h)) != hipSuccess)
+  if (dev_alloc(p, state_bytes(h)) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "adjoint state allocation of %zu bytes failed", state_bytes(h));
   // solid cells are never written by the step kernels: keep them zero
   HIP_TRY(hipMemsetAsync(*p, 0, state_bytes(h), h->stream));
@@ -1325,7 +1325,7 @@ int alloc_state(flb_adjoint_s* h, void** p) {
 
 int alloc_mom(flb_adjoint_s* h, void** p) {
   if (*p) return FLB_OK;
-  if (hipMalloc(p, mom_bytes(h)) != hipSuccess)
+  if (dev_alloc(p, mom_bytes(h)) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "moment record allocation of %zu bytes failed", mom_bytes(h));
   return FLB_OK;
 }
@@ -1375,11 +1375,11 @@ int prepare_forward(flb_adjoint_s* h, int T, int K) {
   if (h->jt_cap < T + 1) {
     if (h->d_jt) (void)hipFree(h->d_jt);
     h->d_jt = nullptr;
-    if (hipMalloc(reinterpret_cast<void**>(&h->d_jt), size_t(T + 1) * sizeof(double)) != hipSuccess)
+    if (dev_alloc(&h->d_jt, size_t(T + 1) * sizeof(double)) != hipSuccess)
       return fail(FLB_ERR_NOMEM, "objective buffer allocation failed");
     h->jt_cap = T + 1;
   }
-  if (!h->d_shares && hipMalloc(reinterpret_cast<void**>(&h->d_shares),
+  if (!h->d_shares && dev_alloc(&h->d_shares,
                                 size_t(kObjStates) * obj_plane(h) * sizeof(double)) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "objective share buffer allocation failed");
   return FLB_OK;
@@ -1556,7 +1556,7 @@ int prepare_backward(flb_adjoint_s* h) {
   for (void*& l : h->d_lam)
     if ((rc = alloc_state(h, &l))) return rc;
   if (!h->d_grad) {
-    if (hipMalloc(&h->d_grad, size_t(h->N) * h->real) != hipSuccess)
+    if (dev_alloc(&h->d_grad, size_t(h->N) * h->real) != hipSuccess)
       return fail(FLB_ERR_NOMEM, "gradient allocation failed");
   }
   return FLB_OK;
@@ -1686,14 +1686,14 @@ int upload_table(flb_adjoint_batch_s* b) {
     if (b->d_slots) (void)hipFree(b->d_slots);
     b->d_slots = nullptr;
     b->slots_cap = 0;
-    if (hipMalloc(&b->d_slots, bytes_slots) != hipSuccess) return fail(FLB_ERR_NOMEM, "slot table allocation failed");
+    if (dev_alloc(&b->d_slots, bytes_slots) != hipSuccess) return fail(FLB_ERR_NOMEM, "slot table allocation failed");
     b->slots_cap = bytes_slots;
   }
   if (bytes_tab > b->tab_cap) {
     if (b->d_tab) (void)hipFree(b->d_tab);
     b->d_tab = nullptr;
     b->tab_cap = 0;
-    if (hipMalloc(&b->d_tab, bytes_tab) != hipSuccess) return fail(FLB_ERR_NOMEM, "entry table allocation failed");
+    if (dev_alloc(&b->d_tab, bytes_tab) != hipSuccess) return fail(FLB_ERR_NOMEM, "entry table allocation failed");
     b->tab_cap = bytes_tab;
   }
   std::vector<R*> slots(n * size_t(nslots), nullptr);
@@ -1782,9 +1782,9 @@ int prepare_march(flb_adjoint_batch_s* b) {
     std::vector<flb::MarchWg> wg;
     const double span = march_plan_batch(boxes, int(b->real), cus, march_nt(b->real, k == 1), mt, wg);
     if (k == 0 && span * 0.9e-6 > 4.0 * double(live) / 4.8e12) return FLB_OK;
-    if (hipMalloc(reinterpret_cast<void**>(&b->d_mt[k]), mt.size() * sizeof(mt[0])) != hipSuccess ||
-        hipMalloc(reinterpret_cast<void**>(&b->d_mwg[k]), wg.size() * sizeof(wg[0])) != hipSuccess)
-      return fail(FLB_ERR_NOMEM, "batch tile table allocation failed");
+    if (dev_alloc(&b->d_mt[k], mt.size() * sizeof(mt[0])) != hipSuccess ||
+        dev_alloc(&b->d_mwg[k], wg.size() * sizeof(wg[0])) != hipSuccess)
+      return FLB_OK;
     HIP_TRY(hipMemcpyAsync(b->d_mt[k], mt.data(), mt.size() * sizeof(mt[0]), hipMemcpyHostToDevice, b->stream));
     HIP_TRY(hipMemcpyAsync(b->d_mwg[k], wg.data(), wg.size() * sizeof(wg[0]), hipMemcpyHostToDevice, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
@@ -2000,9 +2000,9 @@ int flb_adjoint_create(const flb_adjoint_desc* desc, flb_adjoint* out) {
   if (hipGetDevice(&h->device) != hipSuccess) rc = fail(FLB_ERR_HIP, "no HIP device");
   if (rc == FLB_OK && (hipEventCreate(&h->e0) != hipSuccess || hipEventCreate(&h->e1) != hipSuccess))
     rc = fail(FLB_ERR_HIP, "event creation failed");
-  if (rc == FLB_OK && (hipMalloc(reinterpret_cast<void**>(&h->d_solid), size_t(N)) != hipSuccess ||
-                       hipMalloc(reinterpret_cast<void**>(&h->d_link), size_t(N) * sizeof(uint32_t)) != hipSuccess ||
-                       hipMalloc(&h->d_s, size_t(N) * h->real) != hipSuccess))
+  if (rc == FLB_OK && (dev_alloc(&h->d_solid, size_t(N)) != hipSuccess ||
+                       dev_alloc(&h->d_link, size_t(N) * sizeof(uint32_t)) != hipSuccess ||
+                       dev_alloc(&h->d_s, size_t(N) * h->real) != hipSuccess))
     rc = fail(FLB_ERR_NOMEM, "adjoint field allocation failed");
   if (rc == FLB_OK) rc = alloc_state(h, &h->d_f0);
   if (rc == FLB_OK && (hipMemsetAsync(h->d_solid, 0, size_t(N), h->stream) != hipSuccess ||
@@ -2091,7 +2091,7 @@ int flb_adjoint_init_equilibrium(flb_adjoint h, const double* rhou) {
   DeviceGuard g(h->device);
   const size_t count = size_t(4) * size_t(h->N);
   void* stage = nullptr;
-  if (hipMalloc(&stage, count * h->real) != hipSuccess) return fail(FLB_ERR_NOMEM, "staging allocation failed");
+  if (dev_alloc(&stage, count * h->real) != hipSuccess) return fail(FLB_ERR_NOMEM, "staging allocation failed");
   hipError_t e;
   if (h->real == 8) {
     e = hipMemcpyAsync(stage, rhou, count * 8, hipMemcpyHostToDevice, h->stream);

@@ -69,7 +69,7 @@ struct flb_batch_s {
   flb::MarchArgs* d_mt = nullptr;
   flb::MarchWg* d_mwg = nullptr;
   size_t mwg_cap = 0;
-  char* d_alt = nullptr;
+  flbh::Twin twin;  // the blocks' second arrays
   double march_span = 0.0;  // estimated time of a pass, in march_plan_batch's unit
 };
 
@@ -156,7 +156,7 @@ int refresh(flb_batch_s* t, bool force) {
     if (t->d_wblk) HIP_TRY(hipFree(t->d_wblk));
     t->d_wblk = nullptr;
     t->wblk_cap = 0;
-    if (hipMalloc(reinterpret_cast<void**>(&t->d_wblk), std::max<size_t>(waves, 1) * sizeof(int)) != hipSuccess)
+    if (dev_alloc(&t->d_wblk, std::max<size_t>(waves, 1) * sizeof(int)) != hipSuccess)
       return fail(FLB_ERR_NOMEM, "batch wave table allocation failed");
     t->wblk_cap = waves;
   }
@@ -183,7 +183,7 @@ int refresh(flb_batch_s* t, bool force) {
 // a 256^3 block.
 int prepare_march(flb_batch_s* t) {
   flb_batch_s::March& mc = t->march;
-  if (mc.state >= 0 || capturing(t->stream)) return FLB_OK;
+  if (mc.state == 0 || (mc.state == 1 && t->twin.p) || capturing(t->stream)) return FLB_OK;
   mc.state = 0;
   size_t live = 0, alt = 0;
   if (t->halo) return FLB_OK;
@@ -217,14 +217,7 @@ int prepare_march(flb_batch_s* t) {
   }
   // a unit of the estimate is 0.75 to 0.94 us, single steps move 4.2 to 5.5 TB/s
   if (t->march_span * 0.9e-6 > 4.0 * double(live) / 4.8e12) return FLB_OK;
-  if (!t->d_alt) {
-    if (!march_fits(alt)) return FLB_OK;
-    if (hipMalloc(reinterpret_cast<void**>(&t->d_alt), alt) != hipSuccess) {
-      (void)hipGetLastError();
-      t->d_alt = nullptr;
-      return FLB_OK;
-    }
-  }
+  if (!twin_take(t->twin, alt, t->device, t->stream)) return FLB_OK;
   mc.dyn = form[0].dyn;
   size_t off = 0;
   for (size_t k = 0; k < nb; ++k) {
@@ -233,19 +226,17 @@ int prepare_march(flb_batch_s* t) {
     m.dyn = form[k].dyn;
     m.cs = form[k].cs;
     m.mask = form[k].mask;
-    m.dst = t->d_alt + off + size_t(flb::kFrontPad) * b->elem;
+    m.dst = t->twin.p + off + size_t(flb::kFrontPad) * b->elem;
     off += (size_t(b->pop_elems) * b->elem + 255) / 256 * 256;
   }
   mc.wgs = unsigned(t->h_mwg.size());
-  if (!t->d_mt && hipMalloc(reinterpret_cast<void**>(&t->d_mt), nb * sizeof(flb::MarchArgs)) != hipSuccess)
-    return fail(FLB_ERR_NOMEM, "batch tile table allocation failed");
+  if (!t->d_mt && dev_alloc(&t->d_mt, nb * sizeof(flb::MarchArgs)) != hipSuccess) return FLB_OK;
   const size_t mwg_bytes = t->h_mwg.size() * sizeof(flb::MarchWg);
   if (t->mwg_cap < t->h_mwg.size()) {
     if (t->d_mwg) HIP_TRY(hipFree(t->d_mwg));
     t->d_mwg = nullptr;
     t->mwg_cap = 0;
-    if (hipMalloc(reinterpret_cast<void**>(&t->d_mwg), mwg_bytes) != hipSuccess)
-      return fail(FLB_ERR_NOMEM, "batch tile table allocation failed");
+    if (dev_alloc(&t->d_mwg, mwg_bytes) != hipSuccess) return FLB_OK;
     t->mwg_cap = t->h_mwg.size();
   }
   mc.wg = t->d_mwg;
@@ -361,8 +352,8 @@ int flb_batch_create(const flb_block* blocks, int n, void* stream, flb_batch* ou
   for (auto& e : t->events)
     if (rc == FLB_OK && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
       rc = fail(FLB_ERR_HIP, "event creation failed");
-  if (rc == FLB_OK && (hipMalloc(reinterpret_cast<void**>(&t->d_tab), size_t(n) * sizeof(KArgs)) != hipSuccess ||
-                       hipMalloc(reinterpret_cast<void**>(&t->d_wave0), size_t(n + 1) * sizeof(int64_t)) != hipSuccess))
+  if (rc == FLB_OK && (dev_alloc(&t->d_tab, size_t(n) * sizeof(KArgs)) != hipSuccess ||
+                       dev_alloc(&t->d_wave0, size_t(n + 1) * sizeof(int64_t)) != hipSuccess))
     rc = fail(FLB_ERR_NOMEM, "batch table allocation failed");
   if (rc == FLB_OK) rc = refresh(t, true);
   if (rc != FLB_OK) {
@@ -385,7 +376,7 @@ int flb_batch_destroy(flb_batch t) {
   if (t->d_wblk) (void)hipFree(t->d_wblk);
   if (t->d_mt) (void)hipFree(t->d_mt);
   if (t->d_mwg) (void)hipFree(t->d_mwg);
-  if (t->d_alt) (void)hipFree(t->d_alt);
+  twin_drop(t->twin);
   delete t;
   return FLB_OK;
 }
@@ -422,10 +413,12 @@ int flb_batch_step(flb_batch t, int n) {
   if (rc) return rc;
   if ((rc = refresh(t, false))) return rc;
   if (t->halo && (rc = halo_refresh(t->halo))) return rc;
+  const TwinUse use(t->twin);
   const bool run = n >= 5 - parity;  // long enough for a pass of two steps and one back
   if (run && (rc = prepare_march(t))) return rc;
   if ((rc = join_in(t))) return rc;
-  const bool march = run && t->march.state == 1;
+  const bool march = run && t->march.state == 1 && t->twin.p;
+  if (march) t->twin.held = t->twin.held || capturing(t->stream);
   HIP_TRY(enqueue_steps(t, parity, n, march, t->stream));
   advance(t, n, two_steps(parity, n, march));
   return join_out(t);
@@ -457,9 +450,10 @@ int flb_batch_capture(flb_batch t, int n) {
   // the halo's tables are refreshed (host copies and a stream sync) before
   // the capture opens, as flb_batch_step does before its launches
   if (t->halo && (rc = halo_refresh(t->halo))) return rc;
+  const TwinUse use(t->twin);
   const bool run = n >= 5 - parity;
   if (run && (rc = prepare_march(t))) return rc;
-  const bool march = run && t->march.state == 1;
+  const bool march = run && t->march.state == 1 && t->twin.p;
   hipStream_t cs = nullptr;
   HIP_TRY(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
   hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
@@ -505,10 +499,11 @@ int flb_batch_replay(flb_batch t) {
     return fail(FLB_ERR_STATE, "block dynamics changed kernel family since capture: capture again");
   // a graph with passes of two steps is replayed while the blocks still allow
   // the passes it holds; else its steps are launched singly
+  const TwinUse use(t->twin);
   const bool passes = t->graph_march.state == 1;
   if (passes && (rc = prepare_march(t))) return rc;
   if ((rc = join_in(t))) return rc;
-  const bool as_recorded = !passes || t->march.same_launch(t->graph_march);
+  const bool as_recorded = !passes || (t->twin.p && t->march.same_launch(t->graph_march));
   if (as_recorded) HIP_TRY(hipGraphLaunch(t->exec, t->stream));
   else HIP_TRY(enqueue_steps(t, parity, t->graph_steps, false, t->stream));
   advance(t, t->graph_steps, two_steps(parity, t->graph_steps, passes && as_recorded));
@@ -547,7 +542,7 @@ int flb_batch_autotune(flb_batch t, int steps, flb_launch_cfg* best, double* bes
   size_t total = 0;
   for (const Region& r : regions) total += r.bytes;
   char* snap = nullptr;
-  if (hipMalloc(reinterpret_cast<void**>(&snap), total) != hipSuccess)
+  if (dev_alloc(&snap, total) != hipSuccess)
     return fail(FLB_ERR_NOMEM, "autotune snapshot of %zu bytes failed", total);
   if ((rc = join_in(t))) {
     (void)hipFree(snap);

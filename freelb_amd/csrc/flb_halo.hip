@@ -235,9 +235,9 @@ int flb_halo_create(const flb_block* blocks, int n, const int* origins, const in
   h->wgs = unsigned(wg.size());
   int rc = FLB_OK;
   const size_t ni = std::max<size_t>(items.size(), 1);
-  if (hipMalloc(reinterpret_cast<void**>(&h->d_tab), size_t(n) * sizeof(KArgs)) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&h->d_items), ni * sizeof(H::Item)) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&h->d_wg), std::max<size_t>(wg.size(), 1) * sizeof(flb::HaloWg)) != hipSuccess)
+  if (dev_alloc(&h->d_tab, size_t(n) * sizeof(KArgs)) != hipSuccess ||
+      dev_alloc(&h->d_items, ni * sizeof(H::Item)) != hipSuccess ||
+      dev_alloc(&h->d_wg, std::max<size_t>(wg.size(), 1) * sizeof(flb::HaloWg)) != hipSuccess)
     rc = fail(FLB_ERR_NOMEM, "halo table allocation failed");
   if (rc == FLB_OK && !items.empty() &&
       (hipMemcpyAsync(h->d_items, items.data(), items.size() * sizeof(H::Item), hipMemcpyHostToDevice,

@@ -12,6 +12,39 @@
 #include "../../include/flb_abi.h"
 #include "flb_internal.hpp"
 
+namespace flbh {
+
+// The second population array of a block's or a batch's two-step runs: scratch
+// between calls. The library gives those of other objects back where it runs
+// out of device memory (dev_alloc); a later run takes one again if it fits.
+struct Twin {
+  char* p = nullptr;
+  int device = 0;
+  hipStream_t stream = nullptr;  // of the runs that use it
+  int users = 0;                 // runs being enqueued now
+  bool held = false;             // a capture recorded it: it stays while its owner lives
+};
+// Takes the array, if there is none, where march_fits allows it.
+bool twin_take(Twin& t, size_t bytes, int device, hipStream_t s);
+void twin_drop(Twin& t);
+// Keeps the array, if there is one, from being given back while it lives.
+struct TwinUse {
+  Twin& t;
+  explicit TwinUse(Twin& twin);
+  ~TwinUse();
+  TwinUse(const TwinUse&) = delete;
+  TwinUse& operator=(const TwinUse&) = delete;
+};
+// hipMalloc; out of memory, once more after second arrays were given back. A
+// failure leaves *p null and no error for the next launch's check to find.
+hipError_t dev_alloc(void** p, size_t bytes);
+template <class T>
+hipError_t dev_alloc(T** p, size_t bytes) {
+  return dev_alloc(reinterpret_cast<void**>(p), bytes);
+}
+
+}  // namespace flbh
+
 struct flb_block_s {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -52,7 +85,7 @@ struct flb_block_s {
   int vec = 0;  // step kernel form: 0 automatic cell form, -1 row segments, -3 linear runs,
                 // 1/2/4 row form with that many cells per thread
   int wpb = 4;   // wavefronts per workgroup
-  void* d_alt = nullptr;   // second population array of the two-step march (flb_march.hip), scratch between calls
+  flbh::Twin twin;         // second population array of the two-step march (flb_march.hip)
   int march = -1;          // 1: the march may step the block, 0: not, -1: to be checked (flags, tasks or walls changed)
   flb::MarchArgs tiles{};  // its tiles, planned once (ntx 0: not yet)
   int closed = -1;         // 1: no link of an updated cell leads to a cell that is not updated but wall links, 0, -1 likewise

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <functional>
+#include <mutex>
 #include <queue>
 #include <utility>
 #include <vector>
@@ -236,13 +237,94 @@ bool capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
+namespace {
+
+// Every second array there is; mu guards the list and the arrays' fields.
+struct Twins {
+  std::mutex mu;
+  std::vector<Twin*> list;
+};
+Twins& twins() {
+  static Twins* t = new Twins();  // never destroyed: blocks may outlive static objects
+  return *t;
+}
+
+// Frees the second arrays of the current device that no run is using and no
+// capture has recorded; true if there was one.
+bool twins_give_back() {
+  Twins& all = twins();
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> l(all.mu);
+  bool any = false;
+  for (size_t k = all.list.size(); k-- > 0;) {
+    Twin& t = *all.list[k];
+    if (t.users > 0 || t.held || t.device != dev || capturing(t.stream)) continue;
+    if (hipStreamSynchronize(t.stream) != hipSuccess || hipFree(t.p) != hipSuccess) continue;
+    t.p = nullptr;
+    all.list.erase(all.list.begin() + std::ptrdiff_t(k));
+    any = true;
+  }
+  return any;
+}
+
+}  // namespace
+
+bool twin_take(Twin& t, size_t bytes, int device, hipStream_t s) {
+  Twins& all = twins();
+  std::lock_guard<std::mutex> l(all.mu);
+  if (t.p) return true;
+  if (!march_fits(bytes)) return false;
+  if (hipMalloc(reinterpret_cast<void**>(&t.p), bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    t.p = nullptr;
+    return false;
+  }
+  t.device = device;
+  t.stream = s;
+  all.list.push_back(&t);
+  return true;
+}
+
+void twin_drop(Twin& t) {
+  Twins& all = twins();
+  std::lock_guard<std::mutex> l(all.mu);
+  if (!t.p) return;
+  all.list.erase(std::find(all.list.begin(), all.list.end(), &t));
+  (void)hipFree(t.p);
+  t.p = nullptr;
+}
+
+TwinUse::TwinUse(Twin& twin) : t(twin) {
+  std::lock_guard<std::mutex> l(twins().mu);
+  ++t.users;
+}
+TwinUse::~TwinUse() {
+  std::lock_guard<std::mutex> l(twins().mu);
+  --t.users;
+}
+
+hipError_t dev_alloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    if (e == hipErrorOutOfMemory && twins_give_back()) e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+  }
+  return e;
+}
+
 // The second array is taken at the first run of steps and kept with the block
-// (so a captured run stays valid while the block lives). It is scratch: runs
-// begin and end in d_pops. Blocks do without it, and step singly, where it
-// does not fit (march_fits), and in a capture that comes before the first run.
+// until memory is short (twins_give_back; one that a captured run holds, while
+// the block lives). It is scratch: runs begin and end in d_pops. Blocks do
+// without it, and step singly, where it does not fit (march_fits), and in a
+// capture that comes before the first run. The caller holds a TwinUse.
 bool march_ready(flb_block_s* b) {
   if (!b->flags_set || b->march == 0) return false;
-  if (b->march == 1 && (b->nbc == 0 || !b->links_dirty) && b->d_alt) return true;
+  if (b->march == 1 && (b->nbc == 0 || !b->links_dirty) && b->twin.p) return true;
   if (capturing(b->stream)) return false;
   if (b->march < 0) {
     flb::MarchArgs m;
@@ -264,16 +346,7 @@ bool march_ready(flb_block_s* b) {
     if (!ok) return false;
   }
   if (ensure_links(b) != FLB_OK) return false;
-  if (!b->d_alt) {
-    const size_t bytes = size_t(b->pop_elems) * b->elem;
-    if (!march_fits(bytes)) return false;
-    if (hipMalloc(&b->d_alt, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      b->d_alt = nullptr;
-      return false;
-    }
-  }
-  return true;
+  return twin_take(b->twin, size_t(b->pop_elems) * b->elem, b->device, b->stream);
 }
 
 int march_run(flb_block_s* b, int n) {
@@ -281,7 +354,8 @@ int march_run(flb_block_s* b, int n) {
   flb::MarchArgs m = b->tiles;
   one_dynamics(b, &m);
   char* const pops = static_cast<char*>(b->d_pops) + flb::kFrontPad * b->elem;
-  char* const alt = static_cast<char*>(b->d_alt) + flb::kFrontPad * b->elem;
+  char* const alt = b->twin.p + flb::kFrontPad * b->elem;
+  b->twin.held = b->twin.held || capturing(b->stream);
   for (int k = 0; k < n; k += 2) {
     a.pops = k % 4 == 0 ? pops : alt;
     m.dst = k % 4 == 0 ? alt : pops;

@@ -517,9 +517,9 @@ int flb_refine_create(flb_block coarse, flb_block fine, const int* origin, void*
   r->avg_links = avg_links;
   r->intp_links = intp_links;
   DeviceGuard g(r->device);
-  if (hipMalloc(reinterpret_cast<void**>(&r->d_avg), std::max<size_t>(1, avg.size()) * sizeof(RF::AvgItem)) !=
+  if (dev_alloc(&r->d_avg, std::max<size_t>(1, avg.size()) * sizeof(RF::AvgItem)) !=
           hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&r->d_intp), std::max<size_t>(1, intp.size()) * sizeof(RF::IntpItem)) !=
+      dev_alloc(&r->d_intp, std::max<size_t>(1, intp.size()) * sizeof(RF::IntpItem)) !=
           hipSuccess) {
     flb_refine_destroy(r);
     return fail(FLB_ERR_NOMEM, "refinement item allocation failed");
