@@ -1777,7 +1777,7 @@ int prepare_march(flb_adjoint_batch_s* b) {
   if (live < kTwoStepBytes) return FLB_OK;
   int cus = 0;
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < (b->real == 4 ? 2 : 1); ++k) {  // FP64 goes back in single steps
     std::vector<flb::MarchArgs> mt;
     std::vector<flb::MarchWg> wg;
     const double span = march_plan_batch(boxes, int(b->real), cus, march_nt(b->real, k == 1), mt, wg);
@@ -1789,6 +1789,7 @@ int prepare_march(flb_adjoint_batch_s* b) {
     HIP_TRY(hipMemcpyAsync(b->d_mwg[k], wg.data(), wg.size() * sizeof(wg[0]), hipMemcpyHostToDevice, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
     b->nmwg[k] = unsigned(wg.size());
+    for (flb_adjoint_s* h : b->members) h->paths[FLB_ADJ_PATH_PLANS] += 1;
   }
   b->march = 1;
   return FLB_OK;

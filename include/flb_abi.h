@@ -491,7 +491,7 @@ enum {
   FLB_ADJ_PATH_FORWARD_TWO = 0,   /* forward launches of two steps, those of recomputed segments included */
   FLB_ADJ_PATH_BACKWARD_TWO = 1,  /* backward launches of two steps */
   FLB_ADJ_PATH_BACKWARD_PULL = 2, /* single backward steps of runs without launches of two */
-  FLB_ADJ_PATH_PLANS = 3,         /* tile plans made for launches of two steps, one per direction */
+  FLB_ADJ_PATH_PLANS = 3,         /* tile plans made for launches of two steps, one per direction, a batch's too */
   FLB_ADJ_PATHS = 4
 };
 int flb_adjoint_paths(flb_adjoint h, int64_t* counts, int n);

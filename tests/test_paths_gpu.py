@@ -199,6 +199,24 @@ def test_tiles_are_planned_once():
             assert adj.paths()["plans"] == plans
 
 
+@pytest.mark.parametrize("storage,plans", [("f32", 2), ("f64", 1)])
+def test_batches_plan_the_directions_they_take(storage, plans):
+    """FP64 goes back in single steps, so only its forward passes are planned."""
+    members = []
+    try:
+        for dims in ((131, 60, 60), (75, 66, 101), (64, 96, 80), (200, 130, 32), (10, 6, 5), (96, 93, 97), (90, 80, 70)):
+            members.append(Adjoint(dims, omega=1.6, periodic=(True, False, False), storage=storage))
+            members[-1].init_equilibrium(np.ones(members[-1].N), np.zeros((3, members[-1].N)))
+        with AdjointBatch(members) as b:
+            for K in (0, 3):
+                b.forward(5, K)
+                b.backward()
+        assert all(a.paths()["forward_two"] > 0 and a.paths()["plans"] == plans for a in members)
+    finally:
+        for a in members:
+            a.close()
+
+
 def test_bad_count_is_refused():
     with cavity_block((8, 8, 8)) as lat:
         with pytest.raises(abi.FLBError):
