@@ -251,33 +251,54 @@ def batch_bench(timer, nblocks=512, seed=2025, graph_steps=500, storage="f32", l
             "diverged_blocks": [(k, round(specs[k]["tau"], 4), round(specs[k]["u_lid"], 3)) for k in diverged]}
 
 
-# algorithmic HBM bytes per cell of the FP32 adjoint's single steps (larger
-# boxes take two steps per launch, which move about half as much: the rates are
-# then what single steps would need), for boxes without solid cells (their link
-# words come from the cell's place; a box with solid cells also reads a 4-byte
-# link word per cell and kernel):
-# - forward push: reads and writes 19 populations, reads s (4 B);
+# algorithmic HBM bytes per cell of the FP32 adjoint, for boxes without solid
+# cells (their link words come from the cell's place; a box with solid cells
+# also reads a 4-byte link word per cell and kernel):
+# - forward push: reads and writes 19 populations, reads s (4 B), per launch of
+#   one step or of two;
 # - moment record (rho - 1, u) a recompute step, or a forward step with
-#   checkpoint_every 0, also writes: 16 B;
-# - moment record alone (the last state of each recomputed segment): reads
-#   19 populations and s, writes 16 B;
+#   checkpoint_every 0, also writes: 16 B per state;
+# - the records alone (the last state, or the last two in one launch, of each
+#   recomputed segment): reads 19 populations and s, writes 16 B per state;
 # - adjoint step: reads the moment record and 19 adjoint values, writes 19
-#   adjoint values, reads s and updates dJ/ds (8 B).
+#   adjoint values, reads s and updates dJ/ds (8 B); in launches of two steps
+#   two records, the rest once.
 ADJ_FWD_BYTES = 19 * 4 * 2 + 4
 ADJ_MOM_BYTES = 4 * 4
-ADJ_MOMONLY_BYTES = 19 * 4 + 4 + 4 * 4
+ADJ_READ_BYTES = 19 * 4 + 4
 ADJ_BWD_BYTES = 4 * 4 + 19 * 4 * 2 + 4 + 8
 
 
-def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms):
+def _adjoint_bytes(T, K, two):
+    """Bytes per cell of a forward run of T steps with a checkpoint every K (0:
+    every state's record), and of the backward run; two: whether the forward
+    and the backward steps are taken two per launch where the segments allow."""
+    fwd = bwd = 0
+    t = 0
+    while t < T:
+        n = 2 if two[0] and t + 2 <= T and not (K > 0 and (t + 1) % K == 0) else 1
+        fwd += ADJ_FWD_BYTES + (n * ADJ_MOM_BYTES if K == 0 else 0)
+        t += n
+    for t0 in range(0, T, K or T):
+        left = steps = min(K or T, T - t0)
+        while K > 0 and left > 0:  # records of the segment's states
+            n = 2 if two[0] and left >= 2 else 1
+            bwd += (ADJ_READ_BYTES if left == n else ADJ_FWD_BYTES) + n * ADJ_MOM_BYTES
+            left -= n
+        pairs = steps // 2 if two[1] else 0
+        bwd += pairs * (ADJ_BWD_BYTES + ADJ_MOM_BYTES) + (steps - 2 * pairs) * ADJ_BWD_BYTES
+    return fwd, bwd
+
+
+def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms, two=(False, False)):
     """Cell updates per second of the forward pass, of the adjoint pass
     (T adjoint steps plus the T - ceil(T/K) recomputed forward steps and the
     ceil(T/K) moment records of segment ends) and of the whole gradient, with
-    the bandwidth each pass reaches."""
+    the bandwidth each pass reaches; two: which of the passes took two steps
+    per launch."""
     nseg = -(-T // K) if K > 0 else 0
     rec = T - nseg if K > 0 else 0
-    fwd_b = cells * T * (ADJ_FWD_BYTES + (ADJ_MOM_BYTES if K == 0 else 0))
-    bwd_b = cells * (T * ADJ_BWD_BYTES + rec * (ADJ_FWD_BYTES + ADJ_MOM_BYTES) + nseg * ADJ_MOMONLY_BYTES)
+    fwd_b, bwd_b = (cells * b for b in _adjoint_bytes(T, K, two))
     return {"forward_mlups": round(cells * T / fwd_ms / 1e3, 1),
             "adjoint_mlups": round(cells * T / bwd_ms / 1e3, 1),
             "gradient_mlups": round(cells * T / (fwd_ms + bwd_ms) / 1e3, 1),
@@ -285,7 +306,13 @@ def _adjoint_rates(cells, T, K, fwd_ms, bwd_ms):
             "forward_gbs": round(fwd_b / fwd_ms / 1e6, 1), "backward_gbs": round(bwd_b / bwd_ms / 1e6, 1),
             "forward_frac": round(fwd_b / fwd_ms / 1e6 / HBM_PEAK_GBS, 4),
             "backward_frac": round(bwd_b / bwd_ms / 1e6 / HBM_PEAK_GBS, 4),
-            "recomputed_steps": rec}
+            "steps_per_launch": [1 + int(t) for t in two], "recomputed_steps": rec}
+
+
+def _two_step(adj):
+    """Which of a box's passes, forward and backward, take two steps per launch."""
+    p = adj.paths()
+    return p["forward_two"] > 0, p["backward_two"] > 0
 
 
 def adjoint_bench(T=800, K=28):
@@ -301,17 +328,18 @@ def adjoint_bench(T=800, K=28):
         J = adj.forward(T, K)
         g = adj.backward()
         fwd_ms, bwd_ms = adj.timing()
+        two = _two_step(adj)
     rec = f"checkpoint every {K}" if K > 0 else "moment record of every state (checkpoint_every 0), no recompute"
     out = {"workload": f"channel 192x96x96, T {T}, {rec}, FP32", "cells": int(s.size),
            "J": J, "grad_finite": bool(np.isfinite(g).all())}
-    out.update(_adjoint_rates(s.size, T, K, fwd_ms, bwd_ms))
+    out.update(_adjoint_rates(s.size, T, K, fwd_ms, bwd_ms, two))
     return out
 
 
 def adjoint_batch_bench(n=64, T=400, seed=11, fp64_check=False, K=None):
     """n channels with seeded extents uniform in [64,32,32]..[128,64,64]
     (numpy default_rng(seed)), each with its own seeded Brinkman field,
-    stepped as one batch (one launch per step over all boxes), T steps with
+    stepped as one batch (one launch over all boxes per step or per two), T steps with
     a checkpoint every round(sqrt(T)) steps (or every K; K = 0 records every
     state's moments and recomputes nothing), then the batched adjoint. With
     fp64_check the same batch runs in FP64 and the FP32 objective and
@@ -329,15 +357,16 @@ def adjoint_batch_bench(n=64, T=400, seed=11, fp64_check=False, K=None):
         J32 = b.forward(T, K)
         g32 = b.backward()
         fwd_ms, bwd_ms = b.timing()
+        two = _two_step(mem[0])
     finally:
         b.close()
         for m in mem:
             m.close()
     rec = f"checkpoint every {K}" if K > 0 else "moment record of every state (checkpoint_every 0), no recompute"
     out = {"workload": f"{n} channels, extents U[64..128]xU[32..64]xU[32..64] (seed {seed}), T {T}, "
-                       f"{rec}, FP32, one launch per step", "boxes": n, "cells": cells,
+                       f"{rec}, FP32, one launch per step or two", "boxes": n, "cells": cells,
            "setup_s": round(setup_s, 1), "grad_finite": bool(all(np.isfinite(g).all() for g in g32))}
-    out.update(_adjoint_rates(cells, T, K, fwd_ms, bwd_ms))
+    out.update(_adjoint_rates(cells, T, K, fwd_ms, bwd_ms, two))
     if fp64_check:
         b, mem, _ = channel_batch(dims, storage="f64", seed=seed)
         try:

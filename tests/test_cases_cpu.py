@@ -57,3 +57,16 @@ def test_adjoint_byte_accounting():
     assert r["recomputed_steps"] == 0
     assert r["backward_gbs"] == round(cells * 800 * 180 / 1e6, 1)
     assert r["forward_gbs"] == round(cells * 800 * 172 / 1e6, 1)
+
+
+def test_adjoint_byte_accounting_of_two_steps_per_launch():
+    """Launches of two steps move the populations, s and the gradient once. T = 800, K = 28: each
+    segment of 28 states recomputes 13 launches that store a state (188 B) and one of the last two
+    records (112 B), and goes back in 14 of 196 B; the segment of 16, in 7, 1 and 8. Forward, 400
+    launches of 156 B. K = 0: 400 of 188 B and of 196 B; T = 7, K = 3: spans of 2, 1, 2, 1, 1."""
+    r = bench._adjoint_rates(1000, 800, 28, 1.0, 1.0, (True, True))
+    assert r["forward_gbs"] == round(1000 * 400 * 156 / 1e6, 1)
+    assert r["backward_gbs"] == round(1000 * (28 * (13 * 188 + 112 + 14 * 196) + 7 * 188 + 112 + 8 * 196) / 1e6, 1)
+    assert bench._adjoint_bytes(800, 0, (True, True)) == (400 * 188, 400 * 196)
+    assert bench._adjoint_bytes(7, 3, (True, False)) == (5 * 156, 2 * (188 + 96) + 96 + 7 * 180)
+    assert bench._adjoint_bytes(7, 3, (False, True)) == (7 * 156, 2 * (2 * 172 + 96) + 96 + 2 * (196 + 180) + 180)
