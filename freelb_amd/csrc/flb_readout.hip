@@ -30,6 +30,7 @@ namespace {
 constexpr size_t kChunk = size_t(2) << 20;
 constexpr int kRing = 16;     // 32 MiB of pinned memory while the ring lives
 constexpr int kWorkers = 8;
+constexpr int kCopiesFirst = 4;  // DirectOut
 
 // The ring serves one read-out at a time (busy); it is made at the first large
 // read-out and given back when the last block or box of the process goes.
@@ -45,7 +46,7 @@ struct Ring {
   int device = -1;  // of the events
   std::mutex direct_busy;
   char* direct = nullptr;
-  bool second = false;  // small moments were read since the buffer was given back
+  int small = 0;  // small moments read by a copy since the buffer was given back
   std::atomic<int64_t> paths[FLB_READ_PATHS] = {};  // flb_readout_paths
 };
 Ring& ring() {
@@ -211,24 +212,27 @@ void readout_release() {
   drop(r);
   std::lock_guard<std::mutex> d(r.direct_busy);
   unpin(r, &r.direct, kDirect);
-  r.second = false;
+  r.small = 0;
 }
 
 // A kernel's output of at most kDirect bytes may go straight into pinned
 // memory instead of a device buffer that is copied afterwards: one operation
 // less on the stream (a step of 16^3 cells and its moments 39 -> 28 us). Holds the
 // buffer while it lives; ptr is null where another thread holds it, and for
-// the first such read-out, as pinning costs 40 us: a program that makes, reads
-// once and closes a 16^3 block at a time takes 175 us with the copy, 222 without.
+// the first four such read-outs: pinning and giving back cost 47 us, as much
+// as four read-outs save. A program that makes a 16^3 block, steps and reads
+// it k times and closes it, copies only -> buffer from the second read-out on
+// -> now: k = 1 174 -> 169 -> 172 us, k = 2 206 -> 244 -> 203, k = 4 285 -> 300
+// -> 278, k = 8 440 -> 410 -> 446, k = 32 1380 -> 1078 -> 1107.
 DirectOut::DirectOut(size_t bytes) {
   Ring& r = ring();
   if (bytes > kDirect || !r.direct_busy.try_lock()) return;
-  if (r.direct || (r.second && pin(r, &r.direct, kDirect))) {
+  if (r.direct || (r.small >= kCopiesFirst && pin(r, &r.direct, kDirect))) {
     ptr = r.direct;
     r.paths[FLB_READ_DIRECT] += 1;
     return;
   }
-  r.second = true;
+  r.small += r.small < kCopiesFirst;
   r.direct_busy.unlock();
 }
 DirectOut::~DirectOut() {

@@ -57,11 +57,11 @@ def test_moments_of_the_three_ways_agree(storage):
         with lat:
             f = np.where(np.arange(85 * ny) % 17 == 3, VOID, FLUID).astype(np.uint8)
             lat.upload_flags(f)
-            first = lat.moments()  # the buffer of small ones is there from the second on
+            first = [lat.moments() for _ in range(4)]  # the buffer of small ones is there from the fifth on
             was = abi.readout_paths()
             m = lat.moments()
             assert _took(was) == tuple(int(k == way) for k in range(3))
-            assert np.array_equal(first, m)
+            assert all(np.array_equal(v, m) for v in first)
             assert np.array_equal(m[:, f == VOID], np.zeros((3, int((f == VOID).sum()))))
             # 8 additions of terms whose magnitudes sum to at most 1.1
             eps = np.finfo(m.dtype).eps / 2
@@ -80,9 +80,11 @@ def test_small_moments_pin_a_small_buffer_of_their_own():
         with lat:
             was = abi.readout_paths()
             m = lat.moments()
-            assert abi.readout_paths()["pinned"] == 0 and _took(was) == (0, 0, 1)
+            for _ in range(3):
+                assert np.array_equal(lat.moments(), m)
+            assert abi.readout_paths()["pinned"] == 0 and _took(was) == (0, 0, 4)
             assert np.array_equal(lat.moments(), m)
-            assert abi.readout_paths()["pinned"] == DIRECT and _took(was) == (1, 0, 1)
+            assert abi.readout_paths()["pinned"] == DIRECT and _took(was) == (1, 0, 4)
             big, q = _block(400, 331)
             with big:
                 assert np.array_equal(big.pops(), q)
@@ -109,7 +111,8 @@ def test_threads_read_at_once():
             x.join()
         direct, ring, plain = _took(was)
         assert not wrong and direct == 0 and ring >= 1 and ring + plain == 12
-        m = c.moments()
+        for _ in range(4):
+            m = c.moments()
         was = abi.readout_paths()
         t = threading.Thread(target=read, args=(a, pa, 6))
         t.start()
