@@ -207,7 +207,7 @@ int prepare_march(flb_batch_s* t) {
   for (size_t k = 0; mc.per && k < nb; ++k)
     if (t->h_tab[k].pop_total + 37 * uint64_t(t->blocks[k]->dpop) * t->blocks[k]->elem >= (uint64_t(1) << 31))
       return FLB_OK;
-  if (!march_pays(form[0].dyn, t->blocks[0]->elem, live, true, {true, false, mc.per})) return FLB_OK;
+  if (!batch_march_pays(form[0].dyn, t->blocks[0]->elem, live)) return FLB_OK;
   if (ext != t->h_ext) {
     int cus = 0;
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, t->device));

@@ -87,7 +87,8 @@ struct flb_block_s {
   int wpb = 4;   // wavefronts per workgroup
   flbh::Twin twin;         // second population array of the two-step march (flb_march.hip)
   int march = -1;          // 1: the march may step the block, 0: not, -1: to be checked (flags, tasks or walls changed)
-  flb::MarchArgs tiles{};  // its tiles, planned once (ntx 0: not yet)
+  flb::MarchArgs tiles{};  // its tiles, planned once (ntx 0: not yet), and their estimated time
+  double tiles_cost = 0.0;
   int closed = -1;         // 1: no link of an updated cell leads to a cell that is not updated but wall links, 0, -1 likewise
   bool retained = false;   // holds the read-out buffers (readout_retain)
   int64_t paths[FLB_PATHS] = {};  // flb_block_paths
@@ -194,41 +195,26 @@ int march_run(flb_block_s* b, int n);
 // from there on (40 blocks of 481 MB: 234 -> 197 us), all blocks counted.
 //
 // In between lies a band where single steps, on one array, still run out of
-// the 256 MB memory-side cache and the march, on two, no longer does. Its ends
-// were measured every 5 MiB over cubes, boxes of rows of 97 and of 256 cells,
-// walled and periodic, march against single steps (times of the march in it,
-// and just outside): BGK FP32 from 158 to 218 MiB where rows are split into
-// tiles (1.0 to 1.12; 0.90 to 0.97), never where they are not (0.92 to 0.98);
-// BGK FP64 150 to 222 (0.94 to 1.12; 0.88 to 0.97); with a force FP32 148 to
-// 218 (0.98 to 1.17; 0.93 to 0.98), FP64 135 to 230 (0.96 to 1.17; 0.91 to
-// 0.99). Rows of 256 slots and more hold a quarter of padding, which fills the
-// cache for single steps too: no band (0.81 to 0.99), but FP64 with a force on
-// periodic boxes 165 to 205 MiB (1.00 to 1.06; 0.96 to 0.98). Batches behave as
-// blocks of split rows do, FP32 with a force from 140 and FP64 to 230 on.
+// the 256 MB memory-side cache and the march, on two, no longer does
+// (march_pays for a block). Batches behave as blocks of split rows do: BGK FP32
+// 158 to 218 MiB, FP64 150 to 230, with a force from 140 and 135 on (1.0 to
+// 1.16 times the single steps' time in it, 0.9 to 0.97 just outside).
 constexpr size_t kMarchMinBytes = size_t(42) << 20;
-struct MarchRows {
-  bool split, wide, per;  // split into tiles, of 256 slots and more; a periodic axis
-};
-inline bool march_pays(int dyn, size_t elem, size_t bytes, bool batch, const MarchRows& rows) {
-  if (dyn == FLB_DYN_SMAG_MRT) return bytes >= size_t(400) * 1000 * 1000 && (batch || elem == 8);
+inline bool batch_march_pays(int dyn, size_t elem, size_t bytes) {
+  if (dyn == FLB_DYN_SMAG_MRT) return bytes >= size_t(400) * 1000 * 1000;
   const size_t mib = bytes >> 20;
   const bool f64 = elem == 8, force = dyn == FLB_DYN_BGK_FORCE;
-  size_t lo, hi;
-  if (batch) {
-    lo = force ? (f64 ? 135 : 140) : (f64 ? 150 : 158);
-    hi = f64 ? 230 : 218;
-  } else if (rows.wide) {
-    lo = force && f64 && rows.per ? 165 : 0;
-    hi = lo ? 205 : 0;
-  } else if (force) {
-    lo = f64 ? 135 : 148;
-    hi = f64 ? 230 : 218;
-  } else {
-    lo = f64 ? 150 : (rows.split ? 158 : 0);
-    hi = f64 ? 222 : (rows.split ? 218 : 0);
-  }
+  const size_t lo = force ? (f64 ? 135 : 140) : (f64 ? 150 : 158), hi = f64 ? 230 : 218;
   return bytes >= kMarchMinBytes && !(mib >= lo && mib < hi);
 }
+// The rows of one block, its periodic axes, and march_plan's estimate.
+struct MarchRows {
+  int ex, pitch;
+  bool split;  // into tiles
+  bool px, per, all;  // x periodic, any axis, every axis
+  double cost;
+};
+bool march_pays(int dyn, size_t elem, size_t bytes, const MarchRows& rows);
 // march_form sets *ok where a block of any size is of the form the march
 // takes, with its flags and dynamics in m (not its tiles). march_plan: tiles
 // of one box of cells (rows of `pitch` slots) for
@@ -241,7 +227,7 @@ struct MarchBox {
   bool operator==(const MarchBox& o) const { return ex == o.ex && ey == o.ey && ez == o.ez && pitch == o.pitch; }
 };
 int march_form(flb_block_s* b, flb::MarchArgs* m, bool* ok);
-flb::MarchArgs march_plan(const MarchBox& box, int elem, int cus, int threads);
+flb::MarchArgs march_plan(const MarchBox& box, int elem, int cus, int threads, double* cost = nullptr);
 double march_plan_batch(const std::vector<MarchBox>& boxes, int elem, int cus, int threads,
                         std::vector<flb::MarchArgs>& mt, std::vector<flb::MarchWg>& wgs);
 bool march_fits(size_t bytes);

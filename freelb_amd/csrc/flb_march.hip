@@ -55,7 +55,7 @@ void each_tile(const MarchBox& a, int elem, int threads, F&& f) {
 // their tiles do too. Made once per block or box, as a run may be four steps:
 // in each run, and with every aligned width tried over and over, it cost 36 us
 // at 256^3 and 140 us at 1000x60x12 (1 us in the mean now).
-flb::MarchArgs march_plan(const MarchBox& a, int elem, int cus, int threads) {
+flb::MarchArgs march_plan(const MarchBox& a, int elem, int cus, int threads, double* cost_out) {
   flb::MarchArgs best{};
   double best_cost = 1e300;
   each_tile(a, elem, threads, [&](int w, int h, int ntx, int nty) {
@@ -76,6 +76,7 @@ flb::MarchArgs march_plan(const MarchBox& a, int elem, int cus, int threads) {
       }
     }
   });
+  if (cost_out) *cost_out = best_cost;
   return best;
 }
 
@@ -221,6 +222,66 @@ double march_plan_batch(const std::vector<MarchBox>& boxes, int elem, int cus, i
   return best_span;
 }
 
+// Whether one block marches: from 42 MiB on (kMarchMinBytes), but not where
+// single steps gain more from the memory-side cache. Lines drawn by march and
+// single steps of 2700 blocks of 44 to 266 MiB, BGK and with a force, FP32 and
+// FP64, rows of 12 to 1000 cells, walled and periodic in x, in y and z and in
+// all (times of the march over single steps):
+// - rows of less than 256 slots: FP32 loses from 160 MiB (periodic in x only or
+//   also in one more axis, where single steps lose least: 142) to 215 where rows
+//   are split or have at most 64 cells (1.0 to 1.19), from 165 and only if so
+//   periodic where a tile holds rows of 65 to 128 (1.02 to 1.07); with a force
+//   from 140 (x periodic 122) to 222 (1.0 to 1.23). Rows of at most 24 cells,
+//   whose rings are widest, lose with a force and x periodic at any smaller
+//   size too (0.96 to 1.16). FP64 from 160 (split rows 180) to 212 (228), with a
+//   force from 132 (1.0 to 1.23). Below these bands 0.72 to 1.0, above 0.65 to
+//   0.97.
+// - rows of 256 slots and more hold a quarter to half of padding, which fills
+//   the cache for single steps as well: BGK 0.64 to 0.98 throughout, also with
+//   a force where rows leave a tenth of their wavefronts' lanes idle (230, 400
+//   cells: 0.72 to 0.99) and on walled boxes. Periodic ones with a force and
+//   fuller rows lose from 120 to 270 MiB in FP32 (1.0 to 1.13; all axes 140 to
+//   205, to 1.07), from 145 to 230 in FP64, not with all axes (0.8 to 1.0). Thin
+//   boxes whose tiles fit badly (700x20 FP64, 1000x30x21: 1.02 to 1.28) are told
+//   by the estimate per MiB.
+// On 330 other blocks of 43 to 285 MiB, drawn over the same ranges, blocks take
+// 0.902 of their single steps' time in the mean so (0.913 if all marched, 0.900
+// the better of both for each), the worst march 1.07.
+bool march_pays(int dyn, size_t elem, size_t bytes, const MarchRows& r) {
+  const bool f64 = elem == 8, force = dyn == FLB_DYN_BGK_FORCE;
+  if (dyn == FLB_DYN_SMAG_MRT) return f64 && bytes >= size_t(400) * 1000 * 1000;
+  if (bytes < kMarchMinBytes) return false;
+  const size_t mib = bytes >> 20;
+  size_t lo = 0, hi = 0;
+  if (r.pitch >= 256) {
+    if (!linear_form(r.ex) && force) {
+      if (mib < 56 && r.cost >= 1.25 * double(mib)) return false;
+      if (r.per && !r.all) {
+        lo = f64 ? 145 : 120;
+        hi = f64 ? 230 : 270;
+      } else if (r.all && !f64) {
+        lo = 140;
+        hi = 205;
+      }
+    }
+    if (f64 && mib >= 125 && r.cost >= (mib < 210 ? 1.0 : 0.94) * double(mib)) return false;
+  } else if (f64) {
+    lo = force ? 132 : (r.split ? 180 : 160);
+    hi = r.split ? 228 : 212;
+  } else if (force) {
+    lo = !r.px ? 140 : (r.ex <= 24 ? 0 : 122);
+    hi = 222;
+  } else if (r.split || r.ex <= 64) {
+    lo = r.px && !r.all ? 142 : 160;
+    hi = 215;
+  } else if (r.px && !r.all) {
+    lo = 165;
+    hi = 215;
+  }
+  if (r.ex < 16 && !f64) hi = std::min<size_t>(hi, 195);  // their padding ends the band earlier
+  return !(mib >= lo && mib < hi);
+}
+
 // Second arrays take at most a sixteenth of the device's memory and leave
 // half of it free.
 bool march_fits(size_t bytes) {
@@ -337,10 +398,12 @@ bool march_ready(flb_block_s* b) {
       if (b->tiles.ntx == 0) {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess) return false;
-        b->tiles = march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem));
+        b->tiles = march_plan({a.ex, a.ey, a.ez, a.pitch}, int(b->elem), cus, flb::march_threads(b->elem),
+                              &b->tiles_cost);
         b->paths[FLB_PATH_PLANS] += 1;
       }
-      ok = march_pays(m.dyn, b->elem, bytes, false, {b->tiles.ntx > 1, a.pitch >= 256, a.px || a.py || a.pz});
+      ok = march_pays(m.dyn, b->elem, bytes, {a.ex, a.pitch, b->tiles.ntx > 1, a.px != 0, a.px || a.py || a.pz,
+                                              a.px && a.py && a.pz, b->tiles_cost});
     }
     b->march = ok ? 1 : 0;
     if (!ok) return false;

@@ -22,12 +22,27 @@ def _params(test, names):
 @pytest.mark.parametrize("periodic,dyn,obstacles",
                          _params(march_tests.test_runs_equal_single_steps, "periodic,dyn,obstacles"))
 def test_boxes_of_the_run_tests_take_two_steps(storage, dims, periodic, dyn, obstacles):
+    if dyn == abi.DYN_BGK_FORCE and dims in ((23, 29, 880), (700, 31, 27)):
+        pytest.skip("steps singly, which is faster; larger boxes of these rows below")
     with march_tests._box(dims, periodic, storage, dyn, obstacles) as lat:
         for n, two in ((4, 0), (5, 2), (9, 4), (1, 0)):  # parities 0, 0, 1, 0
             before = lat.paths()["two_step"]
             lat.step(n)
             assert lat.paths()["two_step"] - before == two, n
         assert lat.paths()["coupled"] == 0
+
+
+@pytest.mark.parametrize("dims", [(23, 29, 4800), (700, 31, 40)])
+@pytest.mark.parametrize("periodic,obstacles", [((True, False, False), True), ((True, True, True), False)])
+def test_forced_rows_of_large_boxes_equal_single_steps(dims, periodic, obstacles):
+    """Narrow and wide rows, periodic in x and with a force: boxes large enough to march, bit for
+    bit against single steps."""
+    def make():
+        return march_tests._box(dims, periodic, "f32", abi.DYN_BGK_FORCE, obstacles)
+    with make() as lat:
+        lat.step(9)
+        assert lat.paths()["two_step"] == 4
+    march_tests._agree(make, (5, 4, 9))
 
 
 @pytest.mark.parametrize("storage,dims,collision",
@@ -45,11 +60,16 @@ def test_lid_boxes_take_the_meant_path(storage, dims, collision):
     ("f32", abi.DYN_BGK, (148, 146, 141), 0, True), ("f32", abi.DYN_BGK, (97, 160, 160), 0, True),
     ("f32", abi.DYN_BGK, (256, 97, 100), 0, True), ("f64", abi.DYN_BGK, (104, 100, 95), 0, True),
     ("f64", abi.DYN_BGK, (110, 110, 105), 0, False), ("f64", abi.DYN_BGK, (117, 117, 115), 0, True),
-    ("f32", abi.DYN_BGK_FORCE, (97, 150, 125), 1, True), ("f32", abi.DYN_BGK_FORCE, (97, 160, 160), 1, False),
+    ("f32", abi.DYN_BGK_FORCE, (97, 140, 120), 1, True), ("f32", abi.DYN_BGK_FORCE, (97, 160, 160), 1, False),
     ("f32", abi.DYN_BGK_FORCE, (136, 150, 152), 1, True), ("f64", abi.DYN_BGK_FORCE, (97, 100, 90), 0, True),
     ("f64", abi.DYN_BGK_FORCE, (110, 110, 105), 1, False), ("f64", abi.DYN_BGK_FORCE, (117, 118, 120), 1, True),
     ("f64", abi.DYN_BGK_FORCE, (256, 70, 70), 1, False), ("f64", abi.DYN_BGK_FORCE, (256, 70, 70), 0, True),
-    ("f32", abi.DYN_BGK_FORCE, (256, 97, 100), 1, True)])
+    ("f32", abi.DYN_BGK_FORCE, (256, 97, 100), 0, True), ("f32", abi.DYN_BGK_FORCE, (256, 97, 100), 1, False),
+    ("f32", abi.DYN_BGK_FORCE, (400, 64, 100), 1, True), ("f32", abi.DYN_BGK, (20, 200, 600), 0, False),
+    ("f32", abi.DYN_BGK, (20, 200, 350), 0, True), ("f32", abi.DYN_BGK_FORCE, (20, 200, 300), 1, False),
+    ("f32", abi.DYN_BGK, (97, 160, 170), 0, True), ("f32", abi.DYN_BGK, (97, 160, 170), 1, False),
+    ("f64", abi.DYN_BGK, (700, 20, 81), 1, False), ("f64", abi.DYN_BGK_FORCE, (300, 50, 70), 1, False),
+    ("f64", abi.DYN_BGK, (60, 90, 180), 0, True), ("f64", abi.DYN_BGK, (60, 90, 240), 0, False)])
 def test_band_of_the_memory_side_cache_steps_singly(storage, dyn, dims, per, marches):
     with march_tests._box(dims, (bool(per), False, False), storage, dyn, False) as lat:
         lat.step(5)
