@@ -1418,6 +1418,12 @@ int march_nt(size_t real, bool bwd) {
 // -> 15.1 backward; smaller ones run out of the caches); the passes address a
 // state with 31-bit byte offsets.
 constexpr size_t kTwoStepBytes = size_t(32) << 20;
+// Segments recomputed before FP64's single backward steps: those find the
+// records of single steps in the caches longer (backward, every 7: 56x55x76,
+// 35.6 MB, 27.2 -> 29.4 us per step with two-step launches, 79x49x65, 38.2 MB,
+// 28.4 -> 30.7; 52x51x102, 41.1 MB, the same; 89x67x55, 49.9 MB, 39.8 -> 38.1).
+template <class R>
+constexpr size_t kTwoStepRecompute = sizeof(R) == 8 ? size_t(384) * 100 * 1000 : kTwoStepBytes;
 const flb::MarchArgs* march_of(flb_adjoint_s* h, bool bwd) {
   if (state_bytes(h) < kTwoStepBytes || state_bytes(h) >= (size_t(1) << 31)) return nullptr;
   flb::MarchArgs& m = h->tiles[bwd];
@@ -1570,7 +1576,7 @@ int backward_impl(flb_adjoint_s* h, double* grad) {
   if (rc) return rc;
   HIP_TRY(hipEventRecord(h->e0, h->stream));
   HIP_TRY(hipMemsetAsync(h->d_grad, 0, size_t(h->N) * h->real, h->stream));
-  const flb::MarchArgs* const fm = march_of(h, false);
+  const flb::MarchArgs* const fm = state_bytes(h) < kTwoStepRecompute<R> ? nullptr : march_of(h, false);
   const flb::MarchArgs* const m = sizeof(R) == 4 && pairs(T, K) ? march_of(h, true) : nullptr;
   const auto seed = m ? A::k_seed<R, false> : A::k_seed<R, true>;
   hipLaunchKernelGGL(seed, dim3(grid_of(h)), dim3(A::kThreads), 0, h->stream, adj_args<R>(h),

@@ -128,6 +128,16 @@ def test_adjoint_boxes_take_two_steps(storage, dims, per, solids):
             assert now["backward_two"] - was["backward_two"] == b * back, (T, K)
 
 
+@pytest.mark.parametrize("dims,recompute", [((56, 55, 76), 0), ((62, 60, 80), 4)])
+def test_small_fp64_boxes_recompute_singly(dims, recompute):
+    with Adjoint(dims, omega=1.6, periodic=(True, False, False), storage="f64") as adj:
+        adj.init_equilibrium(np.ones(adj.N), np.zeros((3, adj.N)))
+        adj.forward(8, 4)
+        assert adj.paths()["forward_two"] == 4
+        adj.backward()
+        assert adj.paths()["forward_two"] == 4 + recompute
+
+
 @pytest.mark.parametrize("storage", ["f32", "f64"])
 def test_adjoint_batch_takes_two_steps(storage):
     members = []
