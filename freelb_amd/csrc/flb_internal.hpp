@@ -18,6 +18,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace flb {
@@ -63,6 +64,7 @@ struct KArgs {
   void* pops;            // population slot 0 of direction 0
   int64_t dpop;          // elements between directions
   int ypop;              // population slots between rows
+  int dyns;              // bit set of the tasks' dynamics, 0 if two tasks of one dynamics differ in its constant
   int64_t zpop;          // population slots between planes
   const uint8_t* flags;  // slot 0
   const void* rho_f;     // slot 0 of the RHO field (compute type), or null (rho = 1)
@@ -80,8 +82,6 @@ struct KArgs {
   int wpb;               // wavefronts per workgroup
   int nblocks;           // workgroups
   int ntasks;
-  int dyns;              // bit set of the tasks' dynamics, 0 if two tasks of one dynamics differ in its constant
-  uint8_t anymask;       // OR of tmask
   int nbc;
   uint8_t tmask[kMaxTasks];
   uint8_t tdyn[kMaxTasks];
@@ -90,6 +90,7 @@ struct KArgs {
   uint8_t bcvoid[kMaxBc];
   uint8_t bckind[kMaxBc];
   uint8_t bcany;         // OR of bcmask: cells that may have halfway links
+  uint8_t anymask;       // OR of tmask
   const uint64_t* links; // slot 0 of the precomputed wall links (normal | moving << 32)
   uint64_t pop_total;    // bytes of the population allocation
   uint32_t buf;          // 1: the step may address populations through wavefront-based buffer descriptors
@@ -111,6 +112,13 @@ struct KArgs {
   double cpl_gbeta[kMaxCouplings];
   double cpl_rho0[kMaxCouplings];
 };
+// Where the fields lie against the 64-byte lines that a step's scalar loads
+// bring shows in small blocks: 8 bytes before nbc took plain MRT in FP64 from
+// 5.82 to 6.11 us per step (20^3), D2Q9 in FP32 from 4.16 to 4.32 (30^2), BGK
+// from 4.55 to 4.67 (FP64 20^3). New fields go into the holes or to the end.
+static_assert(offsetof(KArgs, nbc) == 148 && offsetof(KArgs, omega) == 240 && offsetof(KArgs, mrt_sn_f) == 400 &&
+                  offsetof(KArgs, u_ext) == 664 && sizeof(KArgs) == 728,
+              "a step's arguments moved: measure small blocks");
 
 // The two-step march (flb_march.hpp): target populations (slot 0 of direction
 // 0), tile extents and counts, planes per workgroup.
