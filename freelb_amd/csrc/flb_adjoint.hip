@@ -462,8 +462,20 @@ __device__ __forceinline__ double wg_sum(double v) {
 // fixed stride, then wg_sum: the same bits however the steps that wrote the
 // shares were launched.
 __device__ __forceinline__ void obj_sum(const double* __restrict__ p, unsigned n, double* __restrict__ jt) {
+  // Sixteen loads at a time, added in order: one workgroup per state waits for
+  // each of its loads in turn otherwise (14x170x259 FP32, 10 forward steps and
+  // their sums: 200 -> 166 us).
+  constexpr unsigned U = 16;
   double v = 0.0;
-  for (unsigned k = threadIdx.x; k < n; k += kThreads) v += p[k];
+  unsigned k = threadIdx.x;
+  for (; k + (U - 1) * kThreads < n; k += U * kThreads) {
+    double t[U];
+#pragma unroll
+    for (unsigned i = 0; i < U; ++i) t[i] = p[k + i * kThreads];
+#pragma unroll
+    for (unsigned i = 0; i < U; ++i) v += t[i];
+  }
+  for (; k < n; k += kThreads) v += p[k];
   const double s = wg_sum(v);
   if (threadIdx.x == 0) *jt = s;
 }

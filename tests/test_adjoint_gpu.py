@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from adjoint_model import Model
+from adjoint_model import C19, Model
 from adjoint_torch import AdjointObjective
 from freelb_amd import Adjoint, AdjointBatch
 from freelb_amd.cases import channel_adjoint
@@ -330,3 +330,26 @@ def test_channel_batch_runs_and_matches_one_member():
         b.close()
         for a in mem:
             a.close()
+
+
+@pytest.mark.parametrize("dims", [(6, 7, 5), (6, 16, 16), (5, 63, 65), (5, 64, 64), (4, 64, 65), (3, 170, 259)])
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+def test_objective_is_the_sum_over_outlet_planes_of_any_size(dims, storage):
+    """J after one and after two steps against the plane's sum of the states they leave, in FP64: the
+    sum takes 16 x 256 shares at a time, then 256. Terms of at most 0.07, 10 per cell, and partial
+    sums of at most 0.02 per cell, each rounded to 1.1e-16."""
+    nx, ny, nz = dims
+    N, n = nx * ny * nz, ny * nz
+    rng = np.random.default_rng(N)
+    with Adjoint(dims, omega=1.6, periodic=(True, False, False), storage=storage) as adj:
+        adj.init_equilibrium(np.ones(N), rng.uniform(-0.02, 0.02, (3, N)))
+        J = [adj.forward(T, -1) for T in (1, 2)]
+        states = []
+        for T in (1, 2):
+            adj.forward(T, -1)
+            f = adj.state().reshape(19, nz, ny, nx)[:, :, :, nx - 1]
+            states.append(float(np.tensordot(C19[:, 0].astype(np.float64), f, axes=(0, 0)).sum()))
+    eps = 2.0 ** -53
+    tol = eps * (n * (10 * 0.7 + 10 * 0.07) + n * 0.02 * n)
+    assert abs(J[0] - states[0]) <= tol
+    assert abs(J[1] - (states[0] + states[1]) / 2) <= tol
